@@ -1,29 +1,36 @@
 // attn_bwd.hip -- fused causal attention backward for gfx950 (recompute).
 //
 // Kernel 1 (bwd_pre): delta[i] = sum_d dO[i,d] * O[i,d] per query row (the
-// row dot that SoftmaxBackward computes as sum_j dP_ij P_ij), and zeroes the
-// fp32 dQ accumulator.  (The bf16 main kernel at D <= 64 forms delta itself,
-// and then this pass only zeroes.)
+// row dot that SoftmaxBackward computes as sum_j dP_ij P_ij), zeroes the
+// fp32 dQ accumulator and, for fp32, leaves the largest |q| and |dO| of its
+// rows.  (The bf16 main kernel at D <= 64 forms delta itself, and then this
+// pass only zeroes.)
 //
-// Kernel 2 (bwd_main): one workgroup = 4 waves = 128 keys of one (b, h); each
-// wave owns 32 keys and keeps K and V for them in VGPRs plus its dK^T and dV^T
-// accumulators for the whole kernel, so dK and dV are written exactly once,
-// with no atomics.  The workgroup walks query tiles of 32 rows from the first
-// row that can see its keys to the end.  Per tile and wave:
+// Kernel 2 (bwd_main, fp32): its products run on the fp16 matrix cores, every
+// operand split into two fp16 parts (common.h), three MFMAs per product step.
+// One workgroup = 8 waves = 4 pairs, each pair with 64 keys (or 32) of one
+// (b, h).  In a pair, wave 0 (role 0) holds the keys' K operand and dV^T
+// accumulators in VGPRs, wave 1 (role 1) their V operand and dK^T accumulators,
+// 64 + 64 registers each at D = 64 and 128, so two waves fit a SIMD, one of each
+// role.  dK and dV are written exactly once, with no atomics.  The workgroup
+// walks query tiles of 32 rows, split into LDS once for all waves; per tile,
+// in three phases with a barrier after each:
 //
-//   S  (q x keys)   = Q K^T          A = Q from LDS, B = K^T in VGPRs
-//   dP (q x keys)   = dO V^T         A = dO from LDS, B = V^T in VGPRs
-//   P  = exp2(S*c - lse*log2e), masked entries exactly 0
-//   dS = P * (dP - delta)
-//   dV^T += dO^T P                   B = P straight from the S accumulators
-//   dK^T += Q^T dS                   B = dS straight from the dP accumulators
+//   A  role 0: S = Q K^T, P = exp2(S c - lse log2e) (masked entries exactly 0),
+//      P handed to role 1 through LDS;   role 1: dP = dO V^T
+//   B  role 0: dV^T += dO^T P;   role 1: dS = P (dP - delta), split, to LDS
+//   C  role 0: dQ tile += dS K over the workgroup's keys, fp32 atomics into the
+//      global accumulator;   role 1: dK^T += Q^T dS;   both: the next tile
 //
-// All four keep keys on the lane axis.  dQ = dS K needs queries on the lane
-// axis instead, so each wave writes its dS block to LDS, and after a barrier
-// the four waves compute the tile's dQ (32 x D over all 128 keys) with
-// v_mfma_f32_16x16x4_f32 and add it to the fp32 accumulator with one
-// global atomic add per element per 128-key block.  Workgroup w takes key
-// block w / (B*H), so the blocks with the most query tiles start first.
+// Keys lie on the lane axis in S, dP, dV^T and dK^T, so P and dS are operands
+// straight from the accumulators; the transposed operands (dO^T, Q^T, dS) are
+// transposed LDS reads, and K^T for dQ is staged transposed once.  S is formed
+// in the forward's order, to the same bits, so P is consistent with the LSE.
+// Bound by the phases' latency: a tile's MFMAs take 3840 of its 8100 (D = 128)
+// or 9100 (D = 64) cycles per SIMD, and at config 4 the fp16 MFMAs run at a
+// 2.0 GHz shader clock.  The backward call against the fp32-MFMA kernel that this
+// one replaced (us): config 2 308 -> 163, config 4 5980 -> 2170, B8 H12 T1024 D32
+// 178 -> 128, B1 H12 T333 D64 34 -> 27.
 //
 // bf16 inputs use the bf16-MFMA main kernel (attn_bwd_bf16.hip) between the
 // same pre kernel and a final bwd_cvt that turns the fp32 dQ accumulator into
@@ -76,19 +83,37 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(BwdParams p) {
     constexpr int TPR = bwd_pre_tpr<D, E>();    // threads per row
     constexpr int RPB = bwd_pre_rows_per_block<D, E>();
     const int tid = threadIdx.x;
-    const int64_t row = (int64_t)blockIdx.x * RPB + tid / TPR;
     const int c = tid % TPR;
     const int64_t rows = (int64_t)p.B * p.H * p.Tq;
-    float s = 0.f;
-    if (row < rows) {
-        int64_t b, h, i;
-        bwd_row_split(p, rows, row, b, h, i);
+    // fp32: p.n_amax workgroups per head; bf16: flat over the rows
+    int64_t row, b, h, i;
+    bool in;
+    if constexpr (sizeof(E) == 4) {
+        const unsigned bh = blockIdx.x / (unsigned)p.n_amax;
+        i = (int64_t)(blockIdx.x % (unsigned)p.n_amax) * RPB + tid / TPR;
+        b = bh / (unsigned)p.H;
+        h = bh % (unsigned)p.H;
+        in = i < p.Tq;
+        row = (int64_t)bh * p.Tq + i;
+    } else {
+        row = (int64_t)blockIdx.x * RPB + tid / TPR;
+        in = row < rows;
+        if (in) bwd_row_split(p, rows, row, b, h, i);
+    }
+    float s = 0.f, aq = 0.f, ad = 0.f;
+    if (in) {
         if (p.pre_delta) {
             const E* po = (const E*)p.o + b * p.so.b + h * p.so.h + i * p.so.t + VEC * c;
             const E* pd = (const E*)p.dout + b * p.sdo.b + h * p.sdo.h + i * p.sdo.t + VEC * c;
             if constexpr (sizeof(E) == 4) {
                 const f32x4 o4 = ld4(po), d4 = ld4(pd);
                 s = o4[0] * d4[0] + o4[1] * d4[1] + o4[2] * d4[2] + o4[3] * d4[3];
+                const f32x4 q4 = ld4((const E*)p.q + b * p.sq.b + h * p.sq.h + i * p.sq.t + VEC * c);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    aq = fmaxf(aq, finite_abs(q4[k]));
+                    ad = fmaxf(ad, finite_abs(d4[k]));
+                }
             } else {
                 const u16x8 o8 = *reinterpret_cast<const u16x8*>(po);
                 const u16x8 d8 = *reinterpret_cast<const u16x8*>(pd);
@@ -105,7 +130,20 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(BwdParams p) {
     // (p.pre_delta is uniform: the whole grid takes or skips the exchange)
     if (p.pre_delta) {
         s = group_sum<TPR>(s);
-        if (row < rows && c == 0) p.delta[row] = s;
+        if (in && c == 0) p.delta[row] = s;
+    }
+    if constexpr (sizeof(E) == 4) {
+        __shared__ float red[2][4];
+        aq = wave_max(aq);
+        ad = wave_max(ad);
+        if ((tid & 63) == 0) {
+            red[0][tid >> 6] = aq;
+            red[1][tid >> 6] = ad;
+        }
+        __syncthreads();
+        if (tid < 2)
+            p.amax[(int64_t)blockIdx.x * 2 + tid] =
+                fmaxf(fmaxf(red[tid][0], red[tid][1]), fmaxf(red[tid][2], red[tid][3]));
     }
     if (blockIdx.x == 0)
         for (int i = tid; i < p.n_split * p.B * p.H; i += 256) p.counters[i] = 0u;
@@ -124,50 +162,65 @@ __global__ __launch_bounds__(256) void bwd_zero_kernel(BwdParams p) {
         for (int i = threadIdx.x; i < p.n_split * p.B * p.H; i += 256) p.counters[i] = 0u;
 }
 
-template <int D>
+// KP: keys per pair of waves (32 at D = 128, else 32 or 64)
+template <int D, int KP>
 struct BwdTile {
-    static constexpr int NW = bwd_waves(0, D);  // waves per workgroup, 32 keys each
-    static constexpr int BK = 32 * NW;       // keys per workgroup
-    static constexpr int QS = D + 4;         // Q / dO row stride in LDS (floats)
-    static constexpr int SS = BK + 4;        // dS row stride
-    static constexpr int KTS = BK + 4;       // K^T row stride
+    static constexpr int BK = 4 * KP;              // keys per workgroup
+    // Q / dO row stride in LDS (fp16 elements): row reads want an odd number of
+    // 16-byte units, transposed reads the 32-byte windows of 4 rows in disjoint banks
+    static constexpr int QS = D == 128 ? 152 : D == 64 ? 72 : 56;
+    static constexpr int SS = 36;                  // dS row stride (queries of one key, fp16 elements)
 };
+constexpr float kBwdPBits = 14.f, kBwdPInv = 1.f / 16384.f;  // P enters its products as 2^14 P
+
+// A operand (32 rows of 16 values) read transposed from `t`, rows = the
+// reduction index r0 + {0..3} and + 8 + {0..3} per lane half (r0 includes 4 g),
+// columns c0 + lane % 32.
+template <typename Addr>
+__device__ __forceinline__ f16x8 tr_frag(Addr addr) {
+    const f16x4 lo = ds_read_tr16_f16(addr(0));
+    const f16x4 hi = ds_read_tr16_f16(addr(8));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
 
 // SHORT: the launch has short rows (p.n_short > 0); without them the kernel
 // carries neither the prologue nor the low part of delta.
-template <int D, typename E, bool SHORT>
-__global__ __launch_bounds__(64 * bwd_waves(0, D), (bwd_waves(0, D) == 8 || D >= 128) ? 1 : 2) void bwd_main_kernel(
-    BwdParams p) {
-    constexpr int NW = BwdTile<D>::NW;
-    constexpr int NT = 64 * NW;
+// DQD: dQ comes from the query-major pass (bwd_dq_kernel), not from here.
+template <int D, int KP, bool SHORT, bool DQD>
+__global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
+    using T = BwdTile<D, KP>;
+    constexpr int NT = 512;
     constexpr int BQ = kBwdBQ;
-    constexpr int BK = BwdTile<D>::BK;
-    constexpr int HD = D / 2;
-    constexpr int NDB = D / 32;
-    constexpr int C4 = D / 4;
-    constexpr int QS = BwdTile<D>::QS;
-    constexpr int SS = BwdTile<D>::SS;
-    constexpr int KTS = BwdTile<D>::KTS;
-    constexpr int QLPT = BQ * C4 / NT;    // 4-element loads per thread for a Q / dO tile
-    constexpr int KLPT = BK * C4 / NT;    // for the K^T staging
-    constexpr int NDQ = 2 * (D / 16);     // 16x16 dQ blocks of a query tile, NDQ / NW per wave
-    static_assert(BQ * C4 % NT == 0 && BK * C4 % NT == 0 && NDQ % NW == 0, "whole passes");
+    constexpr int BK = T::BK, QS = T::QS, SS = T::SS;
+    constexpr int NKB = KP / 32;           // 32-key blocks per pair
+    constexpr int NKK = D / 16;            // MFMA steps along the head dim
+    constexpr int NDB = D / 32;            // 32-wide head-dim blocks
+    constexpr int C8 = D / 8;              // 8-element chunks per row
+    constexpr int NCH = BQ * C8;           // chunks of a Q or dO tile, staged by 256 threads
+    constexpr int CPT = (NCH + 255) / 256;
+    constexpr int XB = 32 * SS * 2;        // bytes of one dS part of a 32-key block
+    constexpr int DQP = NDB;               // dQ: pairs of keys per wave (4 / NDB waves share a head-dim block)
+    constexpr int KU = BK / 8 * D / NT;    // K^T units per thread
 
-    __shared__ __attribute__((aligned(16))) float Qs[BQ][QS];
-    __shared__ __attribute__((aligned(16))) float dOs[BQ][QS];
-    __shared__ __attribute__((aligned(16))) float dSs[BQ][SS];
-    __shared__ __attribute__((aligned(16))) float Kts[D][KTS];
+    __shared__ __attribute__((aligned(16))) _Float16 Qs[2][2][BQ][QS];  // [buffer][part]
+    __shared__ __attribute__((aligned(16))) _Float16 dOs[2][BQ][QS];    // [part]
+    __shared__ f16x8 Kt[2][BK / 8][D];  // [part][8 keys][head dim]: K^T in the dQ product's operand order
+    __shared__ __attribute__((aligned(16))) char Xs[4][NKB * 2 * XB];   // P, then dS, of each pair
     __shared__ __attribute__((aligned(16))) float lse_s[BQ];
     __shared__ __attribute__((aligned(16))) float dl_s[BQ];
-    __shared__ __attribute__((aligned(16))) float dlo_s[BQ];  // low part of the short rows' delta (else 0)
+    __shared__ __attribute__((aligned(16))) float dlo_s[BQ];
+    __shared__ float dinv_s[SHORT ? BQ : 1];  // units of the dO rows
+    __shared__ int dqcls_s[4];     // sum of the classes of a pair's dS, V and K
+    __shared__ int kcls_s[4];
+    __shared__ float red_s[2][8];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int role = wave >> 2;  // 0: K, S, P, dV; 1: V, dP, dS, dK
+    const int pr = wave & 3;     // pair
     const int l32 = lane & 31;
     const int g = lane >> 5;
-    const int l16 = lane & 15;
-    const int g4 = lane >> 4;
 
     const BwdWork wk = bwd_work<BK>(p);
     if (wk.bh >= p.B * p.H) return;  // padding workgroup of a split plan's grid
@@ -176,336 +229,481 @@ __global__ __launch_bounds__(64 * bwd_waves(0, D), (bwd_waves(0, D) == 8 || D >=
     const int b = bh / p.H;
     const int h = bh % p.H;
 
-    const E* Q = (const E*)p.q + b * p.sq.b + h * p.sq.h;
-    const E* K = (const E*)p.k + b * p.sk.b + h * p.sk.h;
-    const E* V = (const E*)p.v + b * p.sv.b + h * p.sv.h;
-    const E* dO = (const E*)p.dout + b * p.sdo.b + h * p.sdo.h;
+    const float* Q = (const float*)p.q + b * p.sq.b + h * p.sq.h;
+    const float* dO = (const float*)p.dout + b * p.sdo.b + h * p.sdo.h;
     float* dQa = p.dq_acc + b * p.sacc.b + h * p.sacc.h;
     const float* LSE = p.lse + (int64_t)bh * p.Tq;
     const float* DL = p.delta + (int64_t)bh * p.Tq;
     const float* DLO = p.delta_lo + (int64_t)bh * p.Tq;
-
     const int k0 = kblk * BK;
-    const int k0w = k0 + wave * 32;
-    const int key = k0w + l32;  // this lane's key
-
-    // K^T and V^T operands: lane (l32, g) holds row `key`, columns g*HD + i.
-    float kf[HD], vf[HD];
-    if (key < p.Tk) {
-        const E* ks = K + (int64_t)key * p.sk.t + g * HD;
-        const E* vs = V + (int64_t)key * p.sv.t + g * HD;
-#pragma unroll
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = ld4(ks + i);
-            const f32x4 c = ld4(vs + i);
-            kf[i] = a[0]; kf[i + 1] = a[1]; kf[i + 2] = a[2]; kf[i + 3] = a[3];
-            vf[i] = c[0]; vf[i + 1] = c[1]; vf[i + 2] = c[2]; vf[i + 3] = c[3];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < HD; ++i) kf[i] = vf[i] = 0.f;
-    }
-
-    f32x16 dv_acc[NDB], dk_acc[NDB];
-#pragma unroll
-    for (int i = 0; i < NDB; ++i) {
-        dv_acc[i] = f32x16{};
-        dk_acc[i] = f32x16{};
-    }
+    const int k0p = k0 + pr * KP;  // the pair's first key
 
     const int q_begin = wk.q_begin;
     const int q_end = wk.q_end;
-    const float c = p.c;
 
-    // Query-tile staging.  With PF (D <= 64, where the registers fit) the next
-    // tile's Q, dO, LSE and delta are loaded into registers while the current
-    // tile computes and stored to LDS right after the dS barrier, when every
-    // wave is done with the staged copies: two barriers per tile.  The
-    // prefetch is straight-line (a row limit of 0 past the last tile) and keeps
-    // raw values, so no wait for it lands inside the MFMA blocks.
-    // The loads go through buffer resources over rows [q0, lim): chunk
-    // tid + NT i sits NT i / C4 rows below chunk tid, and rows past the
-    // resource read as zeros, so a load needs no address arithmetic or branch.
-    constexpr bool PF = D <= 64;
-    // The LSE is staged in base 2 (scaled by log2(e) once per row instead of
-    // once per score) except at D = 64, which measured 2% slower that way at
-    // config 2; at D = 32 the staging keeps the kernel within the registers
-    // of three workgroups per CU (B4 H16 T1024: 134 -> 119 us).
-    constexpr float kLseStage = D == 64 ? 1.f : kLog2e;
-    constexpr float kLseRead = D == 64 ? kLog2e : 1.f;
-    static_assert(NT % C4 == 0, "chunk rows must split into thread + load parts");
-    static_assert(sizeof(E) == 4, "fp32 storage (bf16 has its own kernel)");
-    f32x4 ra[QLPT], rd[QLPT];
-    float r_lse = 0.f, r_dl = 0.f, r_dlo = 0.f;
-    const uint32_t q_voff = (uint32_t)(((int64_t)(tid / C4) * p.sq.t + 4 * (tid % C4)) * 4);
-    const uint32_t do_voff = (uint32_t)(((int64_t)(tid / C4) * p.sdo.t + 4 * (tid % C4)) * 4);
-    auto gload_q = [&](int q0, int lim) {
+    // Role 1's threads stage the Q tiles, role 0's the dO tiles, with the rows'
+    // LSE and delta.  Rows at or past `lim` read as zeros.
+    const int ts = tid & 255;
+    const float* Y = role ? Q : dO;
+    const int64_t yt = role ? p.sq.t : p.sdo.t;
+    const uint32_t y_voff = (uint32_t)(((int64_t)(ts / C8) * yt + 8 * (ts % C8)) * 4);
+    f32x4 yr[CPT][2];
+    float r_lse[CPT], r_dl[CPT], r_dlo[CPT];
+    auto gload = [&](int q0, int lim) {
         const int rows = min(lim - q0, BQ);
-        const auto rq = row_rsrc((const float*)Q, p.sq.t, q0, rows, D);
-        const auto rdo = row_rsrc((const float*)dO, p.sdo.t, q0, rows, D);
+        const auto ry = row_rsrc(Y, yt, q0, rows, D);
 #pragma unroll
-        for (int i = 0; i < QLPT; ++i) {
-            ra[i] = buffer_ld4(rq, q_voff, (uint32_t)((int64_t)(NT * i / C4) * p.sq.t * 4));
-            rd[i] = buffer_ld4(rdo, do_voff, (uint32_t)((int64_t)(NT * i / C4) * p.sdo.t * 4));
+        for (int i = 0; i < CPT; ++i) {
+            const uint32_t so = (uint32_t)((int64_t)(256 * i / C8) * yt * 4);
+            yr[i][0] = buffer_ld4(ry, y_voff, so);
+            yr[i][1] = buffer_ld4(ry, y_voff + 16, so);
         }
-        // lanes past the tile's rows (all but the first BQ threads) read zeros
-        r_lse = buffer_ld1(row_rsrc(LSE, 1, q0, rows, 1), (uint32_t)tid * 4, 0);
-        r_dl = buffer_ld1(row_rsrc(DL, 1, q0, rows, 1), (uint32_t)tid * 4, 0);
-        // rows past the short ones (and every row outside key block 0) read 0
-        if constexpr (SHORT) {
-            const int n_sh = kblk == 0 ? max(0, min(p.n_short - q0, rows)) : 0;
-            r_dlo = buffer_ld1(row_rsrc(DLO, 1, q0, n_sh, 1), (uint32_t)tid * 4, 0);
+        if (role == 0) {
+            const int n_sh = SHORT && kblk == 0 ? max(0, min(p.n_short - q0, rows)) : 0;
+            const auto rl = row_rsrc(LSE, 1, q0, rows, 1), rd = row_rsrc(DL, 1, q0, rows, 1), ro = row_rsrc(DLO, 1, q0, n_sh, 1);
+#pragma unroll
+            for (int i = 0; i < CPT; ++i) {
+                const uint32_t off = (uint32_t)((ts + 256 * i) / C8) * 4;
+                r_lse[i] = buffer_ld1(rl, off, 0);
+                r_dl[i] = buffer_ld1(rd, off, 0);
+                r_dlo[i] = SHORT ? buffer_ld1(ro, off, 0) : 0.f;
+            }
         }
     };
-    auto sstore_q = [&]() {
+    // Everything that the workgroup starts from is loaded at once: its operand
+    // rows, K^T, the first Q / dO tile and the maxima of the head's Q and dO rows.
+    // The wave's operand, K or V rows of its pair's keys: MFMA step kk takes
+    // row key, columns 16 kk + 8 g .. + 7.
+    Half2x8 xf[NKB][NKK];
+    int xcls;  // its scale class
+    // K^T for the dQ product: unit f holds column f % D of the 8 keys that an
+    // operand takes together (16 m + 4 g' + {0..3} and + 8 for key group f / D =
+    // 2 m + g'), scaled as its pair's K rows are.
+    f32x4 kt[DQD ? 1 : KU][2];
+    auto kt_key = [](int f) { return 16 * (f / D >> 1) + 4 * (f / D & 1); };
+    {
+        const float* X = role ? (const float*)p.v + b * p.sv.b + h * p.sv.h : (const float*)p.k + b * p.sk.b + h * p.sk.h;
+        const int64_t xt = role ? p.sv.t : p.sk.t;
+        f32x4 raw[NKB][NKK][2];
 #pragma unroll
-        for (int i = 0; i < QLPT; ++i) {
+        for (int kb = 0; kb < NKB; ++kb) {
+            const int key = k0p + kb * 32 + l32;
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) {
+                raw[kb][kk][0] = raw[kb][kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (key < p.Tk) {
+                    raw[kb][kk][0] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g);
+                    raw[kb][kk][1] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g + 4);
+                }
+            }
+        }
+        if constexpr (!DQD) {
+            const float* K = (const float*)p.k + b * p.sk.b + h * p.sk.h;
+            const auto rk = row_rsrc(K, p.sk.t, k0, min(p.Tk - k0, BK), D);
+#pragma unroll
+            for (int i = 0; i < KU; ++i) {
+                const int f = tid + NT * i;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    kt[i][e >> 2][e & 3] = buffer_ld1(rk, (uint32_t)(((int64_t)kt_key(f) * p.sk.t + f % D) * 4),
+                                                      (uint32_t)((int64_t)((e & 3) + 8 * (e >> 2)) * p.sk.t * 4));
+            }
+        }
+        gload(q_begin, p.Tq);
+        const float* am = p.amax + (int64_t)bh * p.n_amax * 2;
+        float aq = 0.f, ad = 0.f;
+        for (int i = tid; i < p.n_amax; i += NT) {
+            aq = fmaxf(aq, am[2 * i]);
+            ad = fmaxf(ad, am[2 * i + 1]);
+        }
+        aq = wave_max(aq);
+        ad = wave_max(ad);
+        if (lane == 0) {
+            red_s[0][wave] = aq;
+            red_s[1][wave] = ad;
+        }
+        float amax = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) amax = absmax8_finite(amax, raw[kb][kk][0], raw[kb][kk][1]);
+        xcls = __builtin_amdgcn_readfirstlane(scale_class(wave_max(amax)));
+        const float xs = class_scale(xcls);
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) xf[kb][kk] = split2(raw[kb][kk][0], raw[kb][kk][1], xs);
+        if (role == 0 && lane == 0) kcls_s[pr] = xcls;
+    }
+    int qcls, docls;  // scale classes of the head's Q and dO rows, from bwd_pre's maxima
+    __syncthreads();
+    {
+        float aq = 0.f, ad = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            aq = fmaxf(aq, red_s[0][w]);
+            ad = fmaxf(ad, red_s[1][w]);
+        }
+        qcls = __builtin_amdgcn_readfirstlane(scale_class(aq));
+        docls = __builtin_amdgcn_readfirstlane(scale_class(ad));
+    }
+    if constexpr (!DQD) {
+#pragma unroll
+        for (int i = 0; i < KU; ++i) {
             const int f = tid + NT * i;
-            *reinterpret_cast<f32x4*>(&Qs[f / C4][4 * (f % C4)]) = ra[i];
-            *reinterpret_cast<f32x4*>(&dOs[f / C4][4 * (f % C4)]) = rd[i];
+            const Half2x8 k = split2(kt[i][0], kt[i][1], class_scale(kcls_s[kt_key(f) / KP]));
+            Kt[0][f / D][f % D] = k.h;
+            Kt[1][f / D][f % D] = k.l;
         }
-        if (tid < BQ) {
-            lse_s[tid] = r_lse * kLseStage;
-            dl_s[tid] = r_dl;
-            if constexpr (SHORT) dlo_s[tid] = r_dlo;
+    }
+    const float qinv = class_inv(qcls), doinv = class_inv(docls);
+    const float xinv = class_inv(xcls);
+    const float ytile = class_scale(role ? qcls : docls);  // scale of the rows this wave stages
+    const float cs = p.c * xinv * qinv;                     // role 0: scores in exp2 units are S cs
+    const float dsu = kBwdPInv * xinv * doinv;              // role 1: dS = ds dsu, ds = (2^14 P) (dP' - delta')
+    const float xscale = class_scale(xcls);                 // role 1
+
+    auto sstore = [&](int buf) {
+        int ts = tid & 255;
+        if constexpr (D == 64 && KP == 64) asm volatile("" : "+v"(ts));
+        _Float16* dst = role ? &Qs[buf][0][0][0] : &dOs[0][0][0];
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int f = ts + 256 * i;
+            float ys = ytile;
+            int rc = docls;
+            if (role == 0) {  // a dO row by its own class: rows may differ by many binades
+                rc = scale_class(group_max<C8>(absmax8_finite(0.f, yr[i][0], yr[i][1])));
+                ys = class_scale(rc);
+            }
+            const Half2x8 y = split2(yr[i][0], yr[i][1], ys);
+            if (NCH % 256 == 0 || f < NCH) {
+                *reinterpret_cast<f16x8*>(dst + (f / C8) * QS + 8 * (f % C8)) = y.h;
+                *reinterpret_cast<f16x8*>(dst + (BQ + f / C8) * QS + 8 * (f % C8)) = y.l;
+                if (role == 0 && f % C8 == 0) {
+                    // P carries the row's unit over the head's, so that dV and dS sum
+                    // rows in one unit: 2^14 P 2^(8 (rc - docls)) = exp2(S c - lse_s)
+                    const int r = f / C8;
+                    lse_s[r] = fmaf(r_lse[i], kLog2e, (float)(8 * (docls - rc)) - kBwdPBits);
+                    dl_s[r] = r_dl[i] * ys;
+                    if constexpr (SHORT) {
+                        dlo_s[r] = r_dlo[i] * ys;
+                        dinv_s[r] = class_inv(rc);
+                    }
+                }
+            }
         }
     };
+
     // Short rows (bwd_split.h): before the main loop, their delta from this
-    // block's own S and dP.  Per short tile each wave forms S^T and dP^T of its
-    // 32 keys (the main loop's chains with the operands swapped, so lane
-    // (l32, g) holds query q0 + l32 and keys 8 (r / 4) + 4 g + r % 4 of the
-    // wave), the weights e = exp2(S c - lse log2 e) (1 for a one-key row's
-    // key), and per query sum(e) and sum(e dP) in fp64 (exact products) over
-    // its registers and the lane pair (l32, l32 + 32); the workgroup's first
-    // BQ threads add the waves' sums in wave order and store delta = sum(e dP)
-    // / sum(e) as hi + lo.  Each tile's loads are issued while the previous one
-    // computes; the main loop's first barrier orders the last sums' reads
-    // before it writes the dS tile they sit in.
+    // block's own S and dP.  Per short tile the pair's waves form S^T and dP^T
+    // (the main loop's products with the operands swapped, in the same order, so
+    // lane (l32, g) holds query q0 + l32 and keys 32 kb + 8 (r / 4) + 4 g + r % 4
+    // of the pair), role 0 hands over the weights e = exp2(S c - lse log2 e) (1 for
+    // a one-key row's key), and role 1 sums e and e dP in fp64 (exact products)
+    // over its registers and the lane pair; the first BQ threads add the pairs'
+    // sums in order and store delta = sum(e dP) / sum(e) as hi + lo.
     const int qs_end = SHORT && kblk == 0 ? min(q_end, p.n_short) : q_begin;  // short tiles: [q_begin, qs_end)
     if (SHORT && q_begin < qs_end) {
-        double* part = reinterpret_cast<double*>(&dSs[0][0]);  // [NW][BQ] pairs (sum e, sum e dP)
-        static_assert(2 * NW * BQ * sizeof(double) <= sizeof(dSs), "the sums fit the dS tile");
-        gload_q(q_begin, p.Tq);
+        double* part = reinterpret_cast<double*>(&Qs[1][0][0][0]);  // [4][BQ] pairs (sum e, sum e dP)
+        static_assert(2 * 4 * BQ * sizeof(double) <= sizeof(Qs[1]), "the sums fit the second Q buffer");
         for (int q0 = q_begin; q0 < qs_end; q0 += BQ) {
-            sstore_q();
+            sstore(0);
             __syncthreads();
-            if (q0 + BQ < qs_end) gload_q(q0 + BQ, p.Tq);
-            double l = 0.0, w = 0.0;
-            if ((!p.causal || (q0 + BQ - 1 + p.off >= k0w)) && k0w < p.Tk) {
-                f32x16 st, dpt;
+            gload(q0 + BQ, q0 + BQ < qs_end ? p.Tq : 0);
+            const bool active = (!p.causal || (q0 + BQ - 1 + p.off >= k0p)) && k0p < p.Tk;
+            f32x16 st[NKB];
+            f32x4* X = reinterpret_cast<f32x4*>(&Xs[pr][0]);
+            if (active) {
+                const _Float16* rows = role ? &dOs[0][0][0] : &Qs[0][0][0][0];
 #pragma unroll
-                for (int i = 0; i < HD; i += 4) {
-                    const f32x4 qa = *reinterpret_cast<const f32x4*>(&Qs[l32][g * HD + i]);
-                    const f32x4 da = *reinterpret_cast<const f32x4*>(&dOs[l32][g * HD + i]);
-                    st = mfma32x32x2(kf[i + 0], qa[0], i == 0 ? f32x16{} : st);
-                    dpt = mfma32x32x2(vf[i + 0], da[0], i == 0 ? f32x16{} : dpt);
-                    st = mfma32x32x2(kf[i + 1], qa[1], st);
-                    dpt = mfma32x32x2(vf[i + 1], da[1], dpt);
-                    st = mfma32x32x2(kf[i + 2], qa[2], st);
-                    dpt = mfma32x32x2(vf[i + 2], da[2], dpt);
-                    st = mfma32x32x2(kf[i + 3], qa[3], st);
-                    dpt = mfma32x32x2(vf[i + 3], da[3], dpt);
+                for (int kk = 0; kk < NKK; ++kk) {
+                    Half2x8 y;
+                    y.h = *reinterpret_cast<const f16x8*>(rows + l32 * QS + 16 * kk + 8 * g);
+                    y.l = *reinterpret_cast<const f16x8*>(rows + (BQ + l32) * QS + 16 * kk + 8 * g);
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb) st[kb] = mfma_split<true>(xf[kb][kk], y, kk == 0 ? f32x16{} : st[kb]);
                 }
-                const int qi = q0 + l32;
-                const float L = lse_s[l32] * kLseRead;
+                if (role == 0) {
+                    const int qi = q0 + l32;
+                    const float L = lse_s[l32];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int kj = k0w + 8 * (r >> 2) + 4 * g + (r & 3);
-                    const bool vis = (qi < p.Tq) && (kj < p.Tk) && (!p.causal || kj <= qi + p.off);
-                    const float e = bwd_short_weight(p, qi, vis, fast_exp2(fmaf(st[r], c, -L)));
-                    l += (double)e;
-                    w += (double)e * (double)dpt[r];
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            f32x4 e;
+#pragma unroll
+                            for (int cc = 0; cc < 4; ++cc) {
+                                const int kj = k0p + 32 * kb + 8 * j + 4 * g + cc;
+                                const bool vis = (qi < p.Tq) && (kj < p.Tk) && (!p.causal || kj <= qi + p.off);
+                                e[cc] = bwd_short_weight(p, qi, vis, fast_exp2(fmaf(st[kb][4 * j + cc], cs, -L)) * kBwdPInv);
+                            }
+                            X[(4 * kb + j) * 64 + lane] = e;
+                        }
                 }
             }
-            l += __shfl_xor(l, 32);
-            w += __shfl_xor(w, 32);
-            if (g == 0) {
-                part[2 * (wave * BQ + l32)] = l;
-                part[2 * (wave * BQ + l32) + 1] = w;
+            __syncthreads();
+            if (role == 1) {
+                double l = 0.0, w = 0.0;
+                if (active) {
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const f32x4 e = X[(4 * kb + j) * 64 + lane];
+#pragma unroll
+                            for (int cc = 0; cc < 4; ++cc) {
+                                l += (double)e[cc];
+                                w += (double)e[cc] * (double)st[kb][4 * j + cc];
+                            }
+                        }
+                }
+                l += __shfl_xor(l, 32);
+                w += __shfl_xor(w, 32);
+                if (g == 0) {
+                    part[2 * (pr * BQ + l32)] = l;
+                    part[2 * (pr * BQ + l32) + 1] = w * ((double)xinv * (double)dinv_s[l32]);
+                }
             }
             __syncthreads();
-            if (tid < BQ) bwd_short_delta_store<NW, BQ>(p, bh, q0 + tid, part + 2 * tid);
+            if (tid < BQ) bwd_short_delta_store<4, BQ>(p, bh, q0 + tid, part + 2 * tid);
         }
+        __syncthreads();  // the deltas are stored: the first tile's are read again
+        gload(q_begin, p.Tq);
     }
 
-    // K^T of the whole key block in LDS, for the dQ product.
+    f32x16 acc[NDB][NKB];  // dV^T (role 0) or dK^T (role 1): row d, column key
 #pragma unroll
-    for (int i = 0; i < KLPT; ++i) {
-        const int f = tid + NT * i;
-        const int r = f / C4;
-        const int c4 = f % C4;
-        f32x4 val = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (k0 + r < p.Tk) val = ld4(K + (int64_t)(k0 + r) * p.sk.t + 4 * c4);
-        Kts[4 * c4 + 0][r] = val[0];
-        Kts[4 * c4 + 1][r] = val[1];
-        Kts[4 * c4 + 2][r] = val[2];
-        Kts[4 * c4 + 3][r] = val[3];
-    }
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = f32x16{};
+    int dscls = 2;  // role 1: class of the largest |ds| so far
 
+    sstore(0);
+    __syncthreads();
 
-    // With PF the next tile's loads are in flight while a tile computes.
-    // Without short rows (EARLY) they are issued right after the store that
-    // frees their registers, ahead of the tile's dQ atomics, so the store's
-    // wait for them (the memory counter drains in issue order) does not wait
-    // for the atomics as well (config 2 302 -> 297 us); the short-row
-    // variant, tighter on registers, measured 3% slower that way and issues
-    // them at the top of the tile.
-    constexpr bool EARLY = PF && !SHORT;
-    // Without PF (D = 128) a tile's loads go out in the previous tile's dQ
-    // section (ahead of its atomics, where fewer registers are live) and are
-    // stored at the top of the tile (B8 H12 T1024 686 -> 678 us, config 4
-    // 5972 -> 5937 us).
-    constexpr bool LATE_EARLY = !PF;
-    if constexpr (PF) {
-        gload_q(q_begin, p.Tq);
-        sstore_q();
+    int buf = 0;
+    for (int q0 = q_begin; q0 < q_end; q0 += BQ, buf ^= 1) {
+        // At D = 64 the lane number passes an empty asm, so that LDS addresses are
+        // formed in each tile instead of being held (and spilled) across the loop.
+        int ln = lane;
+        if constexpr (D == 64 && KP == 64) asm volatile("" : "+v"(ln));
+        const int lane = ln, l32 = ln & 31, g = ln >> 5;
+        // ---- A: S and P (role 0), dP (role 1) -----------------------------------
+        gload(q0 + BQ, q0 + BQ < q_end ? p.Tq : 0);
+        // Does any query of this tile see any key of this pair?
+        const bool active = (!p.causal || (q0 + BQ - 1 + p.off >= k0p)) && k0p < p.Tk;
+        f32x4* X = reinterpret_cast<f32x4*>(&Xs[pr][0]);
+        f32x16 s[NKB];
+        if (active) {
+            const _Float16* rows = role ? &dOs[0][0][0] : &Qs[buf][0][0][0];
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) {
+                Half2x8 y;
+                y.h = *reinterpret_cast<const f16x8*>(rows + l32 * QS + 16 * kk + 8 * g);
+                y.l = *reinterpret_cast<const f16x8*>(rows + (BQ + l32) * QS + 16 * kk + 8 * g);
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) s[kb] = mfma_split<false>(y, xf[kb][kk], kk == 0 ? f32x16{} : s[kb]);
+            }
+            // reg 4j + cc of s[kb]: query row 8 j + 4 g + cc of the tile, key 32 kb + l32 of the pair
+            if (role == 0) {
+                // Only tiles that cross the causal diagonal or the end of the
+                // queries / keys evaluate the visibility test.
+                auto prob = [&](auto masked) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const f32x4 L = *reinterpret_cast<const f32x4*>(&lse_s[8 * j + 4 * g]);
+#pragma unroll
+                        for (int kb = 0; kb < NKB; ++kb) {
+                            f32x4 e;
+#pragma unroll
+                            for (int cc = 0; cc < 4; ++cc) {
+                                float pv = fast_exp2(fmaf(s[kb][4 * j + cc], cs, -L[cc]));
+                                if constexpr (decltype(masked)::value) {
+                                    const int qi = q0 + 8 * j + 4 * g + cc, key = k0p + 32 * kb + l32;
+                                    const bool vis = (qi < p.Tq) && (key < p.Tk) && (!p.causal || key <= qi + p.off);
+                                    pv = vis ? pv : 0.f;
+                                }
+                                s[kb][4 * j + cc] = e[cc] = pv;
+                            }
+                            X[(4 * kb + j) * 64 + lane] = e;
+                        }
+                    }
+                };
+                if (q0 + BQ > p.Tq || k0p + KP > p.Tk || (p.causal && k0p + KP - 1 > q0 + p.off))
+                    prob(std::true_type{});
+                else
+                    prob(std::false_type{});
+            }
+        }
         __syncthreads();
-        if constexpr (EARLY) gload_q(q_begin + BQ, q_begin + BQ < q_end ? p.Tq : 0);
-    }
-    if constexpr (LATE_EARLY) gload_q(q_begin, p.Tq);
 
-    for (int q0 = q_begin; q0 < q_end; q0 += BQ) {
-        if constexpr (PF && !EARLY) {
-            gload_q(q0 + BQ, q0 + BQ < q_end ? p.Tq : 0);
-        } else if constexpr (LATE_EARLY) {
-            sstore_q();
-            __syncthreads();
-        }
-
-        // Does any query of this tile see any key of this wave?
-        const bool active = !p.causal || (q0 + BQ - 1 + p.off >= k0w);
-        f32x16 ds;
-        if (active && k0w < p.Tk) {
-            f32x16 s, dp;
-#pragma unroll
-            for (int i = 0; i < HD; i += 4) {
-                const f32x4 qa = *reinterpret_cast<const f32x4*>(&Qs[l32][g * HD + i]);
-                const f32x4 da = *reinterpret_cast<const f32x4*>(&dOs[l32][g * HD + i]);
-                s = mfma32x32x2(qa[0], kf[i + 0], i == 0 ? f32x16{} : s);  // zero accumulator as an operand
-                dp = mfma32x32x2(da[0], vf[i + 0], i == 0 ? f32x16{} : dp);
-                s = mfma32x32x2(qa[1], kf[i + 1], s);
-                dp = mfma32x32x2(da[1], vf[i + 1], dp);
-                s = mfma32x32x2(qa[2], kf[i + 2], s);
-                dp = mfma32x32x2(da[2], vf[i + 2], dp);
-                s = mfma32x32x2(qa[3], kf[i + 3], s);
-                dp = mfma32x32x2(da[3], vf[i + 3], dp);
-            }
-            // P and dS; reg r holds query row 8*(r/4) + 4*g + r%4 of the tile.
-            // Only tiles that cross the causal diagonal or the end of the
-            // queries / keys evaluate the visibility test.
-            auto p_ds = [&](auto masked) {
+        // ---- B: dV (role 0), dS (role 1) -----------------------------------------
+        Half2x8 pb[NKB][2];  // P or dS: queries 16 mm + 4 g + {0..3} and + 8 of key block kb
+        if (active) {
+            if (role == 1) {
+                float mx = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const f32x4 L = *reinterpret_cast<const f32x4*>(&lse_s[8 * j + 4 * g]) * kLseRead;
                     const f32x4 Dl = *reinterpret_cast<const f32x4*>(&dl_s[8 * j + 4 * g]);
                     const f32x4 Dlo = SHORT ? *reinterpret_cast<const f32x4*>(&dlo_s[8 * j + 4 * g])
                                             : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) {
-                        const int r = 4 * j + cc;
-                        float pr = fast_exp2(fmaf(s[r], c, -L[cc]));
-                        if constexpr (decltype(masked)::value) {
-                            const int qi = q0 + 8 * j + 4 * g + cc;
-                            const bool vis = (qi < p.Tq) && (key < p.Tk) && (!p.causal || key <= qi + p.off);
-                            pr = vis ? pr : 0.f;
+                    for (int kb = 0; kb < NKB; ++kb) {
+                        const f32x4 pv = X[(4 * kb + j) * 64 + lane];
+#pragma unroll
+                        for (int cc = 0; cc < 4; ++cc) {
+                            float t = fmaf(-Dl[cc], xscale, s[kb][4 * j + cc]);
+                            if constexpr (SHORT) t = fmaf(-Dlo[cc], xscale, t);
+                            s[kb][4 * j + cc] = pv[cc] * t;
                         }
-                        s[r] = pr;
-                        ds[r] = pr * (SHORT ? (dp[r] - Dl[cc]) - Dlo[cc] : dp[r] - Dl[cc]);
                     }
                 }
-            };
-            const bool need_mask = q0 + BQ > p.Tq || k0w + 32 > p.Tk || (p.causal && k0w + 31 > q0 + p.off);
-            if (need_mask)
-                p_ds(std::true_type{});
-            else
-                p_ds(std::false_type{});
-            // A row with one visible key: dS = P (dP - dP) = 0.  (At D = 32 without
-            // short rows the kernel keeps three workgroups per CU only without this
-            // fix, 168 VGPRs; its short-row prologue, on small problems, forms
-            // delta = dP bit for bit instead.)
-            if constexpr (D != 32 || SHORT) {
-                if (bwd_one_key_tile(p, q0, k0w)) {
+                // A row with one visible key: dS = P (dP - dP) = 0.
+                if (bwd_one_key_tile(p, q0, k0p)) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
-                        if (bwd_one_key_row(p, q0 + 8 * (r >> 2) + 4 * g + (r & 3))) ds[r] = 0.f;
+                        if (bwd_one_key_row(p, q0 + 8 * (r >> 2) + 4 * g + (r & 3))) s[0][r] = 0.f;
                 }
-            }
-            // dV^T += dO^T P ; dK^T += Q^T dS
 #pragma unroll
-            for (int kk = 0; kk < 16; ++kk) {
-                const int qr = 8 * (kk >> 2) + 4 * g + (kk & 3);
+                for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 16; r += 8)
+                        mx = absmax8(mx, f32x4{s[kb][r], s[kb][r + 1], s[kb][r + 2], s[kb][r + 3]},
+                                     f32x4{s[kb][r + 4], s[kb][r + 5], s[kb][r + 6], s[kb][r + 7]});
+                if (__any(mx >= class_limit(dscls))) {  // dK^T is kept in units of ds's scale
+                    mx = 0.f;
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, finite_abs(s[kb][r]));
+                    const int nc = max(dscls, min(31, __builtin_amdgcn_readfirstlane(scale_class(wave_max(mx)))));
+                    const float f = class_scale(nc) * class_inv(dscls);
+#pragma unroll
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int kb = 0; kb < NKB; ++kb) acc[db][kb] *= f;
+                    dscls = nc;
+                }
+                if (lane == 0) dqcls_s[pr] = dscls + xcls + kcls_s[pr];
+            }
+            const float psc = role ? class_scale(dscls) : 1.f;
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm) {
+                    const f32x16& e = s[kb];
+                    pb[kb][mm] = split2(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
+                                        f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]}, psc);
+                }
+        } else if (role == 1 && !DQD) {
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm) pb[kb][mm] = Half2x8{};
+            if (lane == 0) dqcls_s[pr] = -1;
+        }
+        if (role == 1 && !DQD) {
+            {
+                // dS over P (read above by this wave): row key l32, queries along it
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                    for (int mm = 0; mm < 2; ++mm)
+#pragma unroll
+                        for (int hl = 0; hl < 2; ++hl) {
+                            const f16x8 v = hl ? pb[kb][mm].l : pb[kb][mm].h;
+                            _Float16* row = reinterpret_cast<_Float16*>(&Xs[pr][(2 * kb + hl) * XB]) + l32 * SS + 16 * mm + 4 * g;
+                            *reinterpret_cast<f16x4*>(row) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+                            *reinterpret_cast<f16x4*>(row + 8) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+                        }
+            }
+        }
+        // acc += rows^T pb (dO^T P or Q^T dS), rows read transposed
+        auto accumulate = [&](const _Float16* rows) {
+            const int a_off = (4 * (ln >> 5) + ((ln & 15) >> 2)) * QS + 16 * ((ln >> 4) & 1) + 4 * (ln & 3);
+#pragma unroll
+            for (int mm = 0; mm < 2; ++mm)
 #pragma unroll
                 for (int db = 0; db < NDB; ++db) {
-                    const float ado = dOs[qr][db * 32 + l32];
-                    const float aq = Qs[qr][db * 32 + l32];
-                    dv_acc[db] = mfma32x32x2(ado, s[kk], dv_acc[db]);
-                    dk_acc[db] = mfma32x32x2(aq, ds[kk], dk_acc[db]);
+                    const _Float16* at = rows + a_off + 16 * mm * QS + db * 32;
+                    Half2x8 a;
+                    a.h = tr_frag([&](int r) { return at + r * QS; });
+                    a.l = tr_frag([&](int r) { return at + (BQ + r) * QS; });
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = mfma_split(a, pb[kb][mm], acc[db][kb]);
                 }
-            }
-        } else {
-            ds = f32x16{};
-        }
-        // dS block of this wave -> LDS (rows = queries, columns = the 128 keys);
-        // with the query-major dQ pass (dq_direct) there is no dQ product here
-        if (!p.dq_direct) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) dSs[8 * (r >> 2) + 4 * g + (r & 3)][wave * 32 + l32] = ds[r];
-        }
+        };
+        if (active && role == 0) accumulate(&dOs[0][0][0]);
         __syncthreads();
-        if constexpr (PF) sstore_q();  // the next tile (zeros after the last one, never read)
-        if constexpr (EARLY) gload_q(q0 + 2 * BQ, q0 + 2 * BQ < q_end ? p.Tq : 0);
-        if constexpr (LATE_EARLY) gload_q(q0 + BQ, q0 + BQ < q_end ? p.Tq : 0);
-        if (p.dq_direct) {
-            __syncthreads();
-            continue;
-        }
 
-        // ---- dQ tile (32 x D) += dS (32 x BK) K (BK x D) ---------------------
-        // Each wave takes NDQ / NW adjacent 16x16 blocks; lane group g4
-        // reduces keys g4 * BK/4 .. + BK/4 - 1.  fp32 atomics through a buffer
-        // resource over the tile's rows: rows past Tq fall outside it and the
-        // hardware drops those adds.
-        const auto rdq = row_rsrc(dQa, p.sacc.t, q0, min(p.Tq - q0, BQ), D);
+        // ---- C: dQ (both), dK (role 1), the next dO tile (role 0) ------------------
+        sstore(buf ^ 1);
+        if (active && role == 1) accumulate(&Qs[buf][0][0][0]);
+        if constexpr (!DQD) {
+            if (role == 0) {
+                // dQ tile (32 x D) = dS K: a wave takes a 32-wide head-dim block, over all
+                // of the workgroup's keys at D = 128 and a half (a quarter) of them at
+                // D = 64 (32), and adds it to the global accumulator with fp32 atomics.
+                // (One 16x16 block per wave of both roles over all keys made this phase
+                // LDS-bound: twice the operand bytes.  Adding the waves' shares in LDS
+                // took 160 cycles per ds_add_f32.)
+                const int db = pr % NDB;
+                f32x16 dq = f32x16{};
+                int unit = -1;  // dq is in units of 2^(8 unit)
 #pragma unroll
-        for (int bi = 0; bi < NDQ / NW; ++bi) {
-            const int blk = wave * (NDQ / NW) + bi;  // adjacent blocks share K^T rows
-            const int qh = blk & 1;
-            const int dc = blk >> 1;
-            f32x4 acc;
+                for (int pi = 0; pi < DQP; ++pi) {
+                    const int pp = pr / NDB * DQP + pi;
+                    const int u = __builtin_amdgcn_readfirstlane(dqcls_s[pp]);  // < 0: the pair's dS is zero
+                    const int d = u >= 0 && unit >= 0 ? min(max(unit - u, -15), 15) : 0;
+                    unit = u >= 0 ? u : unit;
+                    if (pi > 0) dq *= __uint_as_float((uint32_t)(127 + 8 * d) << 23);
 #pragma unroll
-            for (int kk = 0; kk < BK / 4; kk += 4) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&dSs[16 * qh + l16][g4 * (BK / 4) + kk]);
-                const f32x4 bb = *reinterpret_cast<const f32x4*>(&Kts[16 * dc + l16][g4 * (BK / 4) + kk]);
-                acc = mfma16x16x4(a[0], bb[0], kk == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc);
-                acc = mfma16x16x4(a[1], bb[1], acc);
-                acc = mfma16x16x4(a[2], bb[2], acc);
-                acc = mfma16x16x4(a[3], bb[3], acc);
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int m = 0; m < 2; ++m) {
+                            const _Float16* ds = reinterpret_cast<const _Float16*>(&Xs[pp][2 * kb * XB]) +
+                                                 (16 * m + 4 * g + ((lane & 15) >> 2)) * SS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+                            Half2x8 a, kf;
+                            a.h = tr_frag([&](int r) { return ds + r * SS; });
+                            a.l = tr_frag([&](int r) { return ds + XB / 2 + r * SS; });
+                            kf.h = Kt[0][(pp * KP + 32 * kb + 16 * m) / 8 + g][db * 32 + l32];
+                            kf.l = Kt[1][(pp * KP + 32 * kb + 16 * m) / 8 + g][db * 32 + l32];
+                            dq = mfma_split(a, kf, dq);
+                        }
+                }
+                const float f = ldexpf(kBwdPInv * doinv * p.scale, 8 * unit - 414);
+                const auto rdq = row_rsrc(dQa, p.sacc.t, q0, min(p.Tq - q0, BQ), D);  // rows past Tq are dropped
+                const uint32_t voff = (uint32_t)(((int64_t)(4 * g) * p.sacc.t + db * 32 + l32) * 4);
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    buffer_atomic_add(rdq, dq[r] * f, voff, (uint32_t)((int64_t)(8 * (r >> 2) + (r & 3)) * p.sacc.t * 4));
             }
-            const uint32_t voff = (uint32_t)(((int64_t)(16 * qh + 4 * g4) * p.sacc.t + 16 * dc + l16) * 4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                buffer_atomic_add(rdq, acc[r] * p.scale, voff, (uint32_t)((int64_t)r * p.sacc.t * 4));
         }
         __syncthreads();
     }
 
     // ---- dK = scale * dK^T^T, dV = dV^T^T ------------------------------------------
-    if (!bwd_fixup<NT>(p, wk, dk_acc, dv_acc)) return;
-    if (key < p.Tk) {
-        E* dKp = (E*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)key * p.sdk.t;
-        E* dVp = (E*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)key * p.sdv.t;
+    const float unit = role ? class_inv(dscls) * dsu * qinv * p.scale : kBwdPInv * doinv;
+    f32x16 out[NDB * NKB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) out[db * NKB + kb] = acc[db][kb] * unit;
+    if (!bwd_fixup<NT>(p, wk, out)) return;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+        const int key = k0p + 32 * kb + l32;
+        if (key >= p.Tk) continue;
+        float* dst = role ? (float*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)key * p.sdk.t
+                          : (float*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)key * p.sdv.t;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                f32x4 a, v;
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc) {
-                    a[cc] = dk_acc[db][4 * j + cc] * p.scale;
-                    v[cc] = dv_acc[db][4 * j + cc];
-                }
-                st4(dKp + db * 32 + 8 * j + 4 * g, a);
-                st4(dVp + db * 32 + 8 * j + 4 * g, v);
+                const f32x16& v = out[db * NKB + kb];
+                st4(dst + db * 32 + 8 * j + 4 * g, f32x4{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]});
             }
     }
 }
@@ -548,13 +746,15 @@ __global__ __launch_bounds__(256) void bwd_cvt_kernel(BwdParams p) {
 // Query-major dQ pass, fp32 (the deterministic mode: the main kernel then
 // skips its dQ product).  One workgroup = 4 waves x 32 query rows of one
 // (b, h), laid out as the forward: each lane keeps its query row of Q and dO
-// as the B operand (Q^T, dO^T) in VGPRs, with that row's log-sum-exp and
-// delta; tiles of 32 keys stream through LDS as K and V rows and K^T
-// (double-buffered, one barrier per tile).  Per wave and tile:
-//   S^T = K Q^T, dP^T = V dO^T        v_mfma_f32_32x32x2_f32, A from LDS
+// as split B operands (Q^T, dO^T) in VGPRs, with that row's log-sum-exp and
+// delta; tiles of 32 keys of K and V, split, are double-buffered in LDS (loaded
+// two tiles ahead, scaled by the class of the largest magnitude so far).  Per
+// wave and tile:
+//   S^T = K Q^T, dP^T = V dO^T        in the forward's and the main kernel's
+//                                     order, to the same bits
 //   P^T = exp2(S^T c - lse log2 e), dS^T = P^T (dP^T - delta)
-//   dQ^T += K^T dS^T                  B = dS^T straight from the accumulators
-//                                     (as the forward feeds P^T to P V)
+//   dQ^T += K^T dS^T                  A = K^T read transposed from the K rows,
+//                                     B = dS^T straight from the accumulators
 // dQ stays in VGPRs and is stored once, times the scale: every element is the
 // sum of its key tiles in key order, with no accumulator, zeroing or atomics,
 // so the result is the same on every run.  It recomputes S and dP (two more
@@ -563,24 +763,24 @@ template <int D>
 __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams p) {
     constexpr int BM = kBwdDqBM;
     constexpr int BN = 32;               // keys per tile
-    constexpr int HD = D / 2;            // reduction elements per lane half
+    constexpr int NKK = D / 16;          // MFMA steps along the head dim
     constexpr int NDB = D / 32;          // 32-wide d blocks of dQ^T
-    constexpr int C4 = D / 4;            // 4-element chunks per row
-    constexpr int KS = D + 4;            // K / V row stride in LDS (floats)
-    constexpr int TS = BN + 4;           // K^T row stride in LDS (floats)
-    constexpr int LPT = BN * C4 / 256;   // 4-element loads per thread per tensor per tile
-    static_assert(BM == 128 && BN * C4 % 256 == 0, "4 waves x 32 rows, whole staging passes");
-    static_assert(256 % C4 == 0, "chunk rows must split into thread + load parts");
+    constexpr int C8 = D / 8;            // 8-element chunks per row
+    constexpr int NCH = BN * C8;         // chunks of a tile
+    constexpr int CPT = (NCH + 255) / 256;
+    constexpr int QS = BwdTile<D, 32>::QS;
+    static_assert(BM == 128 && 256 % C8 == 0, "4 waves x 32 rows, whole staging passes");
 
-    __shared__ __attribute__((aligned(16))) float Ks[2][BN][KS];
-    __shared__ __attribute__((aligned(16))) float Vs[2][BN][KS];
-    __shared__ __attribute__((aligned(16))) float Kt[2][D][TS];
+    __shared__ __attribute__((aligned(16))) _Float16 Ks[2][2][BN][QS];  // [buffer][part]
+    __shared__ __attribute__((aligned(16))) _Float16 Vs[2][2][BN][QS];
+    __shared__ int cls_s[2][2][4];  // scale class that each wave's loads need: [K, V][tile parity]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31;
     const int g = lane >> 5;
+    const int tr_row = (lane & 15) >> 2, tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
     const int BH = p.B * p.H;
     const int w = blockIdx.x;
@@ -596,25 +796,35 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
 
     const int q0w = qtile * BM + wave * 32;
     const int qrow = q0w + l32;
-    // B operands: lane (l32, g) holds row qrow, columns g*HD + i.
-    float qf[HD], df[HD];
-    if (qrow < p.Tq) {
-        const float* qs = Q + (int64_t)qrow * p.sq.t + g * HD;
-        const float* ds = dO + (int64_t)qrow * p.sdo.t + g * HD;
+    // B operands: MFMA step kk takes row qrow, columns 16 kk + 8 g .. + 7, scaled by the row's class.
+    Half2x8 qf[NKK], df[NKK];
+    float qinv, doscale, doinv;
+    auto load_row = [&](const float* src, int64_t st, Half2x8 (&f)[NKK]) {
+        f32x4 raw[NKK][2];
+        float amax = 0.f;
 #pragma unroll
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = ld4(qs + i);
-            const f32x4 c = ld4(ds + i);
-            qf[i] = a[0]; qf[i + 1] = a[1]; qf[i + 2] = a[2]; qf[i + 3] = a[3];
-            df[i] = c[0]; df[i + 1] = c[1]; df[i + 2] = c[2]; df[i + 3] = c[3];
+        for (int kk = 0; kk < NKK; ++kk) {
+            raw[kk][0] = raw[kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (qrow < p.Tq) {
+                raw[kk][0] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g);
+                raw[kk][1] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g + 4);
+            }
+            amax = absmax8_finite(amax, raw[kk][0], raw[kk][1]);
         }
-    } else {
+        const int k = scale_class(max_xor32(amax));
 #pragma unroll
-        for (int i = 0; i < HD; ++i) qf[i] = df[i] = 0.f;
+        for (int kk = 0; kk < NKK; ++kk) f[kk] = split2(raw[kk][0], raw[kk][1], class_scale(k));
+        return k;
+    };
+    qinv = class_inv(load_row(Q, p.sq.t, qf));
+    {
+        const int k = load_row(dO, p.sdo.t, df);
+        doscale = class_scale(k);
+        doinv = class_inv(k);
     }
-    const float Lq = qrow < p.Tq ? p.lse[(int64_t)bh * p.Tq + qrow] * kLog2e : 0.f;
-    const float Dq = qrow < p.Tq ? p.delta[(int64_t)bh * p.Tq + qrow] : 0.f;
-    const float Dqlo = bwd_short_row(p, qrow) ? p.delta_lo[(int64_t)bh * p.Tq + qrow] : 0.f;
+    const float Lq = qrow < p.Tq ? fmaf(p.lse[(int64_t)bh * p.Tq + qrow], kLog2e, -kBwdPBits) : 0.f;
+    const float Dq = qrow < p.Tq ? p.delta[(int64_t)bh * p.Tq + qrow] * doscale : 0.f;
+    const float Dqlo = bwd_short_row(p, qrow) ? p.delta_lo[(int64_t)bh * p.Tq + qrow] * doscale : 0.f;
     const bool one_key = qrow < p.Tq && bwd_one_key_row(p, qrow);
     const bool one_key_wave = p.causal ? (-p.off >= q0w && -p.off < q0w + 32) : p.Tk == 1;  // wave-uniform
 
@@ -623,71 +833,119 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
     const int nt = (kv_end + BN - 1) / BN;
     const int wave_kend = p.causal ? min(kv_end, q0w + 32 + p.off) : kv_end;
 
-    // Chunk f of a tile -> (row f / C4, column chunk f % C4); chunk tid + 256 i
-    // is 256 i / C4 rows below chunk tid.  Rows at or past the resource's end
-    // (<= Tk) read as zeros.
-    f32x4 kr[LPT], vr[LPT];
-    const uint32_t k_voff = (uint32_t)(((int64_t)(tid / C4) * p.sk.t + 4 * (tid % C4)) * 4);
-    const uint32_t v_voff = (uint32_t)(((int64_t)(tid / C4) * p.sv.t + 4 * (tid % C4)) * 4);
-    auto gload = [&](int u) {
+    // Chunk tid + 256 i of a tile: row f / C8, 8 columns from 8 (f % C8).  Rows at
+    // or past the resource's end (<= Tk) read as zeros.
+    struct Raw {
+        f32x4 k[CPT][2], v[CPT][2];
+    };
+    const uint32_t k_voff = (uint32_t)(((int64_t)(tid / C8) * p.sk.t + 8 * (tid % C8)) * 4);
+    const uint32_t v_voff = (uint32_t)(((int64_t)(tid / C8) * p.sv.t + 8 * (tid % C8)) * 4);
+    auto gload = [&](Raw& r, int u) {
         const int rows = u < nt ? min(p.Tk - u * BN, BN) : 0;
         const auto rk = row_rsrc(K, p.sk.t, u * BN, rows, D);
         const auto rv = row_rsrc(V, p.sv.t, u * BN, rows, D);
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) {
-            kr[i] = buffer_ld4(rk, k_voff, (uint32_t)((int64_t)(256 * i / C4) * p.sk.t * 4));
-            vr[i] = buffer_ld4(rv, v_voff, (uint32_t)((int64_t)(256 * i / C4) * p.sv.t * 4));
+        for (int i = 0; i < CPT; ++i) {
+            const uint32_t ko = (uint32_t)((int64_t)(256 * i / C8) * p.sk.t * 4);
+            const uint32_t vo = (uint32_t)((int64_t)(256 * i / C8) * p.sv.t * 4);
+            r.k[i][0] = buffer_ld4(rk, k_voff, ko);
+            r.k[i][1] = buffer_ld4(rk, k_voff + 16, ko);
+            r.v[i][0] = buffer_ld4(rv, v_voff, vo);
+            r.v[i][1] = buffer_ld4(rv, v_voff + 16, vo);
         }
     };
-    auto sstore = [&](int buf) {
+    int kcls = 2, vcls = 2;  // classes of the tile in LDS (as in the forward)
+    auto need_classes = [&](const Raw& r, int par) {
+        float mk = 0.f, mv = 0.f;
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) {
-            const int f = tid + 256 * i;
-            const int r = f / C4, c4 = f % C4;
-            *reinterpret_cast<f32x4*>(&Ks[buf][r][4 * c4]) = kr[i];
-            *reinterpret_cast<f32x4*>(&Vs[buf][r][4 * c4]) = vr[i];
+        for (int i = 0; i < CPT; ++i) {
+            mk = absmax8(mk, r.k[i][0], r.k[i][1]);
+            mv = absmax8(mv, r.v[i][0], r.v[i][1]);
+        }
+        int nk = 0, nv = 0;
+        if (__any(mk >= class_limit(kcls) || mv >= class_limit(vcls))) {
+            mk = mv = 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) Kt[buf][4 * c4 + e][r] = kr[i][e];
+            for (int i = 0; i < CPT; ++i) {
+                mk = absmax8_finite(mk, r.k[i][0], r.k[i][1]);
+                mv = absmax8_finite(mv, r.v[i][0], r.v[i][1]);
+            }
+            nk = scale_class(wave_max(mk));
+            nv = scale_class(wave_max(mv));
+        }
+        if (lane == 0) {
+            cls_s[0][par][wave] = nk;
+            cls_s[1][par][wave] = nv;
+        }
+    };
+    auto class_of = [&](int which, int par, int cur) {  // after the barrier
+        int m = cur;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = max(m, cls_s[which][par][i]);
+        return __builtin_amdgcn_readfirstlane(m);
+    };
+    auto sstore = [&](const Raw& r, int buf, int kc, int vc) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const int f = tid + 256 * i, row = f / C8, col = 8 * (f % C8);
+            if (NCH % 256 == 0 || f < NCH) {
+                const Half2x8 k = split2(r.k[i][0], r.k[i][1], class_scale(kc));
+                const Half2x8 v = split2(r.v[i][0], r.v[i][1], class_scale(vc));
+                *reinterpret_cast<f16x8*>(&Ks[buf][0][row][col]) = k.h;
+                *reinterpret_cast<f16x8*>(&Ks[buf][1][row][col]) = k.l;
+                *reinterpret_cast<f16x8*>(&Vs[buf][0][row][col]) = v.h;
+                *reinterpret_cast<f16x8*>(&Vs[buf][1][row][col]) = v.l;
+            }
         }
     };
 
     f32x16 dq[NDB];
 #pragma unroll
     for (int i = 0; i < NDB; ++i) dq[i] = f32x16{};
-    const float c = p.c;
+    int dscls = 2;  // class of the row's largest |ds| so far, per lane
 
-    gload(0);
-    sstore(0);
+    Raw ra, rb;
+    gload(ra, 0);
+    need_classes(ra, 0);
+    gload(rb, 1);
     __syncthreads();
-    for (int u = 0; u < nt; ++u) {
+    kcls = class_of(0, 0, kcls);
+    vcls = class_of(1, 0, vcls);
+    sstore(ra, 0, kcls, vcls);
+    need_classes(rb, 1);
+    __syncthreads();
+    auto step = [&](int u, Raw& nxt, Raw& far) {
         const int buf = u & 1;
         const int k0 = u * BN;
-        gload(u + 1);  // zero rows past the last tile: straight-line
+        gload(far, u + 2);
+        const int nk = class_of(0, (u + 1) & 1, kcls), nv = class_of(1, (u + 1) & 1, vcls);
         if (k0 < wave_kend) {
-            f32x16 s = f32x16{}, dp = f32x16{};
+            f32x16 s, dp;
 #pragma unroll
-            for (int i = 0; i < HD; i += 4) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&Ks[buf][l32][g * HD + i]);
-                const f32x4 v = *reinterpret_cast<const f32x4*>(&Vs[buf][l32][g * HD + i]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    s = mfma32x32x2(a[j], qf[i + j], s);
-                    dp = mfma32x32x2(v[j], df[i + j], dp);
-                }
+            for (int kk = 0; kk < NKK; ++kk) {
+                Half2x8 k, v;
+                k.h = *reinterpret_cast<const f16x8*>(&Ks[buf][0][l32][16 * kk + 8 * g]);
+                k.l = *reinterpret_cast<const f16x8*>(&Ks[buf][1][l32][16 * kk + 8 * g]);
+                v.h = *reinterpret_cast<const f16x8*>(&Vs[buf][0][l32][16 * kk + 8 * g]);
+                v.l = *reinterpret_cast<const f16x8*>(&Vs[buf][1][l32][16 * kk + 8 * g]);
+                s = mfma_split(k, qf[kk], kk == 0 ? f32x16{} : s);
+                dp = mfma_split(v, df[kk], kk == 0 ? f32x16{} : dp);
             }
             // reg r: key k0 + 8 (r / 4) + 4 g + r % 4 of query qrow
             const bool need_mask = (k0 + BN > p.Tk) || (qtile * BM + BM > p.Tq) || (p.causal && (k0 + BN - 1 > q0w + p.off));
             const int lim = p.causal ? min(p.Tk - 1, qrow + p.off) : p.Tk - 1;
+            const float cs = p.c * qinv * class_inv(kcls), vscale = class_scale(vcls);
             // the visibility test only on tiles that cross the diagonal or the ends
+            float mx = 0.f;
             auto p_ds = [&](auto masked) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    float pr = fast_exp2(fmaf(s[r], c, -Lq));
+                    float pr = fast_exp2(fmaf(s[r], cs, -Lq));
                     if constexpr (decltype(masked)::value) {
                         const int key = k0 + 8 * (r >> 2) + 4 * g + (r & 3);
                         pr = (key <= lim && qrow < p.Tq) ? pr : 0.f;
                     }
-                    s[r] = pr * ((dp[r] - Dq) - Dqlo);  // dS^T
+                    s[r] = pr * fmaf(-Dqlo, vscale, fmaf(-Dq, vscale, dp[r]));  // dS^T
                 }
             };
             if (need_mask)
@@ -695,33 +953,58 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
             else
                 p_ds(std::false_type{});
             if (one_key_wave && k0 == 0 && one_key) s = f32x16{};  // one visible key: dS = P (dP - dP) = 0
-            // dQ^T[d][q] += K^T[d][keys] dS^T[keys][q]: MFMA (j, cc) reduces keys 8j + cc, 8j + 4 + cc
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32x4 kt[NDB];
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(s[r]));
+            if (__any(mx >= class_limit(dscls))) {  // a row's dQ is kept in units of its ds scale
+                mx = 0.f;
 #pragma unroll
-                for (int db = 0; db < NDB; ++db)
-                    kt[db] = *reinterpret_cast<const f32x4*>(&Kt[buf][db * 32 + l32][8 * j + 4 * g]);
+                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, finite_abs(s[r]));
+                const int nc = max(dscls, min(31, scale_class(max_xor32(mx))));
+                const float f = class_scale(nc) * class_inv(dscls);
 #pragma unroll
-                for (int cc = 0; cc < 4; ++cc)
+                for (int db = 0; db < NDB; ++db) dq[db] *= f;
+                dscls = nc;
+            }
+            const float sc = class_scale(dscls);
+            // dQ^T[d][q] += K^T[d][keys] dS^T[keys][q]: step m takes keys 16 m + 4 g + {0..3} and + 8
 #pragma unroll
-                    for (int db = 0; db < NDB; ++db) dq[db] = mfma32x32x2(kt[db][cc], s[4 * j + cc], dq[db]);
+            for (int m = 0; m < 2; ++m) {
+                const Half2x8 ds = split2(f32x4{s[8 * m], s[8 * m + 1], s[8 * m + 2], s[8 * m + 3]},
+                                          f32x4{s[8 * m + 4], s[8 * m + 5], s[8 * m + 6], s[8 * m + 7]}, sc);
+                const int r0 = 16 * m + 4 * g + tr_row;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) {
+                    Half2x8 kt;
+                    kt.h = tr_frag([&](int r) { return &Ks[buf][0][r0 + r][db * 32 + tr_col]; });
+                    kt.l = tr_frag([&](int r) { return &Ks[buf][1][r0 + r][db * 32 + tr_col]; });
+                    dq[db] = mfma_split(kt, ds, dq[db]);
+                }
             }
         }
-        sstore(buf ^ 1);
+        if (nk != kcls || nv != vcls) {  // ... and of K's and V's scales
+            const float f = (class_scale(nk) * class_inv(kcls)) * (class_scale(nv) * class_inv(vcls));
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) dq[db] *= f;
+        }
+        kcls = nk;
+        vcls = nv;
+        sstore(nxt, buf ^ 1, nk, nv);
+        need_classes(far, u & 1);
         __syncthreads();
+    };
+    for (int u = 0; u < nt; u += 2) {
+        step(u, rb, ra);
+        if (u + 1 < nt) step(u + 1, ra, rb);
     }
     if (qrow < p.Tq) {
+        const float unit = class_inv(dscls) * kBwdPInv * class_inv(vcls) * doinv * class_inv(kcls) * p.scale;
         float* dst = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)qrow * p.sdq.t;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32x4 val;
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc) val[cc] = dq[db][4 * j + cc] * p.scale;
-                st4(dst + db * 32 + 8 * j + 4 * g, val);
-            }
+            for (int j = 0; j < 4; ++j)
+                st4(dst + db * 32 + 8 * j + 4 * g,
+                    f32x4{dq[db][4 * j], dq[db][4 * j + 1], dq[db][4 * j + 2], dq[db][4 * j + 3]} * unit);
     }
 }
 
@@ -744,8 +1027,8 @@ static constexpr double kBwdPairGain = 0.08;  // throughput gained per extra res
 // same time; the bf16 figures are set from measurement (splits lost 5-8% at
 // B4 H12 and config 2 with smaller ones), so bf16 splits only grids far below
 // the device's size.
-static constexpr double kBwdOverhead[2] = {0.3, 5.0};
-static constexpr double kBwdFixup[2] = {0.4, 8.0};
+static constexpr double kBwdOverhead[2] = {1.0, 5.0};
+static constexpr double kBwdFixup[2] = {1.0, 8.0};
 // The short-row prologue of key block 0 (the S and dP chains of each short
 // query tile, run once more to form delta) per short tile, in the same units.
 static constexpr double kBwdShortTile[2] = {0.55, 0.5};
@@ -810,17 +1093,12 @@ static int bwd_slots(int D, int bf16, int* per_cu, int* cus_per_xcd) {
     const std::array<int, 3> key{dev, D, bf16};
     auto it = cache.find(key);
     if (it == cache.end()) {
-        int cus = 256, occ = (D >= 128 || bwd_waves(bf16, D) == 8) ? 1 : 2;  // MI355X defaults
+        int cus = 256, occ = (!bf16 || D >= 64) ? 1 : 2;  // MI355X defaults
         if (dev >= 0) {
             int n = 0, o = 0;
             if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
             hipError_t e = hipErrorInvalidValue;
-            if (!bf16 && D == 32)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, bwd_main_kernel<32, float, false>, 64 * bwd_waves(0, 32), 0);
-            if (!bf16 && D == 64)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, bwd_main_kernel<64, float, false>, 64 * bwd_waves(0, 64), 0);
-            if (!bf16 && D == 128)
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, bwd_main_kernel<128, float, false>, 64 * bwd_waves(0, 128), 0);
+            if (!bf16) o = 1, e = hipSuccess;  // fp32: 512 threads of 208-256 VGPRs, one workgroup per CU
             if (bf16) e = (hipError_t)bwd_main_bf16_occupancy(D, &o);
             if (e == hipSuccess && o > 0) occ = o;
             (void)hipGetLastError();  // a failed query of ours: the defaults stand
@@ -835,7 +1113,7 @@ static int bwd_slots(int D, int bf16, int* per_cu, int* cus_per_xcd) {
 static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int per_cu, int cus_per_xcd,
                              BwdPlan* out) {
     const int BH = B * H;
-    const int bk = bwd_keys_per_wg(bf16, D);
+    const int bk = bwd_keys_per_wg(bf16, D, BH, Tq, Tk);
     const int nkb = (Tk + bk - 1) / bk;
     const int off = Tk - Tq;
     if ((int64_t)nkb * BH > 8LL * 8 * cus_per_xcd * per_cu) return;  // the tail is a small share
@@ -847,7 +1125,7 @@ static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int 
         max_nt = std::max(max_nt, nt[(size_t)j]);
     }
     // query tiles [0, s_tiles) of key block 0 hold its short rows and run the prologue
-    const int s_tiles = (bwd_short_rows(B, H, Tq, Tk, 1, bk) + kBwdBQ - 1) / kBwdBQ;
+    const int s_tiles = (bwd_short_rows(B, H, Tq, Tk, 1, bwd_short_keys(bf16, bk)) + kBwdBQ - 1) / kBwdBQ;
     struct G { double cost; int kb, a, b, chunk, n; };
     // A key block of more than ch tiles is split into ceil(n / ch) chunks of
     // near-equal cost, block 0's short tiles counted with the prologue's share
@@ -930,7 +1208,7 @@ static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int 
 
 int bwd_plan(int B, int H, int Tq, int Tk, int D, int causal, int bf16, BwdPlan* out) {
     *out = BwdPlan{};
-    out->bk = bwd_keys_per_wg(bf16, D);
+    out->bk = bwd_keys_per_wg(bf16, D, (int64_t)B * H, Tq, Tk);
     if (!causal) return 0;
     int per_cu = 0, cus_per_xcd = 0;
     if (const int e = bwd_slots(D, bf16, &per_cu, &cus_per_xcd)) return e;
@@ -959,6 +1237,16 @@ size_t bwd_split_workspace_bytes(const BwdPlan& plan, int B, int H, int D) {
     return part + (size_t)plan.n_split * bh * sizeof(unsigned);
 }
 
+template <int D, int KP>
+static void launch_bwd_main_f32(const BwdParams& p, dim3 grid, hipStream_t s) {
+    if (p.dq_direct)
+        hipLaunchKernelGGL((bwd_main_kernel<D, KP, true, true>), grid, dim3(512), 0, s, p);
+    else if (p.n_short > 0)
+        hipLaunchKernelGGL((bwd_main_kernel<D, KP, true, false>), grid, dim3(512), 0, s, p);
+    else
+        hipLaunchKernelGGL((bwd_main_kernel<D, KP, false, false>), grid, dim3(512), 0, s, p);
+}
+
 template <int D, typename E>
 static int launch_bwd_t(const BwdParams& p_in, hipStream_t s) {
     BwdParams p = p_in;
@@ -970,7 +1258,7 @@ static int launch_bwd_t(const BwdParams& p_in, hipStream_t s) {
     const int64_t rows = (int64_t)p.B * p.H * p.Tq;
     const dim3 pre_grid((unsigned)((rows + RPB - 1) / RPB));  // bwd_cvt: 4 elements per thread
     constexpr int PRE_RPB = bwd_pre_rows_per_block<D, E>();
-    const dim3 delta_grid((unsigned)((rows + PRE_RPB - 1) / PRE_RPB));
+    const dim3 delta_grid((unsigned)(sizeof(E) == 4 ? (int64_t)p.B * p.H * p.n_amax : (rows + PRE_RPB - 1) / PRE_RPB));
     if (!p.pre_delta && !p.dq_direct) {
         // zeroing only: a few grid-stride workgroups per CU
         const int64_t n4 = rows * D / 4;
@@ -995,10 +1283,10 @@ static int launch_bwd_t(const BwdParams& p_in, hipStream_t s) {
         }
     } else {
         const dim3 grid((unsigned)(p.n_groups ? p.n_groups * bwd_padded_heads(p.B * p.H) : p.n_kblocks * p.B * p.H));
-        if (p.n_short > 0)
-            hipLaunchKernelGGL((bwd_main_kernel<D, E, true>), grid, dim3(64 * bwd_waves(0, D)), 0, s, p);
+        if (p.keys_per_wg == 128)
+            launch_bwd_main_f32<D, 32>(p, grid, s);
         else
-            hipLaunchKernelGGL((bwd_main_kernel<D, E, false>), grid, dim3(64 * bwd_waves(0, D)), 0, s, p);
+            launch_bwd_main_f32<D, D >= 128 ? 32 : 64>(p, grid, s);
         if (p.dq_direct)
             hipLaunchKernelGGL((bwd_dq_kernel<D>), dim3((unsigned)(p.n_qtiles * p.B * p.H)), dim3(256), 0, s, p);
     }

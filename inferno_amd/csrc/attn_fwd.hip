@@ -1,28 +1,37 @@
-// attn_fwd.hip -- fused causal attention forward for gfx950.
+// attn_fwd.hip -- fused causal attention forward for gfx950, fp32.
 //
-// One workgroup = 4 waves = 128 query rows of one (b, h); each wave owns 32
-// rows for the whole kernel.  K and V tiles of BN keys are streamed through
-// LDS (double-buffered, one barrier per tile, the next tile's global loads in
-// flight in registers while the current one is consumed).  Per wave and tile:
+// One workgroup = 8 waves = 256 query rows of one (b, h); each wave owns 32
+// rows for the whole kernel.  Both products run on the fp16 matrix cores, every
+// operand split into two fp16 parts (common.h), three MFMAs per product step.
+// K and V tiles of BN keys are loaded two tiles ahead into registers, split
+// once for all eight waves into double-buffered LDS, one barrier per tile.  Per
+// wave and tile:
 //
-//   S^T (keys x queries) = K Q^T      v_mfma_f32_32x32x2_f32, A = K from LDS,
-//                                     B = Q^T resident in VGPRs
+//   S^T (keys x queries) = K Q^T      v_mfma_f32_32x32x16_f16, A = K from LDS,
+//                                     B = Q^T resident in VGPRs, split
 //   online softmax on S^T             query = lane%32, so the row max needs one
 //                                     xor-32 exchange; the row sum stays
-//                                     per-lane until the end
-//   O^T (d x queries) += V^T P^T      A = V^T from LDS, B = P^T straight from
+//                                     per-lane until the end; fp32
+//   O^T (d x queries) += V^T P^T      A = V^T from LDS, B = P^T split from
 //                                     the S^T accumulators (reduction index
 //                                     permuted to match their layout)
 //
-// V is stored transposed in LDS (Vt[d][key]) so that the four keys a lane
-// feeds to four consecutive MFMAs are adjacent: one ds_read_b128 per four
-// MFMAs in both products, issued well ahead of use, instead of a dependent
-// ds_read_b32 per MFMA.  V tiles are fetched with a row-fastest lane mapping
-// (16 keys x 4 column chunks per wave) so the transposing LDS stores hit 64
-// distinct banks.
+// V lies transposed in LDS in the operand's order, one 16-byte read per operand
+// part: a thread loads one column of the 8 keys that an operand takes together,
+// so the transposition costs no store.
+//
+// At D = 128 the kernel keeps the matrix cores 49% busy at a 1.97 GHz shader
+// clock (the rest is softmax and split VALU work, 39% of the issue slots, that
+// overlaps only in part); at D = 64 a workgroup's serial chain of tiles, about
+// 6500 cycles each for 3072 of MFMA, sets causal grids of a round or two.
+// Against the fp32-MFMA kernel it replaced (us): config 2 128.8 -> 58.4, config 4
+// 2281 -> 726, B8 H12 T1024 D32 73 -> 38, B1 H12 T1024 D64 37 -> 26.  With three
+// bf16 parts and six MFMAs instead: 78.6 and 1229.  128-row workgroups of four
+// waves (each tile split twice as often) lost at every D = 128 shape and config
+// 4 (726 -> 988), gaining only on large D = 64 grids (B16 H12 117 -> 110).
 //
 // Keeping queries on the lane axis in both products is what lets P stay in
-// registers.  The scale is folded into exp2: p = exp2(s*c - m*c) with
+// registers.  The scale is folded into exp2: p = exp2(s*c - m) with
 // c = scale*log2(e).  Masked scores (key > query + Tk - Tq, or key >= Tk)
 // become -inf, so their probabilities are exactly 0, as the reference's
 // -1e9f fill followed by exp((double)(-1e9 - max)) is.  The row
@@ -43,6 +52,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -52,46 +62,37 @@ namespace inf {
 
 template <int D>
 struct FwdTile {
-    static constexpr int BN = (D >= 128) ? 32 : 64;  // keys per LDS tile
-    static constexpr int KS = D + 4;                 // K row stride in LDS (floats)
-    static constexpr int VTS = BN + 4;               // V^T row stride in LDS (floats)
-    // Software-pipelined loop (two score blocks live): fits two waves per
-    // SIMD up to D = 64; D = 128 keeps one score block.
-    static constexpr bool PIPE = D <= 64;
-    // V chunk f of a tile: row and first column (elements) within the tile.
-    static constexpr int vrow(int f) { return (f & 15) + 16 * (f / (16 * (D / 4))); }
-    static constexpr int vcol(int f) { return 4 * ((f >> 4) % (D / 4)); }
-    // Chunk tid + 256 i sits at (row, column) of chunk tid plus that of chunk
-    // 256 i, for K and V, for every thread and load of a tile.
-    static constexpr bool chunks_split() {
-        constexpr int C4 = D / 4, LPT = BN * C4 / 256;
-        for (int i = 0; i < LPT; ++i)
-            for (int tid = 0; tid < 256; ++tid) {
-                const int f = tid + 256 * i;
-                if (f / C4 != tid / C4 + 256 * i / C4 || f % C4 != tid % C4) return false;
-                if (vrow(f) != vrow(tid) + vrow(256 * i) || vcol(f) != vcol(tid) + vcol(256 * i)) return false;
-            }
-        return true;
-    }
+    static constexpr int NW = 8;  // waves per workgroup, 32 query rows each
+    static constexpr int BM = 32 * NW;
+    static constexpr int BN = D == 32 ? 128 : D == 64 ? 64 : 32;  // keys per LDS tile: one 8-element unit per thread
+    static constexpr int KS = D + 8;                              // K row stride in LDS (fp16 elements)
 };
 
 // Headroom of the forward's lazy rescaling, in exp2 units: P <= 2^8.
 constexpr float kLazyLog2 = 8.f;
+// P enters its products as 2^kPBits P, at most 2^14: the low part of a
+// probability of 2^-9 or more is then a normal fp16 number, and a smaller one
+// carries an absolute error of 2^-31 of the row's reference.
+constexpr float kPBits = 6.f, kPInv = 1.f / 64.f;
 
-template <int D, typename E>
-__global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
-    constexpr int BM = kFwdBM;
+template <int D>
+__global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdParams p) {
+    constexpr int NT = 64 * FwdTile<D>::NW;
+    constexpr int BM = FwdTile<D>::BM;
     constexpr int BN = FwdTile<D>::BN;
     constexpr int KS = FwdTile<D>::KS;
-    constexpr int VTS = FwdTile<D>::VTS;
-    constexpr int HD = D / 2;        // reduction elements per lane half
-    constexpr int NKB = BN / 32;     // 32-key blocks per tile
-    constexpr int NDB = D / 32;      // 32-wide head-dim blocks
-    constexpr int C4 = D / 4;        // 4-element chunks per row
-    constexpr int LPT = BN * C4 / 256;  // 4-element loads per thread per tensor per tile
+    constexpr int NKK = D / 16;          // MFMA steps along the head dim for S^T
+    constexpr int NKB = BN / 32;         // 32-key blocks per tile
+    constexpr int NDB = D / 32;          // 32-wide head-dim blocks of O^T
+    constexpr int C8 = D / 8;            // 8-element chunks per K row
+    constexpr int UPT = BN * C8 / NT;    // 8-element units per thread per tensor per tile
+    static_assert(BN * C8 % NT == 0 && NT % D == 0 && NT % C8 == 0, "whole staging passes");
 
-    __shared__ __attribute__((aligned(16))) float Ks[2][BN][KS];
-    __shared__ __attribute__((aligned(16))) float Vt[2][D][VTS];
+    __shared__ __attribute__((aligned(16))) _Float16 Ks0[2][BN][KS];
+    __shared__ __attribute__((aligned(16))) _Float16 Ks1[2][BN][KS];
+    __shared__ f16x8 Vt0[2][BN / 8][D];
+    __shared__ f16x8 Vt1[2][BN / 8][D];
+    __shared__ __attribute__((aligned(16))) int cls_s[2][2][8];  // scale class that each wave's loads need: [K, V][tile parity]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -115,29 +116,34 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
     const int b = bh / p.H;
     const int h = bh % p.H;
 
-    const E* Q = (const E*)p.q + b * p.sq.b + h * p.sq.h;
-    const E* K = (const E*)p.k + b * p.sk.b + h * p.sk.h;
-    const E* V = (const E*)p.v + b * p.sv.b + h * p.sv.h;
-    E* O = (E*)p.o + b * p.so.b + h * p.so.h;
+    const float* Q = (const float*)p.q + b * p.sq.b + h * p.sq.h;
+    const float* K = (const float*)p.k + b * p.sk.b + h * p.sk.h;
+    const float* V = (const float*)p.v + b * p.sv.b + h * p.sv.h;
+    float* O = (float*)p.o + b * p.so.b + h * p.so.h;
 
     const int q0w = qtile * BM + wave * 32;  // first query row of this wave
     const int qrow = q0w + l32;              // this lane's query row
 
-    // Q^T operand: lane (l32, g) holds Q[qrow][g*HD + i], i = 0..HD-1.
-    float qf[HD];
-    if (qrow < p.Tq) {
-        const E* src = Q + (int64_t)qrow * p.sq.t + g * HD;
+    // Q^T operand: MFMA step kk takes Q[qrow][16 kk + 8 g .. + 7], scaled by the
+    // row's own class.
+    Half2x8 qf[NKK];
+    float cq;  // scale * log2(e) over the row's scale
+    {
+        f32x4 qa[NKK][2];
+        float amax = 0.f;
 #pragma unroll
-        for (int i = 0; i < HD; i += 4) {
-            f32x4 t = ld4(src + i);
-            qf[i] = t[0];
-            qf[i + 1] = t[1];
-            qf[i + 2] = t[2];
-            qf[i + 3] = t[3];
+        for (int kk = 0; kk < NKK; ++kk) {
+            qa[kk][0] = qa[kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (qrow < p.Tq) {
+                qa[kk][0] = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g);
+                qa[kk][1] = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g + 4);
+            }
+            amax = absmax8_finite(amax, qa[kk][0], qa[kk][1]);
         }
-    } else {
+        const int k = scale_class(max_xor32(amax));
+        cq = p.c * class_inv(k);
 #pragma unroll
-        for (int i = 0; i < HD; ++i) qf[i] = 0.f;
+        for (int kk = 0; kk < NKK; ++kk) qf[kk] = split2(qa[kk][0], qa[kk][1], class_scale(k));
     }
 
     // Keys this workgroup needs, and this wave's visible limit (exclusive).
@@ -146,198 +152,251 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
     const int n_tiles = min((kv_end + BN - 1) / BN, t_end);
     const int wave_kend = p.causal ? min(kv_end, q0w + 32 + p.off) : kv_end;
 
-    // K: chunk f -> (row f / C4, column chunk f % C4), row-major 16-byte loads.
-    // V: chunk f -> (row f % 16 + 16 * (f / (16 * C4)), column chunk (f / 16) % C4).
-    // Loads go through a buffer resource per tile: each chunk's offset is a
-    // per-thread part (chunk tid) plus a uniform part (chunk 256 i), and rows
-    // at or past `lim` (<= Tk) are outside the resource and read as zeros, so
-    // a load costs no address arithmetic, compare or branch.
-    static_assert(FwdTile<D>::chunks_split(), "chunk offsets must split into thread + load parts");
-    static_assert(sizeof(E) == 4, "fp32 storage (bf16 has its own kernel)");
-    f32x4 kr[LPT], vr[LPT];
-    const uint32_t k_voff = (uint32_t)(((int64_t)(tid / C4) * p.sk.t + 4 * (tid % C4)) * 4);
-    const uint32_t v_voff = (uint32_t)(((int64_t)FwdTile<D>::vrow(tid) * p.sv.t + FwdTile<D>::vcol(tid)) * 4);
-    auto gload_k = [&](int t, int lim) {
-        const auto rs = row_rsrc((const float*)K, p.sk.t, t * BN, min(lim - t * BN, BN), D);
-#pragma unroll
-        for (int i = 0; i < LPT; ++i)
-            kr[i] = buffer_ld4(rs, k_voff, (uint32_t)(((int64_t)(256 * i / C4) * p.sk.t) * 4));
+    // K unit tid + NT i: row f / C8, 8 columns from 8 (f % C8): two 16-byte
+    // loads.  V unit: column f % D of the 8 keys that the P V operand takes
+    // together (keys 16 m + 4 g' + {0..3} and + 8 for key group f / D = 2 m + g'):
+    // eight 4-byte loads, each a run of a row over the wave's lanes, so V lands
+    // transposed without a transposing store.  Loads go through a buffer
+    // resource per tile: rows at or past `lim` read as zeros.
+    struct Raw {
+        f32x4 k[UPT][2];
+        float v[UPT][8];
     };
-    auto gload_v = [&](int t, int lim) {
-        const auto rs = row_rsrc((const float*)V, p.sv.t, t * BN, min(lim - t * BN, BN), D);
+    const uint32_t k_voff = (uint32_t)(((int64_t)(tid / C8) * p.sk.t + 8 * (tid % C8)) * 4);
+    auto vrow0 = [](int kg) { return 16 * (kg >> 1) + 4 * (kg & 1); };
+    const uint32_t vd = (uint32_t)(tid % D) * 4;
+    auto gload = [&](Raw& r, int t) {
+        const int rows = t < n_tiles ? min(p.Tk - t * BN, BN) : 0;
+        const auto rk = row_rsrc(K, p.sk.t, t * BN, rows, D);
+        const auto rv = row_rsrc(V, p.sv.t, t * BN, rows, D);
 #pragma unroll
-        for (int i = 0; i < LPT; ++i)
-            vr[i] = buffer_ld4(rs, v_voff,
-                               (uint32_t)(((int64_t)FwdTile<D>::vrow(256 * i) * p.sv.t + FwdTile<D>::vcol(256 * i)) * 4));
-    };
-    auto gload = [&](int t) {
-        gload_k(t, p.Tk);
-        gload_v(t, p.Tk);
-    };
-    auto sstore_k = [&](int buf) {
+        for (int i = 0; i < UPT; ++i) {
+            const uint32_t so = (uint32_t)((int64_t)(NT * i / C8) * p.sk.t * 4);
+            r.k[i][0] = buffer_ld4(rk, k_voff, so);
+            r.k[i][1] = buffer_ld4(rk, k_voff + 16, so);
+            const int r0 = __builtin_amdgcn_readfirstlane(vrow0((tid + NT * i) / D));  // D >= 64: wave-uniform
+            const uint32_t v_voff = D >= 64 ? vd : (uint32_t)((int64_t)vrow0((tid + NT * i) / D) * p.sv.t * 4) + vd;
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) {
-            const int f = tid + 256 * i;
-            *reinterpret_cast<f32x4*>(&Ks[buf][f / C4][4 * (f % C4)]) = kr[i];
+            for (int e = 0; e < 8; ++e)
+                r.v[i][e] = buffer_ld1(rv, v_voff,
+                                       (uint32_t)((int64_t)((D >= 64 ? r0 : 0) + (e & 3) + 8 * (e >> 2)) * p.sv.t * 4));
         }
     };
-    auto sstore_v = [&](int buf) {
+    // K and V tiles are scaled by the class of the largest magnitude so far in
+    // the workgroup's range (kk_cls, kv_cls: the classes of the split tile in
+    // LDS).  A wave whose loads of a tile exceed the classes that it knows says so
+    // in LDS one barrier ahead of the split; ordinary tensors do it once.
+    int kk_cls = 2, kv_cls = 2;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    auto v4 = [](const float (&v)[8], int j) { return f32x4{v[j], v[j + 1], v[j + 2], v[j + 3]}; };
+    auto need_classes = [&](const Raw& r, int par) {
+        float mk = 0.f, mv = 0.f;
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) {
-            const int f = tid + 256 * i;
-            const int vrow = (f & 15) + 16 * (f / (16 * C4));
-            const int vc = 4 * ((f >> 4) % C4);
-            Vt[buf][vc + 0][vrow] = vr[i][0];
-            Vt[buf][vc + 1][vrow] = vr[i][1];
-            Vt[buf][vc + 2][vrow] = vr[i][2];
-            Vt[buf][vc + 3][vrow] = vr[i][3];
+        for (int i = 0; i < UPT; ++i) {
+            mk = absmax8(mk, r.k[i][0], r.k[i][1]);
+            mv = absmax8(mv, v4(r.v[i], 0), v4(r.v[i], 4));
+        }
+        int nk = 0, nv = 0;
+        if (__any(mk >= class_limit(kk_cls) || mv >= class_limit(kv_cls))) {
+            mk = mv = 0.f;
+#pragma unroll
+            for (int i = 0; i < UPT; ++i) {
+                mk = absmax8_finite(mk, r.k[i][0], r.k[i][1]);
+                mv = absmax8_finite(mv, v4(r.v[i], 0), v4(r.v[i], 4));
+            }
+            nk = scale_class(wave_max(mk));
+            nv = scale_class(wave_max(mv));
+        }
+        if (lane == 0) {
+            cls_s[0][par][wave_u] = nk;
+            cls_s[1][par][wave_u] = nv;
         }
     };
-    auto sstore = [&](int buf) {
-        sstore_k(buf);
-        sstore_v(buf);
+    auto class_of = [&](int which, int par, int cur) {  // after the barrier
+        int m = cur;
+#pragma unroll
+        for (int w = 0; w < FwdTile<D>::NW; ++w) m = max(m, cls_s[which][par][w]);
+        return __builtin_amdgcn_readfirstlane(m);
+    };
+    auto sstore = [&](const Raw& r, _Float16 (&Kd)[2][BN][KS], f16x8 (&Vd)[2][BN / 8][D], int kc, int vc) {
+        const float ks = class_scale(kc), vs = class_scale(vc);
+#pragma unroll
+        for (int i = 0; i < UPT; ++i) {
+            const int f = tid + NT * i;
+            const Half2x8 k = split2(r.k[i][0], r.k[i][1], ks);
+            const Half2x8 v = split2(v4(r.v[i], 0), v4(r.v[i], 4), vs);
+            *reinterpret_cast<f16x8*>(&Kd[0][f / C8][8 * (f % C8)]) = k.h;
+            *reinterpret_cast<f16x8*>(&Kd[1][f / C8][8 * (f % C8)]) = k.l;
+            Vd[0][f / D][f % D] = v.h;
+            Vd[1][f / D][f % D] = v.l;
+        }
     };
 
     f32x16 o[NDB];
 #pragma unroll
     for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
-    float m_run = -INFINITY;  // running max of raw scores for row qrow
-    float l_run = 0.f;        // this lane's partial sum of p (its half of the keys)
-    const float c = p.c;
+    float m_run = -INFINITY;  // reference max of row qrow's scores, in exp2 units
+    float l_run = 0.f;        // this lane's partial sum of 2^kPBits p (its half of the keys)
 
-    // S^T block of key tile in Ks[buf]: s[kb] reg 4j+cc holds key kb*32 + 8j + 4g + cc.
-    auto scores = [&](int buf, f32x16 (&s)[NKB]) {
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) s[kb] = f32x16{};
-#pragma unroll
-        for (int i = 0; i < HD; i += 4) {
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&Ks[buf][kb * 32 + l32][g * HD + i]);
-                s[kb] = mfma32x32x2(a[0], qf[i + 0], s[kb]);
-                s[kb] = mfma32x32x2(a[1], qf[i + 1], s[kb]);
-                s[kb] = mfma32x32x2(a[2], qf[i + 2], s[kb]);
-                s[kb] = mfma32x32x2(a[3], qf[i + 3], s[kb]);
-            }
-        }
-    };
+    Raw ra, rb;
+    gload(ra, t_begin);
+    need_classes(ra, t_begin & 1);
+    gload(rb, t_begin + 1);
+    __syncthreads();
+    kk_cls = class_of(0, t_begin & 1, kk_cls);
+    kv_cls = class_of(1, t_begin & 1, kv_cls);
+    sstore(ra, Ks0, Vt0, kk_cls, kv_cls);
+    need_classes(rb, (t_begin + 1) & 1);
+    __syncthreads();
 
-    // Mask, online softmax and O^T += V^T P^T for key tile t (V^T in Vt[vbuf]).
-    auto softmax_pv = [&](f32x16 (&s)[NKB], int t, int vbuf) {
+    // Step t reads tile t from buffer BUF = (t - t_begin) % 2 while tile t + 2
+    // loads into registers; tile t + 1, loaded in the previous step, is split
+    // into the other buffer, which every wave finished reading before the
+    // previous step's barrier.
+    auto step = [&](int t, auto buf_c, Raw& nxt, Raw& far) {
+        constexpr int BUF = decltype(buf_c)::value;
+        _Float16(&Kc)[2][BN][KS] = BUF ? Ks1 : Ks0;
+        f16x8(&Vc)[2][BN / 8][D] = BUF ? Vt1 : Vt0;
         const int k0 = t * BN;
-        const bool need_mask = (k0 + BN > p.Tk) || (p.causal && (k0 + BN - 1 > q0w + p.off));
-        if (need_mask) {
-            const int lim = p.causal ? min(p.Tk - 1, qrow + p.off) : p.Tk - 1;
+        gload(far, t + 2);
+        const int nk = class_of(0, (t + 1) & 1, kk_cls), nv = class_of(1, (t + 1) & 1, kv_cls);
+        if (k0 < wave_kend) {
+            f32x16 s[NKB];
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk)
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) {
+                    Half2x8 a;
+                    a.h = *reinterpret_cast<const f16x8*>(&Kc[0][kb * 32 + l32][16 * kk + 8 * g]);
+                    a.l = *reinterpret_cast<const f16x8*>(&Kc[1][kb * 32 + l32][16 * kk + 8 * g]);
+                    s[kb] = mfma_split(a, qf[kk], kk == 0 ? f32x16{} : s[kb]);
+                }
+            // scores in exp2 units are s * cs (at least the smallest normal
+            // number, so a masked score times it stays -inf)
+            const float cs = fmaxf(cq * class_inv(kk_cls), 1.17549435e-38f);
+            // reg 4j+cc of s[kb] holds key kb*32 + 8j + 4g + cc
+            const bool need_mask = (k0 + BN > p.Tk) || (p.causal && (k0 + BN - 1 > q0w + p.off));
+            if (need_mask) {
+                const int lim = p.causal ? min(p.Tk - 1, qrow + p.off) : p.Tk - 1;
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key = k0 + kb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+                        if (key > lim) s[kb][r] = -INFINITY;
+                    }
+            }
+            float mp[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mp[r & 3] = fmaxf(mp[r & 3], s[kb][r]);
+            const float mloc = max_xor32(fmaxf(fmaxf(mp[0], mp[1]), fmaxf(mp[2], mp[3]))) * cs;
+            // Lazy rescaling: a row's reference max m_run moves only when the row
+            // sees a score more than kLazyLog2 above it, so P stays
+            // <= 2^kLazyLog2; the O / l rescale and its exp2 run only on tiles where
+            // some row of the wave moved, and for the other rows it multiplies by
+            // exactly 1, so every row depends on its own scores only.  O / l and the
+            // LSE do not depend on the reference.  m_run = -inf with a visible key
+            // always moves it.
+            const bool grow = mloc > m_run + kLazyLog2;
+            if (__any(grow)) {
+                // A row can see no key of a chunk that does not start at key 0:
+                // keep m = -inf, l = 0, O = 0 for it instead of exp2(NaN).
+                const float alpha = grow ? fast_exp2(m_run - mloc) : 1.f;  // m_run = -inf -> 0
+                l_run *= alpha;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+                m_run = grow ? mloc : m_run;
+            }
+            const float mc = m_run == -INFINITY ? 0.f : kPBits - m_run;
+            // row sum as four independent partial chains
+            float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int key = k0 + kb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (key > lim) s[kb][r] = -INFINITY;
+                    const float e = fast_exp2(fmaf(s[kb][r], cs, mc));
+                    s[kb][r] = e;
+                    ls[r & 3] += e;
+                }
+            l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm) {
+                    const f32x16& e = s[kb];
+                    const Half2x8 pb =
+                        split2(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
+                               f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]}, 1.f);
+#pragma unroll
+                    for (int db = 0; db < NDB; ++db) {
+                        Half2x8 a;
+                        a.h = Vc[0][4 * kb + 2 * mm + g][db * 32 + l32];
+                        a.l = Vc[1][4 * kb + 2 * mm + g][db * 32 + l32];
+                        o[db] = mfma_split(a, pb, o[db]);
+                    }
                 }
         }
-        float mloc = -INFINITY;
+        if (nv != kv_cls) {  // O is kept in units of V's scale
+            const float f = class_scale(nv) * class_inv(kv_cls);
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[kb][r]);
-        mloc = fmaxf(mloc, shfl_xor(mloc, 32));
-        // Lazy rescaling: a row's reference max m_run moves only when the row
-        // sees a score more than kLazyLog2 / c above it, so P stays
-        // <= 2^kLazyLog2; the O / l rescale and its exp2 run only on tiles where
-        // some row of the wave moved (VALU issue adds to fp32 MFMA time one for
-        // one), and for the other rows it multiplies by exactly 1, so every row
-        // depends on its own scores only.  O / l and the LSE do not depend on
-        // the reference.  m_run = -inf with a visible key always moves it.
-        const bool grow = mloc > m_run + kLazyLog2 / c;
-        if (__any(grow)) {
-            // A row can see no key of a chunk that does not start at key 0:
-            // keep m = -inf, l = 0, O = 0 for it instead of exp2(NaN).
-            const float alpha = grow ? fast_exp2((m_run - mloc) * c) : 1.f;  // m_run = -inf -> 0
-            l_run *= alpha;
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) o[db] *= alpha;
-            m_run = grow ? mloc : m_run;
+            for (int db = 0; db < NDB; ++db) o[db] *= f;
         }
-        const float mc = m_run == -INFINITY ? 0.f : m_run * c;
-        // row sum as four independent partial chains
-        float ls[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float e = fast_exp2(fmaf(s[kb][r], c, -mc));
-                s[kb][r] = e;
-                ls[r & 3] += e;
-            }
-        l_run += (ls[0] + ls[1]) + (ls[2] + ls[3]);
-
-        // reg 4j+cc of s[kb] holds key kb*32 + 8j + 4g + cc
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32x4 va[NDB];
-#pragma unroll
-                for (int db = 0; db < NDB; ++db)
-                    va[db] = *reinterpret_cast<const f32x4*>(&Vt[vbuf][db * 32 + l32][kb * 32 + 8 * j + 4 * g]);
-#pragma unroll
-                for (int cc = 0; cc < 4; ++cc)
-#pragma unroll
-                    for (int db = 0; db < NDB; ++db)
-                        o[db] = mfma32x32x2(va[db][cc], s[kb][4 * j + cc], o[db]);
-            }
+        kk_cls = nk;
+        kv_cls = nv;
+        if constexpr (BUF)
+            sstore(nxt, Ks0, Vt0, nk, nv);
+        else
+            sstore(nxt, Ks1, Vt1, nk, nv);
+        need_classes(far, t & 1);
+        __syncthreads();
     };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    for (int t = t_begin; t < n_tiles; t += 2) {
+        step(t, B0{}, rb, ra);
+        if (t + 1 < n_tiles) step(t + 1, B1{}, ra, rb);
+    }
+    float o_unit = class_inv(kv_cls);  // the accumulators' unit over 2^kPBits
 
-    if constexpr (FwdTile<D>::PIPE) {
-        // Software pipeline: S of tile t+1 is issued before the softmax of tile
-        // t, so the matrix pipe has independent work while the softmax runs.
-        // K runs one tile ahead of V: at the top of step t, Ks[i&1] and
-        // Ks[(i+1)&1] hold K_t (already consumed) and K_{t+1}, Vt[i&1] holds
-        // V_t (i = t - t_begin).  Step t writes K_{t+2} over K_t and V_{t+1}
-        // over V_{t-1}, both last read before the previous barrier.
-        gload(t_begin);  // bounds-checked rows: safe even past the last tile
-        sstore_k(0);
-        sstore_v(0);
-        gload_k(t_begin + 1, t_begin + 1 < n_tiles ? p.Tk : 0);
-        sstore_k(1);
-        __syncthreads();
-        f32x16 sa[NKB], sb[NKB];
-        if (t_begin * BN < wave_kend) scores(0, sa);
-        __syncthreads();  // Ks[0] is overwritten at the end of the first step
-
-        // The prefetch and the stores run unconditionally (straight-line code
-        // keeps the loads overlapped); past the last tile they move zeros
-        // into buffers that are not read again.
-        auto step = [&](int t, f32x16 (&cur)[NKB], f32x16 (&nxt)[NKB]) {
-            const int i = t - t_begin;
-            const bool has_next = t + 1 < n_tiles;
-            gload_k(t + 2, t + 2 < n_tiles ? p.Tk : 0);
-            gload_v(t + 1, has_next ? p.Tk : 0);
-            if (has_next && (t + 1) * BN < wave_kend) scores((i + 1) & 1, nxt);
-            if (t * BN < wave_kend) softmax_pv(cur, t, i & 1);
-            sstore_k(i & 1);
-            sstore_v((i + 1) & 1);
-            __syncthreads();
-        };
-        for (int t = t_begin; t < n_tiles; t += 2) {
-            step(t, sa, sb);
-            if (t + 1 < n_tiles) step(t + 1, sb, sa);
-        }
-    } else {
-        gload(t_begin);  // bounds-checked rows: safe even past the last tile
-        sstore(0);
-        __syncthreads();
-        for (int t = t_begin; t < n_tiles; ++t) {
-            const int buf = (t - t_begin) & 1;
-            if (t + 1 < n_tiles) gload(t + 1);
-            if (t * BN < wave_kend) {
-                f32x16 s[NKB];
-                scores(buf, s);
-                softmax_pv(s, t, buf);
-            }
-            if (t + 1 < n_tiles) sstore(buf ^ 1);
-            __syncthreads();
+    // ---- non-finite inputs ------------------------------------------------------
+    // An infinity in q, k or v (or a value past the largest bf16) is NaN in its
+    // split parts, where the fp32 formula may still be finite or infinite (a
+    // score of -inf is a probability of 0).  A wave whose sums are not finite
+    // recomputes its rows from memory in plain fp32, one key at a time.
+    float chk = l_run * 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) chk = fmaf(o[db][r], 0.f, chk);
+    if (__any(chk != 0.f)) {
+        m_run = -INFINITY;
+        l_run = 0.f;
+        o_unit = 1.f;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+        const int j_end = qrow < p.Tq ? min(n_tiles * BN, p.causal ? min(p.Tk, qrow + p.off + 1) : p.Tk) : 0;
+#pragma unroll 1
+        for (int j = t_begin * BN; j < j_end; ++j) {
+            const float* qp = Q + (int64_t)qrow * p.sq.t;
+            const float* kp = K + (int64_t)j * p.sk.t;
+            float s = 0.f;
+#pragma unroll 1
+            for (int d = 0; d < D; ++d) s = fmaf(qp[d], kp[d], s);
+            s *= p.c;
+            const float mn = fmaxf(m_run, s);
+            const float mc = mn == -INFINITY ? 0.f : mn;
+            const float alpha = m_run == -INFINITY ? 0.f : fast_exp2(m_run - mc);
+            const float e = fast_exp2(s - mc + kPBits);
+            m_run = mn;
+            l_run = fmaf(l_run, alpha, g == 0 ? e : 0.f);
+            const float* vp = V + (int64_t)j * p.sv.t + 4 * g;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    o[db][r] = fmaf(e, vp[db * 32 + 8 * (r >> 2) + (r & 3)], o[db][r] * alpha);
         }
     }
 
@@ -353,7 +412,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     st4(po + db * 32 + 8 * j + 4 * g,
-                        f32x4{o[db][4 * j + 0], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]});
+                        f32x4{o[db][4 * j + 0], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]} * o_unit);
             if (g == 0) {
                 float* pml = p.part + (int64_t)p.n_slots * BH * BM * D + (((int64_t)slot * BH + bh) * BM + r) * 2;
                 pml[0] = m_run;
@@ -362,9 +421,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
         }
         return;
     }
-    const float inv = 1.f / l_tot;
+    const float inv = o_unit / l_tot;
     if (qrow < p.Tq) {
-        E* dst = O + (int64_t)qrow * p.so.t;
+        float* dst = O + (int64_t)qrow * p.so.t;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -376,7 +435,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
                 val[3] = o[db][4 * j + 3] * inv;
                 st4(dst + db * 32 + 8 * j + 4 * g, val);
             }
-        if (g == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] = m_run * p.scale + logf(l_tot);
+        if (g == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] = fmaf(m_run, kLn2, logf(l_tot * kPInv));
     }
 }
 
@@ -385,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(FwdParams p) {
 // LSE = M * scale + ln(sum_s w_s l_s).  One thread per (row, 4 columns).
 template <int D, typename E>
 __global__ __launch_bounds__(256) void attn_fwd_merge_kernel(FwdParams p) {
-    constexpr int BM = kFwdBM;
+    constexpr int BM = fwd_bm(sizeof(E) == 2);
     constexpr int C4 = D / 4;
     constexpr int TPT = BM * C4;  // threads per (split tile, head)
     const int BH = p.B * p.H;
@@ -409,7 +468,7 @@ __global__ __launch_bounds__(256) void attn_fwd_merge_kernel(FwdParams p) {
         const int64_t base = ((int64_t)(s0 + s) * BH + bh) * BM + r;
         const float m = ml[base * 2];
         if (m == -INFINITY) continue;
-        const float wgt = fast_exp2((m - M) * p.c);
+        const float wgt = fast_exp2(sizeof(E) == 4 ? m - M : (m - M) * p.c);
         L = fmaf(ml[base * 2 + 1], wgt, L);
         const f32x4 v = *reinterpret_cast<const f32x4*>(p.part + base * D + 4 * c4);
         acc[0] = fmaf(v[0], wgt, acc[0]);
@@ -421,21 +480,22 @@ __global__ __launch_bounds__(256) void attn_fwd_merge_kernel(FwdParams p) {
     const int b = bh / p.H, h = bh % p.H;
     E* dst = (E*)p.o + b * p.so.b + h * p.so.h + (int64_t)qrow * p.so.t + 4 * c4;
     st4(dst, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
-    if (c4 == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] = M * p.scale + logf(L);
+    if (c4 == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] =
+            sizeof(E) == 4 ? fmaf(M, kLn2, logf(L * kPInv)) : M * p.scale + logf(L);
 }
 
 template <int D, typename E>
 static void launch_merge_t(const FwdParams& p, hipStream_t s) {
-    const int64_t threads = (int64_t)p.n_split * p.B * p.H * kFwdBM * (D / 4);
+    const int64_t threads = (int64_t)p.n_split * p.B * p.H * fwd_bm(sizeof(E) == 2) * (D / 4);
     hipLaunchKernelGGL((attn_fwd_merge_kernel<D, E>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p);
 }
 
-template <int D, typename E>
+template <int D>
 static int launch_fwd_t(const FwdParams& p, hipStream_t s) {
     const int BH = p.B * p.H;
     const dim3 grid((unsigned)((p.n_groups ? p.n_groups : p.n_qtiles) * BH));
-    hipLaunchKernelGGL((attn_fwd_kernel<D, E>), grid, dim3(256), 0, s, p);
-    if (p.n_split) launch_merge_t<D, E>(p, s);
+    hipLaunchKernelGGL((attn_fwd_kernel<D>), grid, dim3(64 * FwdTile<D>::NW), 0, s, p);
+    if (p.n_split) launch_merge_t<D, float>(p, s);
     return (int)hipGetLastError();
 }
 
@@ -487,16 +547,16 @@ static int fwd_slots(int D, int bf16, FwdSlots* out) {
         *out = it->second;
         return 0;
     }
-    // MI355X: 256 CUs; fp32: two D <= 64 workgroups per CU, one at D = 128.
-    int cus = 256, per_cu = bf16 ? (D >= 128 ? 2 : 4) : (D >= 128 ? 1 : 2);
+    // MI355X: 256 CUs; fp32: one workgroup per CU.
+    int cus = 256, per_cu = bf16 ? (D >= 128 ? 2 : 4) : 1;
     if (dev >= 0) {
         int n = 0, occ = 0;
         if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
         hipError_t e = hipErrorInvalidValue;
         if (bf16) e = (hipError_t)fwd_bf16_occupancy(D, &occ);
-        else if (D == 32) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<32, float>, 256, 0);
-        else if (D == 64) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<64, float>, 256, 0);
-        else if (D == 128) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<128, float>, 256, 0);
+        else if (D == 32) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<32>, 64 * FwdTile<32>::NW, 0);
+        else if (D == 64) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<64>, 64 * FwdTile<64>::NW, 0);
+        else if (D == 128) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, attn_fwd_kernel<128>, 64 * FwdTile<128>::NW, 0);
         if (e == hipSuccess && occ > 0) per_cu = occ;
         (void)hipGetLastError();  // a failed query of ours: the defaults stand
     }
@@ -531,7 +591,7 @@ static constexpr double kFwdCuRate[2] = {0.0, 1.1};      // tiles per CU per til
 static constexpr int kFwdMinSplitTiles[2] = {0, 32};
 
 static void fwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, FwdSlots slots, FwdPlan* out) {
-    const int BM = kFwdBM, BN = bf16 ? kFwdBf16BN : D >= 128 ? FwdTile<128>::BN : FwdTile<64>::BN;
+    const int BM = fwd_bm(bf16), BN = bf16 ? kFwdBf16BN : D >= 128 ? FwdTile<128>::BN : D >= 64 ? FwdTile<64>::BN : FwdTile<32>::BN;
     const int ix = bf16 ? 1 : 0;
     const double overhead = kFwdOverhead[ix], merge_cost = kFwdMergeCost[ix], cap = kFwdCuRate[ix] * slots.cus;
     const int slots_per_xcd = slots.per_xcd;
@@ -647,15 +707,15 @@ int fwd_plan(int B, int H, int Tq, int Tk, int D, int causal, int bf16, FwdPlan*
     // 5-7% slower (B2 H8 T4096, B1 H16 T4096, B4 H8 T2048, B1 H8 T8192: 512
     // workgroups on 512 slots) and on larger ones 1-10% faster (config 4, B4
     // H16 T2048, B8 H16 T1024, B8 H12 T1024).
-    out->pv_prio = (int64_t)((Tq + kFwdBM - 1) / kFwdBM) * B * H > 8LL * slots.per_xcd;
+    out->pv_prio = (int64_t)((Tq + fwd_bm(bf16) - 1) / fwd_bm(bf16)) * B * H > 8LL * slots.per_xcd;
     std::lock_guard<std::mutex> lk(mu);
     if (cache.size() > 256) cache.clear();
     cache[key] = *out;
     return 0;
 }
 
-size_t fwd_workspace_bytes(const FwdPlan& plan, int B, int H, int D) {
-    return (size_t)plan.n_slots * B * H * kFwdBM * (size_t)(D + 2) * sizeof(float);
+size_t fwd_workspace_bytes(const FwdPlan& plan, int B, int H, int D, int bf16) {
+    return (size_t)plan.n_slots * B * H * fwd_bm(bf16) * (size_t)(D + 2) * sizeof(float);
 }
 
 int launch_attn_fwd(const FwdParams& p, int bf16, hipStream_t s) {
@@ -671,9 +731,9 @@ int launch_attn_fwd(const FwdParams& p, int bf16, hipStream_t s) {
         return (int)hipGetLastError();
     }
     switch (p.D) {
-        case 32: return launch_fwd_t<32, float>(p, s);
-        case 64: return launch_fwd_t<64, float>(p, s);
-        case 128: return launch_fwd_t<128, float>(p, s);
+        case 32: return launch_fwd_t<32>(p, s);
+        case 64: return launch_fwd_t<64>(p, s);
+        case 128: return launch_fwd_t<128>(p, s);
         default: return (int)hipErrorInvalidValue;
     }
 }

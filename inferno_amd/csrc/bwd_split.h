@@ -144,12 +144,10 @@ __device__ __forceinline__ void bwd_short_delta_store(const BwdParams& p, int bh
 // in the last workgroup to arrive, replace the accumulators by the
 // chunk-ordered sum of all partials.  Returns whether this workgroup goes on
 // to store dK and dV.  Must be reached by every thread of the workgroup.
-template <int NT, int N>
-__device__ __forceinline__ bool bwd_fixup(const BwdParams& p, const BwdWork& wk, f32x16 (&dk)[N], f32x16 (&dv)[N]) {
+template <int NT, int NACC, typename Acc>
+__device__ __forceinline__ bool bwd_fixup_acc(const BwdParams& p, const BwdWork& wk, Acc acc) {
     if (wk.split < 0) return true;
-    constexpr int NACC = 2 * N;
     constexpr int kDeviceScope = 0x10;  // buffer cache policy: sc1
-    auto acc = [&](int a) -> f32x16& { return a < N ? dk[a] : dv[a - N]; };
     __shared__ int s_last;
     const int tid = threadIdx.x;
     const int BH = p.B * p.H;
@@ -190,6 +188,15 @@ __device__ __forceinline__ bool bwd_fixup(const BwdParams& p, const BwdWork& wk,
             }
     }
     return true;
+}
+template <int NT, int N>
+__device__ __forceinline__ bool bwd_fixup(const BwdParams& p, const BwdWork& wk, f32x16 (&dk)[N], f32x16 (&dv)[N]) {
+    return bwd_fixup_acc<NT, 2 * N>(p, wk, [&](int a) -> f32x16& { return a < N ? dk[a] : dv[a - N]; });
+}
+// The same where each wave holds either dK^T or dV^T accumulators.
+template <int NT, int N>
+__device__ __forceinline__ bool bwd_fixup(const BwdParams& p, const BwdWork& wk, f32x16 (&dkv)[N]) {
+    return bwd_fixup_acc<NT, N>(p, wk, [&](int a) -> f32x16& { return dkv[a]; });
 }
 
 }  // namespace inf

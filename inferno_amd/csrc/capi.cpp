@@ -28,7 +28,7 @@ std::atomic<int> g_deterministic{0};
 // in the deterministic mode, else bf16 shapes where the atomics bound the
 // fused kernel (bwd_dq_direct).
 bool dq_from_pass(int det, int B, int H, int Tq, int Tk, int D, inf_dtype dt) {
-    return det || (dt == INF_BF16 && inf::bwd_dq_direct(B * H, Tq, Tk, D, inf::bwd_keys_per_wg(1, D)));
+    return det || (dt == INF_BF16 && inf::bwd_dq_direct(B * H, Tq, Tk, D, inf::bwd_keys_per_wg(1, D, (int64_t)B * H, Tq, Tk)));
 }
 
 size_t round_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
@@ -133,11 +133,16 @@ int inf_get_deterministic(void) { return g_deterministic.load(); }
 namespace {
 
 // INF_OK, or INF_ERR_HIP when an earlier call left a HIP error pending.
+size_t amax_bytes(size_t bh, int Tq, int D) {  // the heads' maxima (fp32)
+    return round_up(bh * inf::bwd_amax_blocks(Tq, D) * 2 * sizeof(float));
+}
+
 int bwd_workspace_bytes(int det, int B, int H, int Tq, int Tk, int D, inf_dtype dt, size_t* out) {
     const size_t bh = (size_t)B * H;
     size_t n = 2 * round_up(bh * Tq * sizeof(float));  // delta and its low part (short rows)
     if (dt == INF_BF16 && !dq_from_pass(det, B, H, Tq, Tk, D, dt))
         n += round_up(bh * Tq * (size_t)D * sizeof(float));  // dQ accumulator
+    if (dt == INF_F32) n += amax_bytes(bh, Tq, D);
     inf::BwdPlan plan;                                        // causal split plan
     if (inf::bwd_plan(B, H, Tq, Tk, D, 1, dt == INF_BF16, &plan)) return INF_ERR_HIP;
     *out = n + round_up(inf::bwd_split_workspace_bytes(plan, B, H, D));
@@ -158,7 +163,7 @@ int inf_attn_workspace_bytes(int op, int B, int H, int Tq, int Tk, int D, inf_dt
         case INF_OP_ATTN_FWD: {
             inf::FwdPlan plan;
             if (inf::fwd_plan(B, H, Tq, Tk, D, 1, dt == INF_BF16, &plan)) return INF_ERR_HIP;
-            *out_bytes = round_up(inf::fwd_workspace_bytes(plan, B, H, D));
+            *out_bytes = round_up(inf::fwd_workspace_bytes(plan, B, H, D, dt == INF_BF16));
             return INF_OK;
         }
         case INF_OP_ATTN_BWD:
@@ -191,11 +196,11 @@ int inf_attn_fwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     p.off = Tk - Tq;
     p.scale = scale;
     p.c = scale * 1.4426950408889634f;
-    p.n_qtiles = (Tq + inf::kFwdBM - 1) / inf::kFwdBM;
+    p.n_qtiles = (Tq + inf::fwd_bm(dt == INF_BF16) - 1) / inf::fwd_bm(dt == INF_BF16);
     inf::FwdPlan plan;
     if (inf::fwd_plan(B, H, Tq, Tk, D, p.causal, dt == INF_BF16, &plan)) return INF_ERR_HIP;
     p.pv_prio = plan.pv_prio;
-    const size_t need = inf::fwd_workspace_bytes(plan, B, H, D);
+    const size_t need = inf::fwd_workspace_bytes(plan, B, H, D, dt == INF_BF16);
     if (need && (!workspace || ws_bytes < need)) return INF_ERR_WORKSPACE;
     if (need && reinterpret_cast<uintptr_t>(workspace) % kAlign) return INF_ERR_ALIGNMENT;
     if (plan.n_groups) {
@@ -247,15 +252,18 @@ int inf_attn_bwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     } else {
         p.dq_acc = static_cast<float*>(dq);
         p.sacc = view(sdq);
+        p.amax = reinterpret_cast<float*>(ws + 2 * round_up(bh * Tq * sizeof(float)));
+        p.n_amax = inf::bwd_amax_blocks(Tq, D);
     }
     p.B = B; p.H = H; p.Tq = Tq; p.Tk = Tk; p.D = D;
     p.causal = causal ? 1 : 0;
     p.off = Tk - Tq;
     p.scale = scale;
     p.c = scale * 1.4426950408889634f;
-    const int bk = inf::bwd_keys_per_wg(dt == INF_BF16, D);
+    const int bk = inf::bwd_keys_per_wg(dt == INF_BF16, D, (int64_t)B * H, Tq, Tk);
+    p.keys_per_wg = bk;
     p.n_kblocks = (Tk + bk - 1) / bk;
-    p.n_short = inf::bwd_short_rows(B, H, Tq, Tk, p.causal, bk);
+    p.n_short = inf::bwd_short_rows(B, H, Tq, Tk, p.causal, inf::bwd_short_keys(dt == INF_BF16, bk));
     p.dq_direct = dq_from_pass(det, B, H, Tq, Tk, D, dt) ? 1 : 0;
     p.n_qtiles = (Tq + inf::kBwdDqBM - 1) / inf::kBwdDqBM;
     if (p.dq_direct) p.dq_acc = nullptr;  // dq is written by the dQ pass
@@ -264,6 +272,7 @@ int inf_attn_bwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     if (plan.n_groups) {
         size_t offset = 2 * round_up(bh * Tq * sizeof(float));
         if (dt == INF_BF16 && !p.dq_direct) offset += round_up(bh * Tq * (size_t)D * sizeof(float));
+        if (dt == INF_F32) offset += amax_bytes(bh, Tq, D);
         const size_t part_bytes = (size_t)plan.n_slots * bh * 2 * (size_t)D * plan.bk * sizeof(float);
         p.part = reinterpret_cast<float*>(ws + offset);
         p.counters = reinterpret_cast<unsigned*>(ws + offset + part_bytes);

@@ -38,7 +38,7 @@ struct FwdParams {
     int n_qtiles;
     int n_groups;         // 0: one group per query tile, heaviest first (no split)
     int n_slots;          // partial slots in use
-    float* part;          // workspace: n_slots * B*H * kFwdBM * (D + 2) floats
+    float* part;          // workspace: n_slots * B*H * fwd_bm * (D + 2) floats
     int n_split;          // query tiles whose key range is split
     int pv_prio;          // bf16 D = 128 unsplit: P.V MFMAs at raised wave priority (see fwd_plan)
     FwdGroup groups[kMaxFwdGroups];
@@ -58,7 +58,7 @@ struct FwdPlan {
 };
 // Returns 0, or the HIP error an earlier call left pending (see report_pending_error).
 int fwd_plan(int B, int H, int Tq, int Tk, int D, int causal, int bf16, FwdPlan* out);
-size_t fwd_workspace_bytes(const FwdPlan& plan, int B, int H, int D);
+size_t fwd_workspace_bytes(const FwdPlan& plan, int B, int H, int D, int bf16);
 
 // Backward work split: a group is one key block's query-tile range [t0, t1)
 // (in 32-row tiles) for every (b, h).  Groups of a split key block write fp32
@@ -100,7 +100,10 @@ struct BwdParams {
     int B, H, Tq, Tk, D;
     int causal, off;
     float scale, c;
+    float* amax;          // fp32: workspace, [B*H, n_amax, 2] largest |q| and |dO| of bwd_pre's workgroups
+    int n_amax;
     int n_kblocks;
+    int keys_per_wg;
     int dq_direct;          // bf16: dQ from the query-major pass (no accumulator, no atomics)
     int pre_delta;          // bwd_pre computes delta (set by the launcher: off where no kernel reads it)
     int n_qtiles;           // query tiles of kBwdDqBM rows (dQ pass)
@@ -323,19 +326,30 @@ int launch_masked_fill(const void* in, const void* mask, void* out, const Masked
                        int mask_bytes, uint64_t fill_bits, hipStream_t s);
 
 // Tile shapes the host needs for grids and workspace sizing.
-constexpr int kFwdBM = 128;      // query rows per forward workgroup
+// Query rows per forward workgroup: 4 waves x 32 (bf16), 8 waves x 32 (fp32).
+constexpr int kFwdBM = 128;
+constexpr int fwd_bm(int bf16) { return bf16 ? kFwdBM : 256; }
 constexpr int kFwdBf16BN = 64;   // keys per K/V tile of the bf16 forward (every D)
-// Backward workgroups: one wave per 32 keys.  bf16 at D = 64: 8 waves = 256
+// bf16 backward workgroups: one wave per 32 keys.  At D = 64: 8 waves = 256
 // keys, half the dQ atomics per key (two waves per SIMD, as with two 4-wave
-// workgroups); at bf16 speed the atomics are a device-wide limit.  fp32 keeps
-// 4 waves (its atomics cost ~2.5%, and 256-key blocks measured 5-10% slower
-// under a causal mask: fewer, heavier workgroups).  fp32 at D = 128 needs
-// ~430 registers per wave (one wave per SIMD) and D = 32 keeps three 4-wave
-// workgroups per CU: both use 4 waves.  bf16 at D = 128 runs its own kernel,
-// 8 waves x 16 keys: 128 keys per workgroup, as with 4 x 32.
-constexpr int bwd_waves(int bf16, int D) { return bf16 && D == 64 ? 8 : 4; }
-constexpr int bwd_bf16_waves(int D) { return bwd_waves(1, D); }
-inline int bwd_keys_per_wg(int bf16, int D) { return bf16 && D == 128 ? 128 : 32 * bwd_waves(bf16, D); }
+// workgroups); at bf16 speed the atomics are a device-wide limit.  D = 32 keeps
+// three 4-wave workgroups per CU.  D = 128 runs its own kernel, 8 waves x 16
+// keys: 128 keys per workgroup, as with 4 x 32.
+constexpr int bwd_bf16_waves(int D) { return D == 64 ? 8 : 4; }
+// BH = B * H.  fp32 at D <= 64 takes 256 keys (64 per pair of waves: fewer dQ
+// atomics, each staged query tile serves twice the keys), or 128 where a
+// workgroup's serial walk over few query tiles is what counts: with one key
+// block, or a grid that leaves CUs idle and short walks (B1 H12 T333 D64 backward
+// 40.6 -> 26.0 us, B8 H12 T256 44 -> 37; but B2 H12 T1024 64 -> 78, B8 H12 T1024
+// 159 -> 207).
+inline int bwd_keys_per_wg(int bf16, int D, int64_t BH, int Tq, int Tk) {
+    if (D == 128) return 128;
+    if (bf16) return 32 * bwd_bf16_waves(D);
+    const int64_t wgs = BH * ((Tk + 127) / 128);
+    return Tk <= 128 || (wgs <= 256 && wgs * ((Tq + 31) / 32) < 4096) ? 128 : 256;
+}
+// bwd_pre's workgroups per head, fp32 (256 threads, 4 elements each).
+inline int bwd_amax_blocks(int Tq, int D) { return (Tq + 1024 / D - 1) / (1024 / D); }
 constexpr int kBwdBQ = 32;       // query rows per backward inner step
 // Leading query rows whose visible keys all lie in key block 0 (keys_per_wg
 // keys): their softmax-backward row dot is formed inside the block-0
@@ -348,6 +362,10 @@ constexpr int kBwdBQ = 32;       // query rows per backward inner step
 // and dP on every short row again).  Rows with one visible key need no row
 // dot: every kernel sets their dS to 0, as P (dP - dP) is.
 constexpr int64_t kBwdShortMaxRows = 4096;
+// ... and, where a key block is wider, only rows that see keys of its first 128
+// (fp32): later rows see enough keys to set no scale of their own, and the
+// prologue is a serial part of small problems.
+constexpr int bwd_short_keys(int bf16, int keys_per_wg) { return bf16 || keys_per_wg < 128 ? keys_per_wg : 128; }
 inline int bwd_short_rows(int B, int H, int Tq, int Tk, int causal, int keys_per_wg) {
     int64_t r = causal ? (int64_t)keys_per_wg - ((int64_t)Tk - Tq) : (Tk <= keys_per_wg ? Tq : 0);
     r = r < 0 ? 0 : (r > Tq ? Tq : r);
