@@ -34,7 +34,7 @@ COMMON = [
 ]
 
 SOURCES = ["capi.cpp", "attn_fwd.hip", "attn_fwd_bf16.hip", "attn_bwd.hip", "attn_bwd_bf16.hip", "decode.hip", "softmax.hip", "elementwise.hip", "nn.hip",
-           "capi_nn.cpp", "gemm.cpp"]
+           "capi_nn.cpp", "gemm.cpp", "gemm_split.hip"]
 
 
 def _compile(src: Path, obj: Path) -> None:

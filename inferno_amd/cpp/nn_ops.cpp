@@ -2,7 +2,7 @@
 // qkv_attention and sum_to_shape, with their backward nodes
 // (include/inferno/core/ops.h, include/inferno/gradfn/nnbackward.h).
 //
-// HIP tensors go through the C-ABI (inf_gemm on hipBLASLt, the nn.hip kernels,
+// HIP tensors go through the C-ABI (inf_gemm, the nn.hip kernels,
 // the fused attention kernels); nothing here falls back to the CPU for a HIP
 // tensor.  CPU tensors run plain loops that follow the reference's CPU kernels
 // (cpu_matmul's k-ordered fp32 sums, cpu_layer_normalization,
@@ -48,13 +48,20 @@ struct Scratch {
     }
 };
 
-// The hipBLASLt workspace of each device, kept for the life of the process.
+// The GEMM workspace of each device, kept for the life of the process.  Calls on a
+// device are ordered on its library stream, but a product may take two launches
+// with its partial sums in the workspace between them: the caller holds
+// gemm_mutex until inf_gemm returns, so that no other thread's product is queued
+// between the two.
+std::mutex& gemm_mutex() {
+    static auto* mu = new std::mutex();
+    return *mu;
+}
+
 void* gemm_workspace(const Device& dev, size_t* bytes) {
-    static std::mutex mu;
     static auto* per_device = new std::vector<Tensor>();
     size_t need = 0;
     status_check(inf_nn_workspace_bytes(INF_OP_GEMM, 0, 0, &need), "inf_nn_workspace_bytes");
-    std::lock_guard<std::mutex> lk(mu);
     if (per_device->size() <= (size_t)dev.index) per_device->resize((size_t)dev.index + 1);
     Tensor& t = (*per_device)[(size_t)dev.index];
     if (!t.defined()) t = Tensor(DType::Float32, {need / 4 + 64}, "gemm_ws", dev, false);
@@ -66,6 +73,7 @@ void* gemm_workspace(const Device& dev, size_t* bytes) {
 void gemm_hip(const Device& dev, DType dt, bool ta, bool tb, int64_t M, int64_t N, int64_t K, float alpha,
               const void* A, int64_t lda, int64_t sa, const void* B, int64_t ldb, int64_t sb, float beta, void* C,
               int64_t ldc, int64_t sc, int64_t batch, const void* bias) {
+    std::lock_guard<std::mutex> lk(gemm_mutex());
     size_t wsb = 0;
     void* ws = gemm_workspace(dev, &wsb);
     DeviceGuard g(dev.index);

@@ -13,7 +13,7 @@
 
 namespace {
 
-constexpr size_t kGemmWorkspace = size_t(32) << 20;  // hipBLASLt workspace offered to the heuristic
+constexpr size_t kGemmWorkspace = size_t(32) << 20;  // offered to hipBLASLt's heuristic; bounds a split K's partial sums
 
 bool dtype_ok(int dt) { return dt == INF_F32 || dt == INF_BF16; }
 int esz(inf_dtype dt) { return dt == INF_F32 ? 4 : 2; }

@@ -1,8 +1,8 @@
-// gemm.cpp -- row-major (batched) GEMM for the Linear / matmul ops, on hipBLASLt.
+// gemm.cpp -- row-major (batched) GEMM for the Linear / matmul ops.
 //
-// The Linear layers of the GPT step are plain dense contractions, so they go
-// to the vendor library rather than a hand-written kernel.  hipBLASLt picks
-// gfx950 MFMA kernels; with fp32 operands it runs the fp32 matrix path
+// Large fp32 products run on the split-operand kernel (gemm_split.hip); the
+// others are plain dense contractions that go to the vendor library.  hipBLASLt
+// picks gfx950 MFMA kernels; with fp32 operands it runs the fp32 matrix path
 // (v_mfma_f32_*_f32), never a reduced-precision one.
 //
 // Row-major C[M,N] = alpha * op(A)[M,K] op(B)[K,N] + beta * C (+ bias[N] per
@@ -144,6 +144,12 @@ int launch_gemm(const GemmArgs& g, hipStream_t s) {
                          " (" + hipGetErrorString(pending) + "); nothing launched");
         return 1;
     }
+    bool taken = false;
+    if (const int e = launch_gemm_split(g, s, &taken)) {
+        set_error_detail(std::string("inf_gemm: ") + hipGetErrorName((hipError_t)e) + " launching the split-operand kernel");
+        return 1;
+    }
+    if (taken) return 0;
     Key k;
     std::memset(&k, 0, sizeof(k));  // padding bytes take part in hashing / comparison
     k.ta = g.ta;

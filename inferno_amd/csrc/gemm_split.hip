@@ -1,0 +1,427 @@
+// gemm_split.hip -- fp32 GEMM on the fp16 matrix cores: every operand split into
+// two fp16 parts (common.h), three MFMAs per product step, fp32 accumulators.
+//
+// Row-major C = alpha * op(A) op(B) + beta * C (+ bias per row).  One workgroup
+// = 8 waves = a 256 x 128 tile of C, each wave 64 x 64 of it (2 x 2 MFMA blocks: a
+// block's operand is read from LDS once for two of them), K in steps of 32.  A
+// step's operands are loaded two steps ahead into registers, split, and stored to
+// double-buffered LDS as 16-byte units of 8 consecutive k of one row of A or
+// column of B, which is what an MFMA lane takes: one barrier per step.
+//   K-contiguous operand (A, or B transposed): a thread loads 8 k of a row (two
+//     16-byte loads; 4 threads cover the row's step).
+//   K-strided operand (A transposed, or B): a thread loads 8 k of one column
+//     (eight 4-byte loads, each a run over the lanes), so the transposition costs
+//     no store.
+// Every row of A and column of B is scaled by the class of its largest magnitude
+// so far, which the threads that stage it agree on without LDS (neighbouring
+// lanes).  When a row's class grows (as a rule in the first step only), the
+// accumulators, kept in units of row times column scale, move with it.
+// The matrix cores' fp16 sums round a little towards -infinity (2e-8 of a result's
+// rms on average, which a sum over thousands of rows of C would show): half of the
+// rows and columns, by the parity of their index's bits, are negated with their
+// scale, so that half of the results are formed as their negatives and what is left
+// cancels in sums over rows or columns of C (8192 rows summed: 1.8e-6 off without,
+// 5e-7 with the vendor library's fp32 kernel, 3e-7 here).
+// A non-finite element makes its row's or column's results NaN; the epilogue
+// forms those again one by one in plain fp32, so infinities come out as before.
+//
+// Few tiles and a long K: the K range is split over workgroups, their partial
+// tiles go to the workspace and a second kernel sums them in order.
+//
+// Bound by the splitting VALU work and the MFMAs, which overlap only in part
+// (4096^3: matrix cores busy 40% of the cycles, VALU 42%), at a shader clock that
+// falls to 1.7-2.0 GHz with the load.  Against the vendor library's fp32 kernels
+// (us): 8192 x 3072 x 768 280 -> 178, 8192 x 768 x 3072 266 -> 158, 768 x 3072 x 8192
+// (A transposed) 291 -> 164, 4096^3 915 -> 470.  Tiles of 128 x 128 in four-wave
+// workgroups, two per CU, split a third more and took 5-8% longer except at
+// 8192 x 2304 x 768 (159 against 169).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+
+namespace inf {
+
+namespace {
+
+constexpr int kBM = 256, kBN = 128, kBK = 32, kNT = 512;
+constexpr int kKG = kBK / 8;  // 8-k units per row and step
+
+struct GemmSplitParams {
+    const float* A;
+    const float* B;
+    float* C;
+    const float* bias;
+    float* part;              // split K: [ksplit, M, N] partial products
+    int M, N, K;
+    int64_t lda, ldb, ldc, sa, sb, sc;
+    float alpha, beta;
+    int tiles_m, tiles_n;
+    int ksplit, kchunk;       // K range per split, a multiple of kBK
+};
+
+// One operand's staging: rows row0 .. row0 + ROWS - 1, U units of 8 k per thread
+// (NT = ROWS * 4 / U threads).
+template <bool KC, int ROWS, int U>
+struct Stage {
+    static constexpr int US = ROWS + 4;  // units per 8-k group in LDS (64 bytes of padding)
+    static constexpr bool ONE_ROW = !KC && U == 2;  // a thread's units belong to one row
+    using Raw = f32x4[U][2];
+    Raw raw[2];          // two steps' loads
+    int cls[U];          // scale class of the unit's row
+    uint32_t neg[U];     // sign bit of the row's scale
+    const float* base;   // KC: row row0, k 0; else: k 0, column row0
+    int64_t ld;
+    int rows, row_a;     // rows of the operand in this tile; this thread's first row
+    int kg;              // this thread's first 8-k group
+    uint32_t voff;
+
+    __device__ __forceinline__ void init(const float* op, int64_t ld_, int row0, int rows_total, int tid) {
+        const int lane = tid & 63, wave = tid >> 6;
+        ld = ld_;
+        rows = min(rows_total - row0, ROWS);
+        if constexpr (KC) {  // 16 rows a wave, 4 neighbouring lanes a row (128 bytes)
+            base = op + (int64_t)row0 * ld;
+            row_a = 16 * wave + (lane >> 2);
+            kg = lane & 3;
+            voff = (uint32_t)(((int64_t)row_a * ld + 8 * kg) * 4);
+        } else {
+            base = op + row0;
+            row_a = U == 2 ? 32 * wave + (lane & 31) : 16 * wave + (lane & 15);
+            kg = U == 2 ? lane >> 5 : lane >> 4;
+            voff = (uint32_t)(((int64_t)(8 * kg) * ld + row_a) * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            cls[i] = 2;
+            neg[i] = (uint32_t)__popc(KC ? row_a + ROWS / 2 * i : row_a) << 31;
+        }
+    }
+    __device__ __forceinline__ float with_sign(float v, int i) const {
+        return __uint_as_float(__float_as_uint(v) ^ neg[i]);
+    }
+    // k0 .. k0 + 31 below kend; elements outside read as zeros.
+    __device__ __forceinline__ void load(Raw& r, int k0, int kend) const {
+        const int ks = min(kend - k0, kBK);
+        if constexpr (KC) {
+            const uint32_t bytes = ks > 0 ? (uint32_t)(((int64_t)(rows - 1) * ld + ks) * 4) : 0u;
+            const auto rs = buffer_rsrc(base + k0, bytes);
+            const uint32_t v = 8 * kg < ks ? voff : 0x40000000u;  // past the end of every resource
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const uint32_t so = (uint32_t)((int64_t)(ROWS / 2 * i) * ld * 4);
+                r[i][0] = buffer_ld4(rs, v, so);
+                r[i][1] = buffer_ld4(rs, v + 16, so);
+            }
+        } else {
+            const uint32_t bytes = ks > 0 ? (uint32_t)(((int64_t)(ks - 1) * ld + rows) * 4) : 0u;
+            const auto rs = buffer_rsrc(base + (int64_t)k0 * ld, bytes);
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    r[i][e >> 2][e & 3] = buffer_ld1(rs, voff, (uint32_t)((int64_t)(16 * i + e) * ld * 4));
+        }
+    }
+    // Split the loaded step into LDS; chg[row] = what the row's accumulators are
+    // to be multiplied by.  Returns whether some row's class changed.
+    __device__ __forceinline__ bool store(const Raw& r, f16x8 (&L)[2][kKG][US], float (&chg)[ROWS]) {
+        float mx[U], f[U];
+        bool over = false;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            mx[i] = absmax8(0.f, r[i][0], r[i][1]);
+            over |= mx[i] >= class_limit(cls[i]);
+            f[i] = 1.f;
+        }
+        const bool grow = __any(over);
+        if (grow) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) mx[i] = absmax8_finite(0.f, r[i][0], r[i][1]);
+            agree(mx);
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const int nc = max(cls[i], scale_class(mx[i]));
+                f[i] = class_scale(nc) * class_inv(cls[i]);
+                cls[i] = nc;
+            }
+        }
+        put_rows(chg, f);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const Half2x8 h = split2(r[i][0], r[i][1], with_sign(class_scale(cls[i]), i));
+            const int g = KC ? kg : kg + 2 * i, row = KC ? row_a + ROWS / 2 * i : row_a;
+            L[0][g][row] = h.h;
+            L[1][g][row] = h.l;
+        }
+        return grow;
+    }
+    __device__ __forceinline__ void put_units(float (&dst)[ROWS]) const {
+        float u[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) u[i] = with_sign(class_inv(cls[i]), i);
+        put_rows(dst, u);
+    }
+
+private:
+    // the largest over the lanes that hold parts of a row's step
+    static __device__ __forceinline__ void agree(float (&mx)[U]) {
+        if constexpr (ONE_ROW) mx[0] = mx[U - 1] = fmaxf(mx[0], mx[U - 1]);
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            if constexpr (KC) mx[i] = group_max<4>(mx[i]);
+            if constexpr (!KC && U == 1) mx[i] = fmaxf(mx[i], shfl_xor(mx[i], 16));
+            if constexpr (!KC) mx[i] = max_xor32(mx[i]);
+        }
+    }
+    __device__ __forceinline__ void put_rows(float (&dst)[ROWS], const float (&v)[U]) const {
+        if (kg == 0) {
+            dst[row_a] = v[0];
+            if constexpr (KC && U == 2) dst[row_a + ROWS / 2] = v[1];
+        }
+    }
+};
+
+}  // namespace
+
+template <bool AKC, bool BKC>
+__global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
+    using StageA = Stage<AKC, kBM, 2>;
+    using StageB = Stage<BKC, kBN, 1>;
+    __shared__ f16x8 Ua[2][2][kKG][StageA::US];  // [buffer][part][8-k group][row]
+    __shared__ f16x8 Ub[2][2][kKG][StageB::US];
+    __shared__ __attribute__((aligned(16))) float chg_a[2][kBM];
+    __shared__ __attribute__((aligned(16))) float chg_b[2][kBN];
+    __shared__ int tag_s[2];  // the last step whose staging changed a class, per buffer
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31;
+    const int g = lane >> 5;
+    const int wm = wave >> 1, wn = wave & 1;
+
+    // Consecutive workgroups go to the 8 XCDs in turn: each XCD takes a run of
+    // tiles, so that it finds their operand panels in its own L2.
+    const int n_tiles = p.tiles_m * p.tiles_n;
+    const int per = (n_tiles + 7) / 8;
+    const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per || tile >= n_tiles) return;
+    const int m0 = tile / p.tiles_n * kBM, n0 = tile % p.tiles_n * kBN;
+    const int split = blockIdx.y;
+    const int kb = split * p.kchunk, ke = min(p.K, kb + p.kchunk);
+    const int nt = (ke - kb + kBK - 1) / kBK;
+    const float* A = p.A + blockIdx.z * p.sa;
+    const float* B = p.B + blockIdx.z * p.sb;
+    float* C = p.C + blockIdx.z * p.sc;
+
+    StageA sa;
+    StageB sb;
+    sa.init(A, p.lda, m0, p.M, tid);
+    sb.init(B, p.ldb, n0, p.N, tid);
+
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+
+    if (tid < 2) tag_s[tid] = -1;
+    sa.load(sa.raw[0], kb, ke);
+    sb.load(sb.raw[0], kb, ke);
+    sa.load(sa.raw[1], kb + kBK, ke);
+    sb.load(sb.raw[1], kb + kBK, ke);
+    __syncthreads();
+    {
+        const bool ga = sa.store(sa.raw[0], Ua[0], chg_a[0]), gb = sb.store(sb.raw[0], Ub[0], chg_b[0]);
+        if ((ga || gb) && lane == 0) tag_s[0] = 0;
+    }
+    __syncthreads();
+
+    // Step t computes on buffer BUF = t % 2; step t + 1, loaded in the previous
+    // step, is split into the other buffer, and step t + 2's loads go out.
+    auto step = [&](int t, auto buf_c) {
+        constexpr int BUF = decltype(buf_c)::value;
+        sa.load(sa.raw[BUF], kb + (t + 2) * kBK, ke);
+        sb.load(sb.raw[BUF], kb + (t + 2) * kBK, ke);
+        if (__builtin_amdgcn_readfirstlane(tag_s[BUF]) == t) {
+            float fb[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) fb[j] = chg_b[BUF][64 * wn + 32 * j + l32];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float fa = chg_a[BUF][64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3)];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j][r] *= fa * fb[j];
+                }
+        }
+#pragma unroll
+        for (int kk = 0; kk < kBK / 16; ++kk) {
+            Half2x8 a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i].h = Ua[BUF][0][2 * kk + g][64 * wm + 32 * i + l32];
+                a[i].l = Ua[BUF][1][2 * kk + g][64 * wm + 32 * i + l32];
+                b[i].h = Ub[BUF][0][2 * kk + g][64 * wn + 32 * i + l32];
+                b[i].l = Ub[BUF][1][2 * kk + g][64 * wn + 32 * i + l32];
+            }
+            // the small part products first, four independent accumulators in turn
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = mfma32x32x16f16(q == 0 ? a[i].l : a[i].h, q == 1 ? b[j].l : b[j].h, acc[i][j]);
+        }
+        const bool ga = sa.store(sa.raw[BUF ^ 1], Ua[BUF ^ 1], chg_a[BUF ^ 1]);
+        const bool gb = sb.store(sb.raw[BUF ^ 1], Ub[BUF ^ 1], chg_b[BUF ^ 1]);
+        if ((ga || gb) && lane == 0) tag_s[BUF ^ 1] = t + 1;
+        __syncthreads();
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    for (int t = 0; t < nt; t += 2) {
+        step(t, B0{});
+        if (t + 1 < nt) step(t + 1, B1{});
+    }
+
+    // ---- epilogue ------------------------------------------------------------------
+    sa.put_units(chg_a[0]);
+    sb.put_units(chg_b[0]);
+    __syncthreads();
+    float chk = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) chk = fmaf(acc[i][j][r], 0.f, chk);
+    const bool bad = __any(chk != 0.f);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int n = n0 + 64 * wn + 32 * j + l32;
+        const float ub = chg_b[0][64 * wn + 32 * j + l32];
+        const float bias = p.bias && n < p.N && p.ksplit == 1 ? p.bias[n] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int ml = 64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
+                const int m = m0 + ml;
+                float v = acc[i][j][r] * chg_a[0][ml] * ub;
+                if (bad && __any(!(fabsf(v) < INFINITY))) {
+                    if (!(fabsf(v) < INFINITY) && m < p.M && n < p.N) {
+                        v = 0.f;
+#pragma unroll 1
+                        for (int k = kb; k < ke && v == v; ++k)  // a NaN stays one
+                            v = fmaf(AKC ? A[(int64_t)m * p.lda + k] : A[(int64_t)k * p.lda + m],
+                                     BKC ? B[(int64_t)n * p.ldb + k] : B[(int64_t)k * p.ldb + n], v);
+                    }
+                }
+                if (m < p.M && n < p.N) {
+                    if (p.ksplit > 1) {
+                        p.part[((int64_t)split * p.M + m) * p.N + n] = v;
+                    } else {
+                        float* c = C + (int64_t)m * p.ldc + n;
+                        v = fmaf(v, p.alpha, bias);
+                        *c = p.beta != 0.f ? fmaf(p.beta, *c, v) : v;
+                    }
+                }
+            }
+    }
+}
+
+// C from the partial products of a split K, summed in order.
+__global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams p) {
+    const int64_t mn = (int64_t)p.M * p.N;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < mn; i += (int64_t)gridDim.x * 256) {
+        float v = 0.f;
+        for (int s = 0; s < p.ksplit; ++s) v += p.part[s * mn + i];
+        const uint32_t m = (uint32_t)(i / (uint32_t)p.N), n = (uint32_t)(i - (int64_t)m * p.N);
+        float* c = p.C + (int64_t)m * p.ldc + n;
+        v = fmaf(v, p.alpha, p.bias ? p.bias[n] : 0.f);
+        *c = p.beta != 0.f ? fmaf(p.beta, *c, v) : v;
+    }
+}
+
+// Whether the kernel takes the problem: fp32; a K-contiguous operand is read 8
+// elements at a time (K % 8, 16-byte rows); 32-bit offsets inside a tile's panel;
+// alpha = 0 must not read operands that may hold infinities.
+static bool split_takes(const GemmArgs& g) {
+    if (g.bf16 || g.alpha == 0.f || g.K % 8 != 0 || g.lda > (1 << 20) || g.ldb > (1 << 20)) return false;
+    auto rows16 = [](const void* p, int64_t ld, int64_t stride) {
+        return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && stride % 4 == 0;
+    };
+    if (!g.ta && !rows16(g.A, g.lda, g.batch > 1 ? g.sa : 0)) return false;
+    if (g.tb && !rows16(g.B, g.ldb, g.batch > 1 ? g.sb : 0)) return false;
+    return g.batch <= 65535;
+}
+
+int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
+    *taken = false;
+    if (!split_takes(g)) return 0;
+    GemmSplitParams p{};
+    p.A = (const float*)g.A;
+    p.B = (const float*)g.B;
+    p.C = (float*)g.C;
+    p.bias = (const float*)g.bias;
+    p.M = (int)g.M;
+    p.N = (int)g.N;
+    p.K = (int)g.K;
+    p.lda = g.lda;
+    p.ldb = g.ldb;
+    p.ldc = g.ldc;
+    p.sa = g.batch > 1 ? g.sa : 0;
+    p.sb = g.batch > 1 ? g.sb : 0;
+    p.sc = g.batch > 1 ? g.sc : 0;
+    p.alpha = g.alpha;
+    p.beta = g.beta;
+    p.tiles_m = (int)((g.M + kBM - 1) / kBM);
+    p.tiles_n = (int)((g.N + kBN - 1) / kBN);
+    // The number of K ranges: the cheapest under a model (microseconds) fitted to
+    // measured shapes: the longest chain of K steps on a CU (1.65 a step, 8 steps
+    // for a workgroup's start and end) or, where the device is full and its clock
+    // falls with the load, the steps over the rate that large products reach;
+    // partials pass through memory once more.
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * g.batch;
+    const int nk = (p.K + kBK - 1) / kBK;
+    double best = 1e30;
+    int ks = 1;
+    for (int c = 1; c <= 8; ++c) {
+        if (c > 1 && (g.batch > 1 || nk / c < 8 || (size_t)c * g.M * g.N * sizeof(float) > g.ws_bytes ||
+                      reinterpret_cast<uintptr_t>(g.ws) % 16))
+            break;
+        const double wgs = (double)(tiles * c), steps = (nk + c - 1) / c + 8;
+        double cost = std::max(steps * 1.65 * std::ceil(wgs / 256), wgs * steps / 146.0);
+        if (c > 1) cost += 4.0 + (double)(c + 1) * g.M * g.N * 4 / 4e6;
+        if (cost < best) {
+            best = cost;
+            ks = c;
+        }
+    }
+    // The vendor library's fp32 kernels (about 142 TFLOP/s, better split for small
+    // problems) where the model says that they are no slower: 1024^3 19 us there
+    // and 35 here, 1536^3 62 and 47, M = 32 rows 9-18 and 25.
+    if (best > 2.0 * g.M * g.N * g.K * g.batch / 142e6 + 8.0) return 0;
+    p.kchunk = (nk + ks - 1) / ks * kBK;
+    p.ksplit = (p.K + p.kchunk - 1) / p.kchunk;
+    p.part = (float*)g.ws;
+    const int per = (p.tiles_m * p.tiles_n + 7) / 8;
+    const dim3 grid((unsigned)(8 * per), (unsigned)p.ksplit, (unsigned)g.batch), block(kNT);
+    if (!g.ta && !g.tb) hipLaunchKernelGGL((gemm_split_kernel<true, false>), grid, block, 0, s, p);
+    else if (!g.ta) hipLaunchKernelGGL((gemm_split_kernel<true, true>), grid, block, 0, s, p);
+    else if (!g.tb) hipLaunchKernelGGL((gemm_split_kernel<false, false>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm_split_kernel<false, true>), grid, block, 0, s, p);
+    if (p.ksplit > 1)
+        hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)std::min<int64_t>((g.M * g.N + 255) / 256, 2048)),
+                           dim3(256), 0, s, p);
+    *taken = true;
+    return (int)hipGetLastError();
+}
+
+}  // namespace inf

@@ -237,6 +237,9 @@ struct GemmArgs {         // row-major C = alpha * op(A) op(B) + beta * C (+ bia
 };
 // 0 = ok, 1 = library error, 2 = no algorithm for the problem
 int launch_gemm(const GemmArgs& g, hipStream_t s);
+// fp32 on the fp16 matrix cores (gemm_split.hip); *taken: whether the problem is one of its
+// own (else nothing was launched).  Returns a hipError_t value.
+int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken);
 
 // Thread-local text about the last failure inside the library (inf_last_error_detail).
 void set_error_detail(const std::string& msg);
