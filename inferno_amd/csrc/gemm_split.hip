@@ -29,10 +29,10 @@
 // tiles go to the workspace and a second kernel sums them in order.
 //
 // Bound by the splitting VALU work and the MFMAs, which overlap only in part
-// (4096^3: matrix cores busy 40% of the cycles, VALU 42%), at a shader clock that
+// (4096^3: matrix cores busy 42% of the cycles, VALU 44%), at a shader clock that
 // falls to 1.7-2.0 GHz with the load.  Against the vendor library's fp32 kernels
-// (us): 8192 x 3072 x 768 280 -> 178, 8192 x 768 x 3072 266 -> 158, 768 x 3072 x 8192
-// (A transposed) 291 -> 164, 4096^3 915 -> 470.  Tiles of 128 x 128 in four-wave
+// (us): 8192 x 3072 x 768 280 -> 174, 8192 x 768 x 3072 266 -> 152, 768 x 3072 x 8192
+// (A transposed) 291 -> 160, 4096^3 915 -> 460, 3309 x 664 x 2656 110 -> 62.  Tiles of 128 x 128 in four-wave
 // workgroups, two per CU, split a third more and took 5-8% longer except at
 // 8192 x 2304 x 768 (159 against 169).
 #include <algorithm>
@@ -60,6 +60,7 @@ struct GemmSplitParams {
     float alpha, beta;
     int tiles_m, tiles_n;
     int ksplit, kchunk;       // K range per split, a multiple of kBK
+    int items;                // tiles x K ranges x batch
 };
 
 // One operand's staging: rows row0 .. row0 + ROWS - 1, U units of 8 k per thread
@@ -108,12 +109,13 @@ struct Stage {
         if constexpr (KC) {
             const uint32_t bytes = ks > 0 ? (uint32_t)(((int64_t)(rows - 1) * ld + ks) * 4) : 0u;
             const auto rs = buffer_rsrc(base + k0, bytes);
-            const uint32_t v = 8 * kg < ks ? voff : 0x40000000u;  // past the end of every resource
+            const uint32_t end = 0x40000000u;  // past the end of every resource
+            const uint32_t v = 8 * kg < ks ? voff : end, v2 = 8 * kg + 4 < ks ? voff + 16 : end;
 #pragma unroll
             for (int i = 0; i < U; ++i) {
                 const uint32_t so = (uint32_t)((int64_t)(ROWS / 2 * i) * ld * 4);
                 r[i][0] = buffer_ld4(rs, v, so);
-                r[i][1] = buffer_ld4(rs, v + 16, so);
+                r[i][1] = buffer_ld4(rs, v2, so);
             }
         } else {
             const uint32_t bytes = ks > 0 ? (uint32_t)(((int64_t)(ks - 1) * ld + rows) * 4) : 0u;
@@ -125,9 +127,9 @@ struct Stage {
                     r[i][e >> 2][e & 3] = buffer_ld1(rs, voff, (uint32_t)((int64_t)(16 * i + e) * ld * 4));
         }
     }
-    // Split the loaded step into LDS; chg[row] = what the row's accumulators are
-    // to be multiplied by.  Returns whether some row's class changed.
-    __device__ __forceinline__ bool store(const Raw& r, f16x8 (&L)[2][kKG][US], float (&chg)[ROWS]) {
+    // The rows' classes for the loaded step; chg[row] = what the row's accumulators
+    // are to be multiplied by.  Returns whether some row's class changed.
+    __device__ __forceinline__ bool classes(const Raw& r, float (&chg)[ROWS]) {
         float mx[U], f[U];
         bool over = false;
 #pragma unroll
@@ -149,6 +151,11 @@ struct Stage {
             }
         }
         put_rows(chg, f);
+        return grow;
+    }
+    // Split the loaded step into LDS (no branch, so that it can be scheduled between
+    // the MFMAs of the step before: 3-5% of the time).
+    __device__ __forceinline__ void store(const Raw& r, f16x8 (&L)[2][kKG][US]) const {
 #pragma unroll
         for (int i = 0; i < U; ++i) {
             const Half2x8 h = split2(r[i][0], r[i][1], with_sign(class_scale(cls[i]), i));
@@ -156,7 +163,6 @@ struct Stage {
             L[0][g][row] = h.h;
             L[1][g][row] = h.l;
         }
-        return grow;
     }
     __device__ __forceinline__ void put_units(float (&dst)[ROWS]) const {
         float u[U];
@@ -203,19 +209,19 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
     const int g = lane >> 5;
     const int wm = wave >> 1, wn = wave & 1;
 
-    // Consecutive workgroups go to the 8 XCDs in turn: each XCD takes a run of
-    // tiles, so that it finds their operand panels in its own L2.
-    const int n_tiles = p.tiles_m * p.tiles_n;
-    const int per = (n_tiles + 7) / 8;
-    const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-    if ((int)(blockIdx.x / 8) >= per || tile >= n_tiles) return;
+    // Consecutive workgroups go to the 8 XCDs in turn: each XCD takes an even share
+    // of the work as one run of tiles (of one K range, then the next), so that it
+    // finds their operand panels in its own L2.
+    const int n_tiles = p.tiles_m * p.tiles_n, xcd = blockIdx.x % 8;
+    const int item = (int)((int64_t)p.items * xcd / 8) + (int)(blockIdx.x / 8);
+    if (item >= (int)((int64_t)p.items * (xcd + 1) / 8)) return;
+    const int tile = item % n_tiles, split = item / n_tiles % p.ksplit, batch = item / n_tiles / p.ksplit;
     const int m0 = tile / p.tiles_n * kBM, n0 = tile % p.tiles_n * kBN;
-    const int split = blockIdx.y;
     const int kb = split * p.kchunk, ke = min(p.K, kb + p.kchunk);
     const int nt = (ke - kb + kBK - 1) / kBK;
-    const float* A = p.A + blockIdx.z * p.sa;
-    const float* B = p.B + blockIdx.z * p.sb;
-    float* C = p.C + blockIdx.z * p.sc;
+    const float* A = p.A + batch * p.sa;
+    const float* B = p.B + batch * p.sb;
+    float* C = p.C + batch * p.sc;
 
     StageA sa;
     StageB sb;
@@ -235,7 +241,9 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
     sb.load(sb.raw[1], kb + kBK, ke);
     __syncthreads();
     {
-        const bool ga = sa.store(sa.raw[0], Ua[0], chg_a[0]), gb = sb.store(sb.raw[0], Ub[0], chg_b[0]);
+        const bool ga = sa.classes(sa.raw[0], chg_a[0]), gb = sb.classes(sb.raw[0], chg_b[0]);
+        sa.store(sa.raw[0], Ua[0]);
+        sb.store(sb.raw[0], Ub[0]);
         if ((ga || gb) && lane == 0) tag_s[0] = 0;
     }
     __syncthreads();
@@ -259,6 +267,9 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
                     for (int j = 0; j < 2; ++j) acc[i][j][r] *= fa * fb[j];
                 }
         }
+        const bool ga = sa.classes(sa.raw[BUF ^ 1], chg_a[BUF ^ 1]);
+        const bool gb = sb.classes(sb.raw[BUF ^ 1], chg_b[BUF ^ 1]);
+        if ((ga || gb) && lane == 0) tag_s[BUF ^ 1] = t + 1;
 #pragma unroll
         for (int kk = 0; kk < kBK / 16; ++kk) {
             Half2x8 a[2], b[2];
@@ -278,9 +289,8 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
                     for (int j = 0; j < 2; ++j)
                         acc[i][j] = mfma32x32x16f16(q == 0 ? a[i].l : a[i].h, q == 1 ? b[j].l : b[j].h, acc[i][j]);
         }
-        const bool ga = sa.store(sa.raw[BUF ^ 1], Ua[BUF ^ 1], chg_a[BUF ^ 1]);
-        const bool gb = sb.store(sb.raw[BUF ^ 1], Ub[BUF ^ 1], chg_b[BUF ^ 1]);
-        if ((ga || gb) && lane == 0) tag_s[BUF ^ 1] = t + 1;
+        sa.store(sa.raw[BUF ^ 1], Ua[BUF ^ 1]);
+        sb.store(sb.raw[BUF ^ 1], Ub[BUF ^ 1]);
         __syncthreads();
     };
     using B0 = std::integral_constant<int, 0>;
@@ -350,16 +360,16 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams 
 }
 
 // Whether the kernel takes the problem: fp32; a K-contiguous operand is read 8
-// elements at a time (K % 8, 16-byte rows); 32-bit offsets inside a tile's panel;
+// elements at a time in halves (K % 4, 16-byte rows); 32-bit offsets inside a tile's panel;
 // alpha = 0 must not read operands that may hold infinities.
 static bool split_takes(const GemmArgs& g) {
-    if (g.bf16 || g.alpha == 0.f || g.K % 8 != 0 || g.lda > (1 << 20) || g.ldb > (1 << 20)) return false;
+    if (g.bf16 || g.alpha == 0.f || (g.K % 4 != 0 && !(g.ta && !g.tb)) || g.lda > (1 << 20) || g.ldb > (1 << 20)) return false;
     auto rows16 = [](const void* p, int64_t ld, int64_t stride) {
         return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && stride % 4 == 0;
     };
     if (!g.ta && !rows16(g.A, g.lda, g.batch > 1 ? g.sa : 0)) return false;
     if (g.tb && !rows16(g.B, g.ldb, g.batch > 1 ? g.sb : 0)) return false;
-    return g.batch <= 65535;
+    return true;
 }
 
 int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
@@ -390,6 +400,7 @@ int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
     // partials pass through memory once more.
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * g.batch;
     const int nk = (p.K + kBK - 1) / kBK;
+    if (tiles > (1 << 24)) return 0;  // 32-bit work counts
     double best = 1e30;
     int ks = 1;
     for (int c = 1; c <= 8; ++c) {
@@ -404,15 +415,16 @@ int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
             ks = c;
         }
     }
-    // The vendor library's fp32 kernels (about 142 TFLOP/s, better split for small
-    // problems) where the model says that they are no slower: 1024^3 19 us there
-    // and 35 here, 1536^3 62 and 47, M = 32 rows 9-18 and 25.
-    if (best > 2.0 * g.M * g.N * g.K * g.batch / 142e6 + 8.0) return 0;
+    // The vendor library's fp32 kernels (about 142 TFLOP/s, 118 at ragged sizes, and
+    // better split for small problems) where the model says that they are no
+    // slower: 1024^3 19 us there and 35 here, 1536^3 62 and 47, M = 32 9-18 and 25.
+    const bool whole = g.M % 128 == 0 && g.N % 128 == 0 && g.K % 32 == 0;
+    if (best > 2.0 * g.M * g.N * g.K * g.batch / (whole ? 142e6 : 118e6) + 8.0) return 0;
     p.kchunk = (nk + ks - 1) / ks * kBK;
     p.ksplit = (p.K + p.kchunk - 1) / p.kchunk;
     p.part = (float*)g.ws;
-    const int per = (p.tiles_m * p.tiles_n + 7) / 8;
-    const dim3 grid((unsigned)(8 * per), (unsigned)p.ksplit, (unsigned)g.batch), block(kNT);
+    p.items = (int)(tiles * p.ksplit);
+    const dim3 grid((unsigned)((p.items + 7) / 8 * 8)), block(kNT);
     if (!g.ta && !g.tb) hipLaunchKernelGGL((gemm_split_kernel<true, false>), grid, block, 0, s, p);
     else if (!g.ta) hipLaunchKernelGGL((gemm_split_kernel<true, true>), grid, block, 0, s, p);
     else if (!g.tb) hipLaunchKernelGGL((gemm_split_kernel<false, false>), grid, block, 0, s, p);
