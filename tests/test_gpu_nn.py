@@ -174,6 +174,23 @@ def test_embedding_parity(ia):
     assert np.array_equal(host(dt), onn.embedding_bwd(ids, gout, vocab))
 
 
+@pytest.mark.parametrize("vocab,dim,n", [(3, 4, 1), (50, 4, 255), (50, 4, 257), (97, 20, 700), (64, 252, 65),
+                                         (1000, 1028, 333), (64, 16384, 131077)])
+def test_embedding_bwd_scatter_edges(ia, vocab, dim, n):
+    """Gradient elements around a wave's 256 and a workgroup's 1024, and 2^31 of them and more
+    (64-bit indices): whole-valued gradients, so that the sums are exact in any order; ids outside
+    [0, vocab) add nothing."""
+    print(f"[case] embedding bwd vocab{vocab} dim{dim} n{n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    ids = torch.randint(-1, vocab + 1, (n,), generator=g, device="cuda", dtype=torch.int32)
+    row = (torch.arange(n, device="cuda", dtype=torch.int32) % 5 - 2).float()
+    col = (torch.arange(dim, device="cuda", dtype=torch.int32) % 3 + 1).float()
+    ok = (ids >= 0) & (ids < vocab)
+    per_id = torch.zeros(vocab, device="cuda").index_add_(0, ids[ok].long(), row[ok])
+    got = ia.embedding_bwd(ids, row[:, None] * col[None, :], vocab)
+    assert torch.equal(got, per_id[:, None] * col[None, :])
+
+
 @pytest.mark.parametrize("vocab,dim,n", [(8192, 768, 8192), (1000, 100, 3000), (37, 16384, 50)])
 def test_embedding_bwd_deterministic(ia, vocab, dim, n):
     """The deterministic mode's embedding backward sums each row in token order, as the
