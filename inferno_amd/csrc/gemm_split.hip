@@ -323,7 +323,11 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
             for (int r = 0; r < 16; ++r) {
                 const int ml = 64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
                 const int m = m0 + ml;
-                float v = acc[i][j][r] * chg_a[0][ml] * ub;
+                // the smaller scale first: a row near the largest floats times a column
+                // of tiny ones must not pass through an infinity
+                const float ua = chg_a[0][ml];
+                const bool a_first = fabsf(ua) < fabsf(ub);
+                float v = acc[i][j][r] * (a_first ? ua : ub) * (a_first ? ub : ua);
                 if (bad && __any(!(fabsf(v) < INFINITY))) {
                     if (!(fabsf(v) < INFINITY) && m < p.M && n < p.N) {
                         v = 0.f;

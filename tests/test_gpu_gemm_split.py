@@ -85,6 +85,17 @@ def test_rows_of_any_magnitude(ia, ta, tb):
     assert (e.norm(dim=1) / (r2 / rs.double()[:, None] / cs.double()).norm(dim=1)).max() <= BAR
 
 
+@pytest.mark.parametrize("ea,eb", [(118, -118), (-118, 118), (118, -20), (-100, 20)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+def test_operands_at_the_ends_of_the_range(ia, ta, tb, ea, eb):
+    """One operand near the largest floats, the other near the smallest: their products are ordinary
+    numbers, and nothing on the way to them overflows or underflows."""
+    a, b = make(2048, 1600, 1024, ta, tb, seed=4)
+    a, b = a * 2.0**ea, b * 2.0**eb
+    got = ia.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb))
+    assert got.isfinite().all() and rel(got, ref(a, b, ta, tb)) <= BAR
+
+
 def test_nonfinite(ia):
     """Infinities and NaN reach the results that they reach in fp32, as what they are there."""
     M, N, K = 2048, 1600, 1024
