@@ -316,48 +316,102 @@ __global__ __launch_bounds__(256) void gelu_bwd_kernel(const void* __restrict__ 
 
 // ============================================================================
 // Cross-entropy, mean over rows (cpuops.h:707-749, crossentropylossbackward.h:
-// 45-86).  Forward: one wave per row, online max / sum of exp over the row in
-// 4-element chunks, row loss = lse - x[target] with lse = max + log(sum); the
-// row's lse is kept for the backward.  A target outside [0, vocab) gives a NaN
-// row loss (the reference exits).  A second kernel sums the row losses in a
-// fixed order.  Backward: dlogits = (exp(x - lse) - [v == target]) * up / rows.
+// 45-86).  Forward: online max / sum of exp over the row in batches of 16 (8
+// where the vocabulary is no multiple of 4), row loss = lse - x[target] with lse =
+// max + log(sum); the row's lse is kept for the backward.  A target outside
+// [0, vocab) gives a NaN row loss (the reference exits).  A second kernel sums the
+// row losses in a fixed order.  Backward: dlogits = (exp(x - lse) - [v == target]) *
+// up / rows.
+//
+// Bound by HBM at thousands of rows, by one lane's chain of loads below that: a
+// batch's loads are in flight together and its maximum moves the sum once, and a row
+// is a whole workgroup's (WPR = 4) instead of one wave's where rows are few.  Before (a
+// wave per row, one load a step) and now, us: 64 x 22197 forward 76 -> 16 (the
+// launches' own time), backward 71 -> 10; 700 x 5001 23 -> 16 and 28 -> 10; 2048 x 22196
+// 51 -> 36 and 93 -> 75; 8192 x 8191 89 -> 51 and 121 -> 117; 8192 x 8192, forward and
+// backward in turn, 176 -> 164 (4.9 TB/s).
 // ============================================================================
-template <typename E>
+
+// One more batch into the running maximum m and s = sum of exp(x - m).  While m is
+// -inf there is nothing to be relative to, and exp(-inf) adds the zeros.
+template <int N>
+__device__ __forceinline__ void lse_add(float& m, float& s, const float (&v)[N]) {
+    float mv = v[0];
+#pragma unroll
+    for (int k = 1; k < N; ++k) mv = fmaxf(mv, v[k]);
+    if (mv > m) {
+        s *= expf(m - mv);
+        m = mv;
+    }
+    const float ref = m == -INFINITY ? 0.f : m;
+    float t[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) t[k] = expf(v[k] - ref);
+#pragma unroll
+    for (int w = N / 2; w >= 1; w /= 2)
+#pragma unroll
+        for (int k = 0; k < w; ++k) t[k] += t[k + w];
+    s += t[0];
+}
+// (m, s) and (mo, so) of two parts of a row as those of both.
+__device__ __forceinline__ void lse_merge(float& m, float& s, float mo, float so) {
+    const float mn = fmaxf(m, mo);
+    s = (mn == -INFINITY) ? 0.f : s * expf(m - mn) + so * expf(mo - mn);
+    m = mn;
+}
+
+template <typename E, int WPR>
 __global__ __launch_bounds__(256) void ce_fwd_kernel(CeParams p) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= p.rows) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
+    if (row >= p.rows) return;  // WPR = 4: no workgroup past the last row
+    const int part = wave % WPR;
     const int64_t V = p.vocab;
     const typename E::T* x = (const typename E::T*)p.logits + row * p.ld;
     float m = -INFINITY, s = 0.f;
     if ((V & 3) == 0) {
-        for (int64_t c = 4 * lane; c < V; c += 256) {
-            const f32x4 v = ld4(x + c);
-            const float mv = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-            if (mv > m) {
-                s *= expf(m - mv);
-                m = mv;
+        constexpr int ST = 256 * WPR;
+        int64_t c = 4 * (64 * part + lane);
+        for (; c + 3 * ST < V; c += 4 * ST) {
+            float v[16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 w = ld4(x + c + j * ST);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[4 * j + k] = w[k];
             }
-            s += (expf(v[0] - m) + expf(v[1] - m)) + (expf(v[2] - m) + expf(v[3] - m));
+            lse_add(m, s, v);
+        }
+        for (; c < V; c += ST) {
+            const f32x4 w = ld4(x + c);
+            lse_add(m, s, {w[0], w[1], w[2], w[3]});
         }
     } else {
-        for (int64_t c = lane; c < V; c += 64) {
-            const float v = E::ld(x + c);
-            if (v > m) {
-                s *= expf(m - v);
-                m = v;
-            }
-            s += expf(v - m);
+        constexpr int ST = 64 * WPR;
+        int64_t c = 64 * part + lane;
+        for (; c + 7 * ST < V; c += 8 * ST) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = E::ld(x + c + j * ST);
+            lse_add(m, s, v);
         }
+        for (; c < V; c += ST) lse_add(m, s, {E::ld(x + c)});
     }
-    // combine (m, s) over the wave
 #pragma unroll
     for (int k = 32; k >= 1; k >>= 1) {
-        const float mo = shfl_xor(m, k);
-        const float so = shfl_xor(s, k);
-        const float mn = fmaxf(m, mo);
-        s = (mn == -INFINITY) ? 0.f : s * expf(m - mn) + so * expf(mo - mn);
-        m = mn;
+        const float mo = shfl_xor(m, k), so = shfl_xor(s, k);
+        lse_merge(m, s, mo, so);
+    }
+    if constexpr (WPR > 1) {
+        __shared__ float part_s[2][WPR];
+        if (lane == 0) {
+            part_s[0][part] = m;
+            part_s[1][part] = s;
+        }
+        __syncthreads();
+        if (part) return;
+#pragma unroll
+        for (int w = 1; w < WPR; ++w) lse_merge(m, s, part_s[0][w], part_s[1][w]);
     }
     if (lane == 0) {
         const float lse = m + logf(s);
@@ -368,43 +422,72 @@ __global__ __launch_bounds__(256) void ce_fwd_kernel(CeParams p) {
     }
 }
 
-// loss[0] = sum(row_loss) / rows, one workgroup, fixed summation order.
-__global__ __launch_bounds__(256) void ce_mean_kernel(const float* __restrict__ row_loss, float* __restrict__ out,
-                                                      int64_t rows) {
-    __shared__ float red[256];
+// loss[0] = sum(row_loss) / rows, one workgroup, fixed summation order.  Latency: eight
+// loads in flight a thread (8192 rows: 10.4 us with one, 256 threads).
+__global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__ row_loss, float* __restrict__ out,
+                                                       int64_t rows) {
+    __shared__ float red[16];
     float s = 0.f;
-    for (int64_t r = threadIdx.x; r < rows; r += 256) s += row_loss[r];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w >= 1; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    for (int64_t r = threadIdx.x; r < rows; r += 8 * 1024) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = r + 1024 * j < rows ? row_loss[r + 1024 * j] : 0.f;
+        s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
-    if (threadIdx.x == 0) out[0] = red[0] / (float)rows;
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) t += red[w];
+        out[0] = t / (float)rows;
+    }
 }
 
-template <typename E>
+template <typename E, int WPR>
 __global__ __launch_bounds__(256) void ce_bwd_kernel(CeParams p) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t row = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
     if (row >= p.rows) return;
+    const int part = wave % WPR;
     const int64_t V = p.vocab;
     const typename E::T* x = (const typename E::T*)p.logits + row * p.ld;
     typename E::T* g = (typename E::T*)p.grad + row * p.ldg;
     const float scale = p.upstream[0] / (float)p.rows;
     const float lse = p.lse[row];
     const int t = p.targets[row];
+    // a batch is read before it is written, by the lane that writes it: dlogits may
+    // lie over the logits
     if ((V & 3) == 0) {
-        for (int64_t c = 4 * lane; c < V; c += 256) {
-            const f32x4 v = ld4(x + c);
+        constexpr int ST = 256 * WPR;
+        auto put = [&](int64_t c, f32x4 v) {
             f32x4 r;
 #pragma unroll
             for (int j = 0; j < 4; ++j) r[j] = expf(v[j] - lse) * scale - ((c + j == t) ? scale : 0.f);
             st4(g + c, r);
+        };
+        int64_t c = 4 * (64 * part + lane);
+        for (; c + 3 * ST < V; c += 4 * ST) {
+            f32x4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = ld4(x + c + j * ST);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) put(c + j * ST, v[j]);
         }
+        for (; c < V; c += ST) put(c, ld4(x + c));
     } else {
-        for (int64_t c = lane; c < V; c += 64)
-            E::st(g + c, expf(E::ld(x + c) - lse) * scale - ((c == t) ? scale : 0.f));
+        constexpr int ST = 64 * WPR;
+        auto put = [&](int64_t c, float v) { E::st(g + c, expf(v - lse) * scale - ((c == t) ? scale : 0.f)); };
+        int64_t c = 64 * part + lane;
+        for (; c + 7 * ST < V; c += 8 * ST) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = E::ld(x + c + j * ST);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) put(c + j * ST, v[j]);
+        }
+        for (; c < V; c += ST) put(c, E::ld(x + c));
     }
 }
 
@@ -758,22 +841,30 @@ int launch_gelu_bwd(const void* x, const void* dy, void* dx, int64_t n, int bf16
     return (int)hipGetLastError();
 }
 
+// Four waves a row while a wave each would leave three quarters of the chip's 8192
+// wave slots empty, and the row is long enough to give every lane of them a load
+// (2048 x 8192 forward 18.3 us so, 2049 x 8192 with a wave per row 17.5; a wave a row
+// before 22.4, and 512 x 8192 backward 16.1 -> 10.0).
+static bool ce_row_per_workgroup(const CeParams& p) { return p.rows <= 2048 && p.vocab >= 1024; }
+
 int launch_ce_fwd(const CeParams& p, float* loss, int bf16, hipStream_t s) {
-    const dim3 grid(blocks_for(p.rows, 4));
-    if (bf16)
-        hipLaunchKernelGGL(ce_fwd_kernel<BF16>, grid, dim3(256), 0, s, p);
-    else
-        hipLaunchKernelGGL(ce_fwd_kernel<F32>, grid, dim3(256), 0, s, p);
-    hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(256), 0, s, p.row_loss, loss, p.rows);
+    const bool wg = ce_row_per_workgroup(p);
+    const dim3 grid(blocks_for(p.rows, wg ? 1 : 4)), block(256);
+    if (wg && bf16) hipLaunchKernelGGL((ce_fwd_kernel<BF16, 4>), grid, block, 0, s, p);
+    else if (wg) hipLaunchKernelGGL((ce_fwd_kernel<F32, 4>), grid, block, 0, s, p);
+    else if (bf16) hipLaunchKernelGGL((ce_fwd_kernel<BF16, 1>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((ce_fwd_kernel<F32, 1>), grid, block, 0, s, p);
+    hipLaunchKernelGGL(ce_mean_kernel, dim3(1), dim3(1024), 0, s, p.row_loss, loss, p.rows);
     return (int)hipGetLastError();
 }
 
 int launch_ce_bwd(const CeParams& p, int bf16, hipStream_t s) {
-    const dim3 grid(blocks_for(p.rows, 4));
-    if (bf16)
-        hipLaunchKernelGGL(ce_bwd_kernel<BF16>, grid, dim3(256), 0, s, p);
-    else
-        hipLaunchKernelGGL(ce_bwd_kernel<F32>, grid, dim3(256), 0, s, p);
+    const bool wg = ce_row_per_workgroup(p);
+    const dim3 grid(blocks_for(p.rows, wg ? 1 : 4)), block(256);
+    if (wg && bf16) hipLaunchKernelGGL((ce_bwd_kernel<BF16, 4>), grid, block, 0, s, p);
+    else if (wg) hipLaunchKernelGGL((ce_bwd_kernel<F32, 4>), grid, block, 0, s, p);
+    else if (bf16) hipLaunchKernelGGL((ce_bwd_kernel<BF16, 1>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((ce_bwd_kernel<F32, 1>), grid, block, 0, s, p);
     return (int)hipGetLastError();
 }
 

@@ -9,6 +9,8 @@ arithmetic is exact (embedding gather, integer-valued scatter and sums).
 Shapes: the GPT-2-small step (rows = 8 x 1024 tokens, C = 768, 4C = 3072,
 vocab 8192) and ragged edges.
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -152,6 +154,31 @@ def test_cross_entropy_parity(ia, rows, vocab):
     up = dev(np.array([0.5], np.float32))
     g = ia.cross_entropy_bwd(dev(x), dev(t), lse, up)
     assert oracle.rel_err(host(g), onn.cross_entropy_bwd(x, t, 0.5)) < TOL
+
+
+# a wave or a workgroup per row (2048 rows; 1024 columns), whole and partial batches of 16-byte
+# and single loads, fewer columns than lanes; hidden (-inf) columns where a lane's first ones lie
+@pytest.mark.parametrize("rows", [1, 2048, 2049])
+@pytest.mark.parametrize("vocab", [1, 64, 1020, 1024, 1025, 4096, 4100, 4107])
+@pytest.mark.parametrize("hide", [False, True])
+def test_cross_entropy_row_splits(ia, rows, vocab, hide):
+    print(f"[case] cross_entropy rows{rows} vocab{vocab} hide{hide}", flush=True)
+    x = torch.from_numpy(rnd(19, (rows, vocab), 2.0)).cuda()
+    t = (torch.arange(rows, device="cuda") * 7919 + 13) % vocab
+    if hide:
+        x[:, : vocab // 2] = -math.inf
+        t = vocab - 1 - t % (vocab - vocab // 2)
+    loss, lse = ia.cross_entropy_fwd(x, t.int())
+    ref = torch.logsumexp(x.double(), 1)
+    # 4107 terms summed in fp32, in parts of 16 at most 65 long: 2^-24 a step, and expf's own 2^-23
+    assert ((lse.double() - ref).abs() <= 4e-6 * ref.abs().clamp(min=1)).all()
+    want = (ref - x.double().gather(1, t[:, None])[:, 0]).mean()
+    assert abs(loss.double().item() - want.item()) <= 4e-6 * max(1.0, abs(want.item()))
+    g = ia.cross_entropy_bwd(x, t.int(), lse, torch.full((1,), 0.5, device="cuda"))
+    gw = torch.softmax(x.double(), 1)
+    gw.scatter_add_(1, t[:, None], torch.full((rows, 1), -1.0, dtype=torch.float64, device="cuda"))
+    gw *= 0.5 / rows
+    assert (g.double() - gw).abs().max() <= 1e-5 * max(gw.abs().max().item(), 0.5 / rows)
 
 
 def test_cross_entropy_bad_target_is_nan(ia):
