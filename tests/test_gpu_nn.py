@@ -326,3 +326,15 @@ def test_binary_bcast(ia, n, nb):
     assert np.array_equal(got, want)
     got = host(ia.binary_bcast(1, dev(a), dev(b)))
     assert np.array_equal(got, (a.reshape(-1, nb) * b).reshape(-1))
+
+
+# ----------------------------------------------------------------------- fill
+# whole 16-byte units and what is left of one, destinations off 16 bytes, more units than threads
+@pytest.mark.parametrize("dtype,bits", [(torch.int32, 0x12345678), (torch.int16, 0x7BCD), (torch.uint8, 0xA5)])
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 4099, 1 << 20])
+@pytest.mark.parametrize("off", [0, 1, 4])
+def test_fill(ia, dtype, bits, n, off):
+    pad = torch.zeros(n + off + 32, dtype=dtype, device="cuda")
+    st = ia.lib().inf_fill(pad[off:].data_ptr(), n, pad.element_size(), bits, torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    assert (pad[off:off + n] == bits).all() and (pad[:off] == 0).all() and (pad[off + n:] == 0).all()
