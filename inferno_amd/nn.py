@@ -31,8 +31,8 @@ def gemm(a, b, trans_a=False, trans_b=False, bias=None, alpha=1.0, beta=0.0, out
     M = a.shape[1] if trans_a else a.shape[0]
     K = a.shape[0] if trans_a else a.shape[1]
     N = b.shape[0] if trans_b else b.shape[1]
-    if out is None:
-        out = torch.zeros((M, N), dtype=a.dtype, device=a.device)
+    if out is None:  # beta = 0 writes every element and reads none
+        out = (torch.empty if beta == 0 else torch.zeros)((M, N), dtype=a.dtype, device=a.device)
     if workspace is None:
         workspace = _ws(nn_workspace_bytes(OP_GEMM), a.device)
     st = lib().inf_gemm(int(trans_a), int(trans_b), M, N, K, float(alpha), a.data_ptr(), _ld(a), 0, b.data_ptr(),
