@@ -1,36 +1,37 @@
 // attn_bwd.hip -- fused causal attention backward for gfx950 (recompute).
 //
 // Kernel 1 (bwd_pre): delta[i] = sum_d dO[i,d] * O[i,d] per query row (the
-// row dot that SoftmaxBackward computes as sum_j dP_ij P_ij), zeroes the
-// fp32 dQ accumulator and, for fp32, leaves the largest |q| and |dO| of its
-// rows.  (The bf16 main kernel at D <= 64 forms delta itself, and then this
-// pass only zeroes.)
+// row dot that SoftmaxBackward computes as sum_j dP_ij P_ij), and zeroes the
+// fp32 dQ accumulator.  (The bf16 main kernel at D <= 64 forms delta itself, and
+// then this pass only zeroes.)
 //
-// Kernel 2 (bwd_main, fp32): its products run on the fp16 matrix cores, every
-// operand split into two fp16 parts (common.h), three MFMAs per product step.
+// Kernel 2 (bwd_main, fp32): its products run on the bf16 matrix cores, every
+// operand split into three bf16 parts (common.h), six MFMAs per product step.
 // One workgroup = 8 waves = 4 pairs, each pair with 64 keys (or 32) of one
-// (b, h).  In a pair, wave 0 (role 0) holds the keys' K operand and dV^T
-// accumulators in VGPRs, wave 1 (role 1) their V operand and dK^T accumulators,
-// 64 + 64 registers each at D = 64 and 128, so two waves fit a SIMD, one of each
-// role.  dK and dV are written exactly once, with no atomics.  The workgroup
-// walks query tiles of 32 rows, split into LDS once for all waves; per tile,
-// in three phases with a barrier after each:
+// (b, h).  In a pair, wave 0 (role 0) has the keys' K operand and dV^T
+// accumulators, wave 1 (role 1) their V operand and dK^T accumulators, so two
+// waves fit a SIMD, one of each role.  dK and dV are written exactly once, with no
+// atomics.  The workgroup walks query tiles of 32 rows, split into LDS once for all
+// waves; per tile, in three phases with a barrier after each:
 //
 //   A  role 0: S = Q K^T, P = exp2(S c - lse log2e) (masked entries exactly 0),
 //      P handed to role 1 through LDS;   role 1: dP = dO V^T
-//   B  role 0: dV^T += dO^T P;   role 1: dS = P (dP - delta), split, to LDS
+//   B  role 0: dV^T += dO^T P;   role 1: dS = P (dP - delta), its parts to LDS,
+//      dK^T += Q^T dS
 //   C  role 0: dQ tile += dS K over the workgroup's keys, fp32 atomics into the
-//      global accumulator;   role 1: dK^T += Q^T dS;   both: the next tile
+//      global accumulator;   both: the next tile into LDS
 //
 // Keys lie on the lane axis in S, dP, dV^T and dK^T, so P and dS are operands
-// straight from the accumulators; the transposed operands (dO^T, Q^T, dS) are
-// transposed LDS reads, and K^T for dQ is staged transposed once.  S is formed
-// in the forward's order, to the same bits, so P is consistent with the LSE.
-// Bound by the phases' latency: a tile's MFMAs take 3840 of its 8100 (D = 128)
-// or 9100 (D = 64) cycles per SIMD, and at config 4 the fp16 MFMAs run at a
-// 2.0 GHz shader clock.  The backward call against the fp32-MFMA kernel that this
-// one replaced (us): config 2 308 -> 163, config 4 5980 -> 2170, B8 H12 T1024 D32
-// 178 -> 128, B1 H12 T333 D64 34 -> 27.
+// straight from the accumulators; dO^T, Q^T, dS and K^T are transposed LDS reads.
+// The K rows' h and m parts lie in LDS, their l parts in registers, V in registers
+// as fp32 (its parts don't fit; split again for each tile).  S is formed in the
+// forward's order, to the same bits, so P is consistent with the LSE.
+// Bound by the MFMAs: 55% busy at D = 128 (7680 of 14000 cycles per tile and SIMD) at a
+// clock that the load holds at 1.9 GHz, which is 1.1 PFLOP/s of them where a large
+// library product reaches 1.25; at D = 64 (42% busy) also by the phases' latency.
+// Against the fp32 MFMAs, the backward call (us): config 2 308 -> 238, config 4 5980 ->
+// 3700.  Two scaled fp16 parts and three MFMAs took 163 and 2170, but blocks shared
+// a scale: a block of zero keys gave infinities, small rows lost bits.
 //
 // bf16 inputs use the bf16-MFMA main kernel (attn_bwd_bf16.hip) between the
 // same pre kernel and a final bwd_cvt that turns the fp32 dQ accumulator into
@@ -85,35 +86,18 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(BwdParams p) {
     const int tid = threadIdx.x;
     const int c = tid % TPR;
     const int64_t rows = (int64_t)p.B * p.H * p.Tq;
-    // fp32: p.n_amax workgroups per head; bf16: flat over the rows
-    int64_t row, b, h, i;
-    bool in;
-    if constexpr (sizeof(E) == 4) {
-        const unsigned bh = blockIdx.x / (unsigned)p.n_amax;
-        i = (int64_t)(blockIdx.x % (unsigned)p.n_amax) * RPB + tid / TPR;
-        b = bh / (unsigned)p.H;
-        h = bh % (unsigned)p.H;
-        in = i < p.Tq;
-        row = (int64_t)bh * p.Tq + i;
-    } else {
-        row = (int64_t)blockIdx.x * RPB + tid / TPR;
-        in = row < rows;
-        if (in) bwd_row_split(p, rows, row, b, h, i);
-    }
-    float s = 0.f, aq = 0.f, ad = 0.f;
+    const int64_t row = (int64_t)blockIdx.x * RPB + tid / TPR;
+    const bool in = row < rows;
+    float s = 0.f;
     if (in) {
+        int64_t b, h, i;
+        bwd_row_split(p, rows, row, b, h, i);
         if (p.pre_delta) {
             const E* po = (const E*)p.o + b * p.so.b + h * p.so.h + i * p.so.t + VEC * c;
             const E* pd = (const E*)p.dout + b * p.sdo.b + h * p.sdo.h + i * p.sdo.t + VEC * c;
             if constexpr (sizeof(E) == 4) {
                 const f32x4 o4 = ld4(po), d4 = ld4(pd);
                 s = o4[0] * d4[0] + o4[1] * d4[1] + o4[2] * d4[2] + o4[3] * d4[3];
-                const f32x4 q4 = ld4((const E*)p.q + b * p.sq.b + h * p.sq.h + i * p.sq.t + VEC * c);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    aq = fmaxf(aq, finite_abs(q4[k]));
-                    ad = fmaxf(ad, finite_abs(d4[k]));
-                }
             } else {
                 const u16x8 o8 = *reinterpret_cast<const u16x8*>(po);
                 const u16x8 d8 = *reinterpret_cast<const u16x8*>(pd);
@@ -131,19 +115,6 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(BwdParams p) {
     if (p.pre_delta) {
         s = group_sum<TPR>(s);
         if (in && c == 0) p.delta[row] = s;
-    }
-    if constexpr (sizeof(E) == 4) {
-        __shared__ float red[2][4];
-        aq = wave_max(aq);
-        ad = wave_max(ad);
-        if ((tid & 63) == 0) {
-            red[0][tid >> 6] = aq;
-            red[1][tid >> 6] = ad;
-        }
-        __syncthreads();
-        if (tid < 2)
-            p.amax[(int64_t)blockIdx.x * 2 + tid] =
-                fmaxf(fmaxf(red[tid][0], red[tid][1]), fmaxf(red[tid][2], red[tid][3]));
     }
     if (blockIdx.x == 0)
         for (int i = tid; i < p.n_split * p.B * p.H; i += 256) p.counters[i] = 0u;
@@ -166,22 +137,49 @@ __global__ __launch_bounds__(256) void bwd_zero_kernel(BwdParams p) {
 template <int D, int KP>
 struct BwdTile {
     static constexpr int BK = 4 * KP;              // keys per workgroup
-    // Q / dO row stride in LDS (fp16 elements): row reads want an odd number of
-    // 16-byte units, transposed reads the 32-byte windows of 4 rows in disjoint banks
-    static constexpr int QS = D == 128 ? 152 : D == 64 ? 72 : 56;
-    static constexpr int SS = 36;                  // dS row stride (queries of one key, fp16 elements)
+    // Rows in LDS (bf16 elements), without padding: the 16-byte units of a row are
+    // permuted by its number, so that row reads (one unit of 8 rows at a time) and
+    // transposed reads (64 bytes of 4 rows) both touch every bank once.
+    static constexpr int QS = D;
+    static constexpr int SS = 36;                  // dS row stride (queries of one key, bf16 elements)
+    static __device__ __forceinline__ int swz(int row) {
+        return D == 128 ? 4 * (row & 3) ^ ((row >> 2) & 3) : D == 64 ? 4 * ((row >> 1) & 1) ^ ((row >> 2) & 3) : (row >> 2) & 3;
+    }
+    // Byte offset of the 8 columns from 8 * unit of a row.
+    static __device__ __forceinline__ uint32_t at(int row, int unit) { return (uint32_t)(row * QS * 2 + 16 * (unit ^ swz(row))); }
+    // A lane's offset for the row operands of 32 rows (row lane % 32, columns 8 (lane /
+    // 32) ..) and for the transposed ones (rows 4 (lane / 32) + {0..3}).
+    static __device__ __forceinline__ uint32_t row_lane(int lane) { return at(lane & 31, lane >> 5); }
+    static __device__ __forceinline__ uint32_t tr_lane(int lane) {
+        return at(4 * (lane >> 5) + ((lane & 15) >> 2), 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) + 8 * (lane & 1);
+    }
+    // From a lane's offset (in LDS at `lds`, the tile's start a multiple of 256) one
+    // part of the operand: the row operand of MFMA step kk (columns 16 kk ..), and the
+    // transposed one with columns 32 db + lane % 32 as its rows and rows row0 + 4 (lane
+    // / 32) + {0..3} and + 8 (row0 a multiple of 16) as reduction index.  The unit's
+    // permutation makes a step of columns (and of 8 rows) an exclusive or.
+    static __device__ __forceinline__ bf16x8 row_part(const char* lds, uint32_t off, int kk, int bytes) {
+        return *reinterpret_cast<const bf16x8*>(lds + (off ^ (uint32_t)(32 * kk)) + bytes);
+    }
+    static __device__ __forceinline__ bf16x8 tr_part(const char* lds, uint32_t off, int row0, int db, int bytes) {
+        const char* lo = lds + (off ^ (uint32_t)(64 * db)) + row0 * QS * 2 + bytes;
+        const char* hi = lds + (off ^ (uint32_t)(64 * db ^ 32)) + (row0 + 8) * QS * 2 + bytes;
+        return __builtin_shufflevector(ds_read_tr16(reinterpret_cast<const __bf16*>(lo)),
+                                       ds_read_tr16(reinterpret_cast<const __bf16*>(hi)), 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+    // All three parts, `part` bytes apart.
+    static __device__ __forceinline__ Bf3x8 row_frag(const char* lds, uint32_t off, int kk, int part) {
+        return Bf3x8{row_part(lds, off, kk, 0), row_part(lds, off, kk, part), row_part(lds, off, kk, 2 * part)};
+    }
+    static __device__ __forceinline__ Bf3x8 tr_frag(const char* lds, uint32_t off, int row0, int db, int part) {
+        return Bf3x8{tr_part(lds, off, row0, db, 0), tr_part(lds, off, row0, db, part), tr_part(lds, off, row0, db, 2 * part)};
+    }
+    static __device__ __forceinline__ void put(char* at, const Bf3x8& y, int part) {
+        *reinterpret_cast<bf16x8*>(at) = y.h;
+        *reinterpret_cast<bf16x8*>(at + part) = y.m;
+        *reinterpret_cast<bf16x8*>(at + 2 * part) = y.l;
+    }
 };
-constexpr float kBwdPBits = 14.f, kBwdPInv = 1.f / 16384.f;  // P enters its products as 2^14 P
-
-// A operand (32 rows of 16 values) read transposed from `t`, rows = the
-// reduction index r0 + {0..3} and + 8 + {0..3} per lane half (r0 includes 4 g),
-// columns c0 + lane % 32.
-template <typename Addr>
-__device__ __forceinline__ f16x8 tr_frag(Addr addr) {
-    const f16x4 lo = ds_read_tr16_f16(addr(0));
-    const f16x4 hi = ds_read_tr16_f16(addr(8));
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
 
 // SHORT: the launch has short rows (p.n_short > 0); without them the kernel
 // carries neither the prologue nor the low part of delta.
@@ -198,21 +196,20 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     constexpr int C8 = D / 8;              // 8-element chunks per row
     constexpr int NCH = BQ * C8;           // chunks of a Q or dO tile, staged by 256 threads
     constexpr int CPT = (NCH + 255) / 256;
+    constexpr int PART = BQ * QS * 2;      // bytes of one part of a Q or dO tile
+    constexpr int KPART = BK * QS * 2;     // ... and of the K rows
     constexpr int XB = 32 * SS * 2;        // bytes of one dS part of a 32-key block
+    constexpr int XPAIR = NKB * 3 * XB;
     constexpr int DQP = NDB;               // dQ: pairs of keys per wave (4 / NDB waves share a head-dim block)
-    constexpr int KU = BK / 8 * D / NT;    // K^T units per thread
+    static_assert(DQP * 2 == NKK, "as many dQ steps as S steps");
 
-    __shared__ __attribute__((aligned(16))) _Float16 Qs[2][2][BQ][QS];  // [buffer][part]
-    __shared__ __attribute__((aligned(16))) _Float16 dOs[2][BQ][QS];    // [part]
-    __shared__ f16x8 Kt[2][BK / 8][D];  // [part][8 keys][head dim]: K^T in the dQ product's operand order
-    __shared__ __attribute__((aligned(16))) char Xs[4][NKB * 2 * XB];   // P, then dS, of each pair
+    // LDS: the h and m parts of the workgroup's K rows, the Q tile and the dO tile
+    // (three parts each), and for each pair P (fp32), then dS (three parts).
+    constexpr int Q_OFF = 2 * KPART, DO_OFF = Q_OFF + 3 * PART, X_OFF = DO_OFF + 3 * PART;
+    __shared__ __attribute__((aligned(256))) char lds[X_OFF + 4 * XPAIR];
     __shared__ __attribute__((aligned(16))) float lse_s[BQ];
     __shared__ __attribute__((aligned(16))) float dl_s[BQ];
-    __shared__ __attribute__((aligned(16))) float dlo_s[BQ];
-    __shared__ float dinv_s[SHORT ? BQ : 1];  // units of the dO rows
-    __shared__ int dqcls_s[4];     // sum of the classes of a pair's dS, V and K
-    __shared__ int kcls_s[4];
-    __shared__ float red_s[2][8];
+    __shared__ __attribute__((aligned(16))) float dlo_s[SHORT ? BQ : 4];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -241,14 +238,14 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     const int q_begin = wk.q_begin;
     const int q_end = wk.q_end;
 
-    // Role 1's threads stage the Q tiles, role 0's the dO tiles, with the rows'
+    // Role 1's threads stage the Q tiles, role 0's the dO tiles, wave 0 the rows'
     // LSE and delta.  Rows at or past `lim` read as zeros.
     const int ts = tid & 255;
     const float* Y = role ? Q : dO;
     const int64_t yt = role ? p.sq.t : p.sdo.t;
     const uint32_t y_voff = (uint32_t)(((int64_t)(ts / C8) * yt + 8 * (ts % C8)) * 4);
     f32x4 yr[CPT][2];
-    float r_lse[CPT], r_dl[CPT], r_dlo[CPT];
+    float r_row = 0.f, r_dlo = 0.f;  // thread ts < 32: row ts's LSE (and delta's low part), 32 + r: row r's delta
     auto gload = [&](int q0, int lim) {
         const int rows = min(lim - q0, BQ);
         const auto ry = row_rsrc(Y, yt, q0, rows, D);
@@ -259,138 +256,153 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
             yr[i][1] = buffer_ld4(ry, y_voff + 16, so);
         }
         if (role == 0) {
-            const int n_sh = SHORT && kblk == 0 ? max(0, min(p.n_short - q0, rows)) : 0;
-            const auto rl = row_rsrc(LSE, 1, q0, rows, 1), rd = row_rsrc(DL, 1, q0, rows, 1), ro = row_rsrc(DLO, 1, q0, n_sh, 1);
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) {
-                const uint32_t off = (uint32_t)((ts + 256 * i) / C8) * 4;
-                r_lse[i] = buffer_ld1(rl, off, 0);
-                r_dl[i] = buffer_ld1(rd, off, 0);
-                r_dlo[i] = SHORT ? buffer_ld1(ro, off, 0) : 0.f;
+            const auto rl = row_rsrc(LSE, 1, q0, rows, 1), rd = row_rsrc(DL, 1, q0, rows, 1);
+            if (wave == 0) {
+                const uint32_t off = (uint32_t)l32 * 4;
+                r_row = g == 0 ? buffer_ld1(rl, off, 0) : buffer_ld1(rd, off, 0);
+                if constexpr (SHORT) {
+                    const int n_sh = kblk == 0 ? max(0, min(p.n_short - q0, rows)) : 0;
+                    r_dlo = buffer_ld1(row_rsrc(DLO, 1, q0, n_sh, 1), off, 0);
+                }
             }
         }
     };
-    // Everything that the workgroup starts from is loaded at once: its operand
-    // rows, K^T, the first Q / dO tile and the maxima of the head's Q and dO rows.
-    // The wave's operand, K or V rows of its pair's keys: MFMA step kk takes
-    // row key, columns 16 kk + 8 g .. + 7.
-    Half2x8 xf[NKB][NKK];
-    int xcls;  // its scale class
-    // K^T for the dQ product: unit f holds column f % D of the 8 keys that an
-    // operand takes together (16 m + 4 g' + {0..3} and + 8 for key group f / D =
-    // 2 m + g'), scaled as its pair's K rows are.
-    f32x4 kt[DQD ? 1 : KU][2];
-    auto kt_key = [](int f) { return 16 * (f / D >> 1) + 4 * (f / D & 1); };
+    // Everything that the workgroup starts from is loaded at once: its operand rows
+    // (K or V rows of the pair's keys: MFMA step kk takes row key, columns 16 kk + 8
+    // g .. + 7), the K^T operand of dQ and the first Q / dO tile.
+    //   role 1: xr is the V rows in fp32, two thirds of the registers of their parts,
+    //     split again for each tile;
+    //   role 0: K's h and m parts go to LDS, where row reads serve S and transposed
+    //     reads dQ; xr[..][0] is the l part in S's layout and xr[..][1], in entry
+    //     step, the one in dQ's.
+    f32x4 xr[NKB][NKK][2];
     {
         const float* X = role ? (const float*)p.v + b * p.sv.b + h * p.sv.h : (const float*)p.k + b * p.sk.b + h * p.sk.h;
         const int64_t xt = role ? p.sv.t : p.sk.t;
-        f32x4 raw[NKB][NKK][2];
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) {
             const int key = k0p + kb * 32 + l32;
 #pragma unroll
             for (int kk = 0; kk < NKK; ++kk) {
-                raw[kb][kk][0] = raw[kb][kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                xr[kb][kk][0] = xr[kb][kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
                 if (key < p.Tk) {
-                    raw[kb][kk][0] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g);
-                    raw[kb][kk][1] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g + 4);
+                    xr[kb][kk][0] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g);
+                    xr[kb][kk][1] = ld4(X + (int64_t)key * xt + 16 * kk + 8 * g + 4);
                 }
-            }
-        }
-        if constexpr (!DQD) {
-            const float* K = (const float*)p.k + b * p.sk.b + h * p.sk.h;
-            const auto rk = row_rsrc(K, p.sk.t, k0, min(p.Tk - k0, BK), D);
-#pragma unroll
-            for (int i = 0; i < KU; ++i) {
-                const int f = tid + NT * i;
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    kt[i][e >> 2][e & 3] = buffer_ld1(rk, (uint32_t)(((int64_t)kt_key(f) * p.sk.t + f % D) * 4),
-                                                      (uint32_t)((int64_t)((e & 3) + 8 * (e >> 2)) * p.sk.t * 4));
             }
         }
         gload(q_begin, p.Tq);
-        const float* am = p.amax + (int64_t)bh * p.n_amax * 2;
-        float aq = 0.f, ad = 0.f;
-        for (int i = tid; i < p.n_amax; i += NT) {
-            aq = fmaxf(aq, am[2 * i]);
-            ad = fmaxf(ad, am[2 * i + 1]);
+        if (role == 0) {
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                for (int kk = 0; kk < NKK; ++kk) {
+                    const Bf3x8 k = split3<true>(xr[kb][kk][0], xr[kb][kk][1]);
+                    char* at = lds + T::at(pr * KP + 32 * kb + l32, 2 * kk + g);
+                    *reinterpret_cast<bf16x8*>(at) = k.h;
+                    *reinterpret_cast<bf16x8*>(at + KPART) = k.m;
+                    xr[kb][kk][0] = __builtin_bit_cast(f32x4, k.l);
+                }
+            if constexpr (!DQD) {
+#pragma unroll
+                for (int st = 0; st < NKB * NKK; ++st) {  // step st: pair pr / NDB * DQP + st / (2 NKB), ...
+                    const int pp = pr / NDB * DQP + st / (2 * NKB);
+                    const int row0 = k0 + pp * KP;
+                    const auto rk = row_rsrc(X, xt, row0, min(p.Tk - row0, KP), D);
+                    f32x4 kt[2];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)  // ... keys 16 (st % (2 NKB)) + 4 g + {0..3} and + 8, column 32 (pr % NDB) + l32
+                        kt[e >> 2][e & 3] =
+                            buffer_ld1(rk, (uint32_t)(((int64_t)(16 * (st % (2 * NKB)) + 4 * g) * xt + 32 * (pr % NDB) + l32) * 4),
+                                       (uint32_t)((int64_t)((e & 3) + 8 * (e >> 2)) * xt * 4));
+                    xr[st / NKK][st % NKK][1] = __builtin_bit_cast(f32x4, split3<true>(kt[0], kt[1]).l);
+                }
+            }
         }
-        aq = wave_max(aq);
-        ad = wave_max(ad);
-        if (lane == 0) {
-            red_s[0][wave] = aq;
-            red_s[1][wave] = ad;
-        }
-        float amax = 0.f;
+    }
+    // This lane's LDS offsets: row operands of the tile whose scores the wave forms
+    // and of its pair's keys, transposed operands of the tile that it sums into dV or
+    // dK and of K, dS as the dQ product reads it.  Each passes an empty asm per tile:
+    // what is derived from them is formed again instead of being held (and spilled).
+    uint32_t row_off = (role ? DO_OFF : Q_OFF) + T::row_lane(lane), krow_off = pr * KP * QS * 2 + T::row_lane(lane);
+    uint32_t tr_off = (role ? Q_OFF : DO_OFF) + T::tr_lane(lane), ktr_off = pr / NDB * DQP * KP * QS * 2 + T::tr_lane(lane);
+    uint32_t ds_off = X_OFF + pr / NDB * DQP * XPAIR + (4 * g + ((lane & 15) >> 2)) * SS * 2 + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+    auto fresh_off = [&]() { asm volatile("" : "+v"(row_off), "+v"(krow_off), "+v"(tr_off), "+v"(ktr_off), "+v"(ds_off)); };
+    const uint32_t st_off = (role ? Q_OFF : DO_OFF) + T::at(ts / C8, ts % C8);
+    // The split parts of role 1's rows don't change from tile to tile: an empty asm
+    // per tile keeps them from being formed once and held (or spilled).
+    auto fresh_xr = [&]() {
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) amax = absmax8_finite(amax, raw[kb][kk][0], raw[kb][kk][1]);
-        xcls = __builtin_amdgcn_readfirstlane(scale_class(wave_max(amax)));
-        const float xs = class_scale(xcls);
+            for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(xr[kb][kk][0]), "+v"(xr[kb][kk][1]));
+    };
+    // The S (role 0) or dP (role 1) chains of the staged tile and the pair's keys;
+    // SWAP: queries as the MFMA's rows (the main loop), else keys (the short rows),
+    // in the same order, to the same bits.
+    auto scores = [&](f32x16 (&s)[NKB], auto swap_c) {
+        constexpr bool SWAP = decltype(swap_c)::value;
+        fresh_xr();
+        fresh_off();
+        Split3Sum sum;
+        auto add = [&](const Bf3x8& y, const Bf3x8& x) {
+            if constexpr (SWAP)
+                mfma_split3<true>(y, x, sum);
+            else
+                mfma_split3<false>(x, y, sum);
+        };
+        // a step's LDS operands are read while the step before runs
+        constexpr int N = NKB * NKK;
+        if (role == 0) {
+            Bf3x8 y[2];
+            y[0] = T::row_frag(lds, row_off, 0, PART);
+            bf16x8 k[2][2];
+            auto k_read = [&](int st) {
+                k[st & 1][0] = T::row_part(lds, krow_off, st % NKK, 32 * (st / NKK) * QS * 2);
+                k[st & 1][1] = T::row_part(lds, krow_off, st % NKK, 32 * (st / NKK) * QS * 2 + KPART);
+            };
+            if constexpr (NKB == 1) k_read(0);
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
+            for (int st = 0; st < N; ++st) {
+                if constexpr (NKB > 1) k_read(st);  // (the registers of another step's K don't fit)
+                if (st + 1 < N) {
+                    y[(st + 1) & 1] = T::row_frag(lds, row_off, (st + 1) % NKK, PART);
+                    if constexpr (NKB == 1) k_read(st + 1);
+                }
+                if (st % NKK == 0) sum.hi = sum.lo = f32x16{};
+                __builtin_amdgcn_sched_barrier(0);
+                add(y[st & 1], Bf3x8{k[st & 1][0], k[st & 1][1], __builtin_bit_cast(bf16x8, xr[st / NKK][st % NKK][0])});
+                __builtin_amdgcn_sched_barrier(0);
+                if (st % NKK == NKK - 1) s[st / NKK] = sum.sum();
+            }
+        } else {
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) xf[kb][kk] = split2(raw[kb][kk][0], raw[kb][kk][1], xs);
-        if (role == 0 && lane == 0) kcls_s[pr] = xcls;
-    }
-    int qcls, docls;  // scale classes of the head's Q and dO rows, from bwd_pre's maxima
-    __syncthreads();
-    {
-        float aq = 0.f, ad = 0.f;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            aq = fmaxf(aq, red_s[0][w]);
-            ad = fmaxf(ad, red_s[1][w]);
+            for (int st = 0; st < N; ++st) {
+                const Bf3x8 y = T::row_frag(lds, row_off, st % NKK, PART);  // (while the rows are split)
+                if (st % NKK == 0) sum.hi = sum.lo = f32x16{};
+                __builtin_amdgcn_sched_barrier(0);
+                add(y, split3(xr[st / NKK][st % NKK][0], xr[st / NKK][st % NKK][1]));
+                __builtin_amdgcn_sched_barrier(0);
+                if (st % NKK == NKK - 1) s[st / NKK] = sum.sum();
+            }
         }
-        qcls = __builtin_amdgcn_readfirstlane(scale_class(aq));
-        docls = __builtin_amdgcn_readfirstlane(scale_class(ad));
-    }
-    if constexpr (!DQD) {
-#pragma unroll
-        for (int i = 0; i < KU; ++i) {
-            const int f = tid + NT * i;
-            const Half2x8 k = split2(kt[i][0], kt[i][1], class_scale(kcls_s[kt_key(f) / KP]));
-            Kt[0][f / D][f % D] = k.h;
-            Kt[1][f / D][f % D] = k.l;
-        }
-    }
-    const float qinv = class_inv(qcls), doinv = class_inv(docls);
-    const float xinv = class_inv(xcls);
-    const float ytile = class_scale(role ? qcls : docls);  // scale of the rows this wave stages
-    const float cs = p.c * xinv * qinv;                     // role 0: scores in exp2 units are S cs
-    const float dsu = kBwdPInv * xinv * doinv;              // role 1: dS = ds dsu, ds = (2^14 P) (dP' - delta')
-    const float xscale = class_scale(xcls);                 // role 1
+    };
 
-    auto sstore = [&](int buf) {
-        int ts = tid & 255;
-        if constexpr (D == 64 && KP == 64) asm volatile("" : "+v"(ts));
-        _Float16* dst = role ? &Qs[buf][0][0][0] : &dOs[0][0][0];
+    auto sstore = [&]() {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int f = ts + 256 * i;
-            float ys = ytile;
-            int rc = docls;
-            if (role == 0) {  // a dO row by its own class: rows may differ by many binades
-                rc = scale_class(group_max<C8>(absmax8_finite(0.f, yr[i][0], yr[i][1])));
-                ys = class_scale(rc);
-            }
-            const Half2x8 y = split2(yr[i][0], yr[i][1], ys);
+            const Bf3x8 y = split3<true>(yr[i][0], yr[i][1]);
             if (NCH % 256 == 0 || f < NCH) {
-                *reinterpret_cast<f16x8*>(dst + (f / C8) * QS + 8 * (f % C8)) = y.h;
-                *reinterpret_cast<f16x8*>(dst + (BQ + f / C8) * QS + 8 * (f % C8)) = y.l;
-                if (role == 0 && f % C8 == 0) {
-                    // P carries the row's unit over the head's, so that dV and dS sum
-                    // rows in one unit: 2^14 P 2^(8 (rc - docls)) = exp2(S c - lse_s)
-                    const int r = f / C8;
-                    lse_s[r] = fmaf(r_lse[i], kLog2e, (float)(8 * (docls - rc)) - kBwdPBits);
-                    dl_s[r] = r_dl[i] * ys;
-                    if constexpr (SHORT) {
-                        dlo_s[r] = r_dlo[i] * ys;
-                        dinv_s[r] = class_inv(rc);
-                    }
-                }
+                T::put(lds + st_off + 256 / C8 * i * QS * 2, y, PART);  // (rows 16 or more apart: the same units)
+            }
+        }
+        if (wave == 0) {
+            if (g == 0) {
+                lse_s[l32] = r_row * kLog2e;
+                if constexpr (SHORT) dlo_s[l32] = r_dlo;
+            } else {
+                dl_s[l32] = r_row;
             }
         }
     };
@@ -405,25 +417,19 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     // sums in order and store delta = sum(e dP) / sum(e) as hi + lo.
     const int qs_end = SHORT && kblk == 0 ? min(q_end, p.n_short) : q_begin;  // short tiles: [q_begin, qs_end)
     if (SHORT && q_begin < qs_end) {
-        double* part = reinterpret_cast<double*>(&Qs[1][0][0][0]);  // [4][BQ] pairs (sum e, sum e dP)
-        static_assert(2 * 4 * BQ * sizeof(double) <= sizeof(Qs[1]), "the sums fit the second Q buffer");
+        // pairs (sum e, sum e dP) of each pair of waves, behind its P
+        constexpr int PSTRIDE = XPAIR / 16;
+        double* part = reinterpret_cast<double*>(lds + X_OFF + NKB * 4096);
+        static_assert(2 * BQ * sizeof(double) + NKB * 4096 <= XPAIR && XPAIR % 16 == 0, "the sums fit behind P");
         for (int q0 = q_begin; q0 < qs_end; q0 += BQ) {
-            sstore(0);
+            sstore();
             __syncthreads();
             gload(q0 + BQ, q0 + BQ < qs_end ? p.Tq : 0);
             const bool active = (!p.causal || (q0 + BQ - 1 + p.off >= k0p)) && k0p < p.Tk;
             f32x16 st[NKB];
-            f32x4* X = reinterpret_cast<f32x4*>(&Xs[pr][0]);
+            f32x4* X = reinterpret_cast<f32x4*>(lds + X_OFF + pr * XPAIR);
             if (active) {
-                const _Float16* rows = role ? &dOs[0][0][0] : &Qs[0][0][0][0];
-#pragma unroll
-                for (int kk = 0; kk < NKK; ++kk) {
-                    Half2x8 y;
-                    y.h = *reinterpret_cast<const f16x8*>(rows + l32 * QS + 16 * kk + 8 * g);
-                    y.l = *reinterpret_cast<const f16x8*>(rows + (BQ + l32) * QS + 16 * kk + 8 * g);
-#pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb) st[kb] = mfma_split<true>(xf[kb][kk], y, kk == 0 ? f32x16{} : st[kb]);
-                }
+                scores(st, std::false_type{});
                 if (role == 0) {
                     const int qi = q0 + l32;
                     const float L = lse_s[l32];
@@ -436,7 +442,7 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                             for (int cc = 0; cc < 4; ++cc) {
                                 const int kj = k0p + 32 * kb + 8 * j + 4 * g + cc;
                                 const bool vis = (qi < p.Tq) && (kj < p.Tk) && (!p.causal || kj <= qi + p.off);
-                                e[cc] = bwd_short_weight(p, qi, vis, fast_exp2(fmaf(st[kb][4 * j + cc], cs, -L)) * kBwdPInv);
+                                e[cc] = bwd_short_weight(p, qi, vis, fast_exp2(fmaf(st[kb][4 * j + cc], p.c, -L)));
                             }
                             X[(4 * kb + j) * 64 + lane] = e;
                         }
@@ -461,12 +467,12 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                 l += __shfl_xor(l, 32);
                 w += __shfl_xor(w, 32);
                 if (g == 0) {
-                    part[2 * (pr * BQ + l32)] = l;
-                    part[2 * (pr * BQ + l32) + 1] = w * ((double)xinv * (double)dinv_s[l32]);
+                    part[2 * (pr * PSTRIDE + l32)] = l;
+                    part[2 * (pr * PSTRIDE + l32) + 1] = w;
                 }
             }
             __syncthreads();
-            if (tid < BQ) bwd_short_delta_store<4, BQ>(p, bh, q0 + tid, part + 2 * tid);
+            if (tid < BQ) bwd_short_delta_store<4, PSTRIDE>(p, bh, q0 + tid, part + 2 * tid);
         }
         __syncthreads();  // the deltas are stored: the first tile's are read again
         gload(q_begin, p.Tq);
@@ -477,34 +483,20 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = f32x16{};
-    int dscls = 2;  // role 1: class of the largest |ds| so far
 
-    sstore(0);
+    sstore();
     __syncthreads();
 
-    int buf = 0;
-    for (int q0 = q_begin; q0 < q_end; q0 += BQ, buf ^= 1) {
-        // At D = 64 the lane number passes an empty asm, so that LDS addresses are
-        // formed in each tile instead of being held (and spilled) across the loop.
-        int ln = lane;
-        if constexpr (D == 64 && KP == 64) asm volatile("" : "+v"(ln));
-        const int lane = ln, l32 = ln & 31, g = ln >> 5;
+    for (int q0 = q_begin; q0 < q_end; q0 += BQ) {
         // ---- A: S and P (role 0), dP (role 1) -----------------------------------
         gload(q0 + BQ, q0 + BQ < q_end ? p.Tq : 0);
-        // Does any query of this tile see any key of this pair?
-        const bool active = (!p.causal || (q0 + BQ - 1 + p.off >= k0p)) && k0p < p.Tk;
-        f32x4* X = reinterpret_cast<f32x4*>(&Xs[pr][0]);
+        // Does any query of this tile see any key of a pair (of this one)?
+        auto sees = [&](int key0) { return (!p.causal || (q0 + BQ - 1 + p.off >= key0)) && key0 < p.Tk; };
+        const bool active = sees(k0p);
+        f32x4* X = reinterpret_cast<f32x4*>(lds + X_OFF + pr * XPAIR);
         f32x16 s[NKB];
         if (active) {
-            const _Float16* rows = role ? &dOs[0][0][0] : &Qs[buf][0][0][0];
-#pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) {
-                Half2x8 y;
-                y.h = *reinterpret_cast<const f16x8*>(rows + l32 * QS + 16 * kk + 8 * g);
-                y.l = *reinterpret_cast<const f16x8*>(rows + (BQ + l32) * QS + 16 * kk + 8 * g);
-#pragma unroll
-                for (int kb = 0; kb < NKB; ++kb) s[kb] = mfma_split<false>(y, xf[kb][kk], kk == 0 ? f32x16{} : s[kb]);
-            }
+            scores(s, std::true_type{});
             // reg 4j + cc of s[kb]: query row 8 j + 4 g + cc of the tile, key 32 kb + l32 of the pair
             if (role == 0) {
                 // Only tiles that cross the causal diagonal or the end of the
@@ -518,7 +510,7 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                             f32x4 e;
 #pragma unroll
                             for (int cc = 0; cc < 4; ++cc) {
-                                float pv = fast_exp2(fmaf(s[kb][4 * j + cc], cs, -L[cc]));
+                                float pv = fast_exp2(fmaf(s[kb][4 * j + cc], p.c, -L[cc]));
                                 if constexpr (decltype(masked)::value) {
                                     const int qi = q0 + 8 * j + 4 * g + cc, key = k0p + 32 * kb + l32;
                                     const bool vis = (qi < p.Tq) && (key < p.Tk) && (!p.causal || key <= qi + p.off);
@@ -538,11 +530,9 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
         }
         __syncthreads();
 
-        // ---- B: dV (role 0), dS (role 1) -----------------------------------------
-        Half2x8 pb[NKB][2];  // P or dS: queries 16 mm + 4 g + {0..3} and + 8 of key block kb
+        // ---- B: dV (role 0), dS and dK (role 1) ------------------------------------
         if (active) {
             if (role == 1) {
-                float mx = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const f32x4 Dl = *reinterpret_cast<const f32x4*>(&dl_s[8 * j + 4 * g]);
@@ -553,8 +543,8 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                         const f32x4 pv = X[(4 * kb + j) * 64 + lane];
 #pragma unroll
                         for (int cc = 0; cc < 4; ++cc) {
-                            float t = fmaf(-Dl[cc], xscale, s[kb][4 * j + cc]);
-                            if constexpr (SHORT) t = fmaf(-Dlo[cc], xscale, t);
+                            float t = s[kb][4 * j + cc] - Dl[cc];
+                            if constexpr (SHORT) t -= Dlo[cc];
                             s[kb][4 * j + cc] = pv[cc] * t;
                         }
                     }
@@ -565,82 +555,45 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                     for (int r = 0; r < 16; ++r)
                         if (bwd_one_key_row(p, q0 + 8 * (r >> 2) + 4 * g + (r & 3))) s[0][r] = 0.f;
                 }
-#pragma unroll
-                for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                    for (int r = 0; r < 16; r += 8)
-                        mx = absmax8(mx, f32x4{s[kb][r], s[kb][r + 1], s[kb][r + 2], s[kb][r + 3]},
-                                     f32x4{s[kb][r + 4], s[kb][r + 5], s[kb][r + 6], s[kb][r + 7]});
-                if (__any(mx >= class_limit(dscls))) {  // dK^T is kept in units of ds's scale
-                    mx = 0.f;
-#pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, finite_abs(s[kb][r]));
-                    const int nc = max(dscls, min(31, __builtin_amdgcn_readfirstlane(scale_class(wave_max(mx)))));
-                    const float f = class_scale(nc) * class_inv(dscls);
-#pragma unroll
-                    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                        for (int kb = 0; kb < NKB; ++kb) acc[db][kb] *= f;
-                    dscls = nc;
-                }
-                if (lane == 0) dqcls_s[pr] = dscls + xcls + kcls_s[pr];
-            }
-            const float psc = role ? class_scale(dscls) : 1.f;
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                for (int mm = 0; mm < 2; ++mm) {
-                    const f32x16& e = s[kb];
-                    pb[kb][mm] = split2(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
-                                        f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]}, psc);
-                }
-        } else if (role == 1 && !DQD) {
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                for (int mm = 0; mm < 2; ++mm) pb[kb][mm] = Half2x8{};
-            if (lane == 0) dqcls_s[pr] = -1;
-        }
-        if (role == 1 && !DQD) {
-            {
-                // dS over P (read above by this wave): row key l32, queries along it
+                // (dS goes over P below, which this wave has read)
                 asm volatile("" ::: "memory");
+            }
+            // dV^T += dO^T P or dK^T += Q^T dS, rows read transposed; step mm takes
+            // queries 16 mm + 4 g + {0..3} and + 8
+            Bf3x8 pb[NKB], a[2];
+            a[0] = T::tr_frag(lds, tr_off, 0, 0, PART);
 #pragma unroll
-                for (int kb = 0; kb < NKB; ++kb)
+            for (int st = 0; st < 2 * NDB; ++st) {
+                const int mm = st / NDB, db = st % NDB;
+                if (db == 0) {
 #pragma unroll
-                    for (int mm = 0; mm < 2; ++mm)
-#pragma unroll
-                        for (int hl = 0; hl < 2; ++hl) {
-                            const f16x8 v = hl ? pb[kb][mm].l : pb[kb][mm].h;
-                            _Float16* row = reinterpret_cast<_Float16*>(&Xs[pr][(2 * kb + hl) * XB]) + l32 * SS + 16 * mm + 4 * g;
-                            *reinterpret_cast<f16x4*>(row) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
-                            *reinterpret_cast<f16x4*>(row + 8) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+                    for (int kb = 0; kb < NKB; ++kb) {
+                        const f32x16& e = s[kb];
+                        pb[kb] = split3<true>(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
+                                              f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]});
+                        if (role == 1 && !DQD) {  // row key l32, queries along it
+                            auto put = [&](int part, const bf16x8& v) {
+                                char* row = lds + X_OFF + pr * XPAIR + (3 * kb + part) * XB + (l32 * SS + 16 * mm + 4 * g) * 2;
+                                *reinterpret_cast<bf16x4*>(row) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+                                *reinterpret_cast<bf16x4*>(row + 16) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+                            };
+                            put(0, pb[kb].h);
+                            put(1, pb[kb].m);
+                            put(2, pb[kb].l);
                         }
+                    }
+                }
+                if (st + 1 < 2 * NDB) a[(st + 1) & 1] = T::tr_frag(lds, tr_off, 16 * ((st + 1) / NDB), (st + 1) % NDB, PART);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = mfma_split3(a[st & 1], pb[kb], acc[db][kb]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // acc += rows^T pb (dO^T P or Q^T dS), rows read transposed
-        auto accumulate = [&](const _Float16* rows) {
-            const int a_off = (4 * (ln >> 5) + ((ln & 15) >> 2)) * QS + 16 * ((ln >> 4) & 1) + 4 * (ln & 3);
-#pragma unroll
-            for (int mm = 0; mm < 2; ++mm)
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) {
-                    const _Float16* at = rows + a_off + 16 * mm * QS + db * 32;
-                    Half2x8 a;
-                    a.h = tr_frag([&](int r) { return at + r * QS; });
-                    a.l = tr_frag([&](int r) { return at + (BQ + r) * QS; });
-#pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = mfma_split(a, pb[kb][mm], acc[db][kb]);
-                }
-        };
-        if (active && role == 0) accumulate(&dOs[0][0][0]);
         __syncthreads();
 
-        // ---- C: dQ (both), dK (role 1), the next dO tile (role 0) ------------------
-        sstore(buf ^ 1);
-        if (active && role == 1) accumulate(&Qs[buf][0][0][0]);
+        // ---- C: dQ (role 0), the next tile (both) -----------------------------------
+        sstore();
         if constexpr (!DQD) {
             if (role == 0) {
                 // dQ tile (32 x D) = dS K: a wave takes a 32-wide head-dim block, over all
@@ -651,41 +604,62 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                 // took 160 cycles per ds_add_f32.)
                 const int db = pr % NDB;
                 f32x16 dq = f32x16{};
-                int unit = -1;  // dq is in units of 2^(8 unit)
+                struct Ops {
+                    Bf3x8 ds;
+                    bf16x8 kh, km;
+                };
+                // step st: pair pr / NDB * DQP + st / (2 NKB), keys 16 (st % (2 NKB)) .. + 15 of it
+                auto ops = [&](int st) {
+                    const int pi = st / (2 * NKB), kb = st % (2 * NKB) / 2, m = st % 2;
+                    auto ds_part = [&](int part) {
+                        const char* at = lds + ds_off + pi * XPAIR + (3 * kb + part) * XB + 16 * m * SS * 2;
+                        return __builtin_shufflevector(ds_read_tr16(reinterpret_cast<const __bf16*>(at)),
+                                                       ds_read_tr16(reinterpret_cast<const __bf16*>(at + 8 * SS * 2)), 0, 1, 2, 3, 4, 5, 6, 7);
+                    };
+                    const int row0 = pi * KP + 32 * kb + 16 * m;
+                    Ops o;
+                    o.ds.h = ds_part(0);
+                    o.ds.m = ds_part(1);
+                    o.ds.l = ds_part(2);
+                    o.kh = T::tr_part(lds, ktr_off, row0, db, 0);
+                    o.km = T::tr_part(lds, ktr_off, row0, db, KPART);
+                    return o;
+                };
+                auto mul = [&](const Ops& o, int st) {
+                    dq = mfma_split3(o.ds, Bf3x8{o.kh, o.km, __builtin_bit_cast(bf16x8, xr[st / NKK][st % NKK][1])}, dq);
+                };
+                const int pp0 = pr / NDB * DQP;
+                if (sees(k0 + (pp0 + DQP - 1) * KP)) {
+                    Ops o[2];
+                    o[0] = ops(0);
 #pragma unroll
-                for (int pi = 0; pi < DQP; ++pi) {
-                    const int pp = pr / NDB * DQP + pi;
-                    const int u = __builtin_amdgcn_readfirstlane(dqcls_s[pp]);  // < 0: the pair's dS is zero
-                    const int d = u >= 0 && unit >= 0 ? min(max(unit - u, -15), 15) : 0;
-                    unit = u >= 0 ? u : unit;
-                    if (pi > 0) dq *= __uint_as_float((uint32_t)(127 + 8 * d) << 23);
+                    for (int st = 0; st < NKB * NKK; ++st) {
+                        if (st + 1 < NKB * NKK) o[(st + 1) & 1] = ops(st + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                        mul(o[st & 1], st);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                } else {
+                    // (a pair that no row sees wrote no dS, and its keys must not reach these rows)
 #pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb)
+                    for (int pi = 0; pi < DQP; ++pi)
+                        if (sees(k0 + (pp0 + pi) * KP)) {
 #pragma unroll
-                        for (int m = 0; m < 2; ++m) {
-                            const _Float16* ds = reinterpret_cast<const _Float16*>(&Xs[pp][2 * kb * XB]) +
-                                                 (16 * m + 4 * g + ((lane & 15) >> 2)) * SS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-                            Half2x8 a, kf;
-                            a.h = tr_frag([&](int r) { return ds + r * SS; });
-                            a.l = tr_frag([&](int r) { return ds + XB / 2 + r * SS; });
-                            kf.h = Kt[0][(pp * KP + 32 * kb + 16 * m) / 8 + g][db * 32 + l32];
-                            kf.l = Kt[1][(pp * KP + 32 * kb + 16 * m) / 8 + g][db * 32 + l32];
-                            dq = mfma_split(a, kf, dq);
+                            for (int i = 0; i < 2 * NKB; ++i) mul(ops(pi * 2 * NKB + i), pi * 2 * NKB + i);
                         }
                 }
-                const float f = ldexpf(kBwdPInv * doinv * p.scale, 8 * unit - 414);
                 const auto rdq = row_rsrc(dQa, p.sacc.t, q0, min(p.Tq - q0, BQ), D);  // rows past Tq are dropped
                 const uint32_t voff = (uint32_t)(((int64_t)(4 * g) * p.sacc.t + db * 32 + l32) * 4);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    buffer_atomic_add(rdq, dq[r] * f, voff, (uint32_t)((int64_t)(8 * (r >> 2) + (r & 3)) * p.sacc.t * 4));
+                    buffer_atomic_add(rdq, dq[r] * p.scale, voff, (uint32_t)((int64_t)(8 * (r >> 2) + (r & 3)) * p.sacc.t * 4));
             }
         }
         __syncthreads();
     }
 
     // ---- dK = scale * dK^T^T, dV = dV^T^T ------------------------------------------
-    const float unit = role ? class_inv(dscls) * dsu * qinv * p.scale : kBwdPInv * doinv;
+    const float unit = role ? p.scale : 1.f;
     f32x16 out[NDB * NKB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -746,10 +720,9 @@ __global__ __launch_bounds__(256) void bwd_cvt_kernel(BwdParams p) {
 // Query-major dQ pass, fp32 (the deterministic mode: the main kernel then
 // skips its dQ product).  One workgroup = 4 waves x 32 query rows of one
 // (b, h), laid out as the forward: each lane keeps its query row of Q and dO
-// as split B operands (Q^T, dO^T) in VGPRs, with that row's log-sum-exp and
-// delta; tiles of 32 keys of K and V, split, are double-buffered in LDS (loaded
-// two tiles ahead, scaled by the class of the largest magnitude so far).  Per
-// wave and tile:
+// (the B operands Q^T, dO^T, split for each tile) in VGPRs, with that row's
+// log-sum-exp and delta; tiles of 32 keys of K and V, split, are double-buffered in
+// LDS (loaded two tiles ahead).  Per wave and tile:
 //   S^T = K Q^T, dP^T = V dO^T        in the forward's and the main kernel's
 //                                     order, to the same bits
 //   P^T = exp2(S^T c - lse log2 e), dS^T = P^T (dP^T - delta)
@@ -768,19 +741,17 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
     constexpr int C8 = D / 8;            // 8-element chunks per row
     constexpr int NCH = BN * C8;         // chunks of a tile
     constexpr int CPT = (NCH + 255) / 256;
-    constexpr int QS = BwdTile<D, 32>::QS;
+    using T = BwdTile<D, 32>;
+    constexpr int PART = BN * T::QS * 2, K_OFF = 0, V_OFF = 6 * PART;
     static_assert(BM == 128 && 256 % C8 == 0, "4 waves x 32 rows, whole staging passes");
 
-    __shared__ __attribute__((aligned(16))) _Float16 Ks[2][2][BN][QS];  // [buffer][part]
-    __shared__ __attribute__((aligned(16))) _Float16 Vs[2][2][BN][QS];
-    __shared__ int cls_s[2][2][4];  // scale class that each wave's loads need: [K, V][tile parity]
+    __shared__ __attribute__((aligned(256))) char lds[12 * PART];  // K, then V: [buffer][part]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31;
     const int g = lane >> 5;
-    const int tr_row = (lane & 15) >> 2, tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
     const int BH = p.B * p.H;
     const int w = blockIdx.x;
@@ -796,35 +767,23 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
 
     const int q0w = qtile * BM + wave * 32;
     const int qrow = q0w + l32;
-    // B operands: MFMA step kk takes row qrow, columns 16 kk + 8 g .. + 7, scaled by the row's class.
-    Half2x8 qf[NKK], df[NKK];
-    float qinv, doscale, doinv;
-    auto load_row = [&](const float* src, int64_t st, Half2x8 (&f)[NKK]) {
-        f32x4 raw[NKK][2];
-        float amax = 0.f;
+    // B operands: MFMA step kk takes row qrow, columns 16 kk + 8 g .. + 7, split for each tile.
+    f32x4 qr[NKK][2], dr[NKK][2];
+    auto load_row = [&](const float* src, int64_t st, f32x4 (&f)[NKK][2]) {
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
-            raw[kk][0] = raw[kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            f[kk][0] = f[kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
             if (qrow < p.Tq) {
-                raw[kk][0] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g);
-                raw[kk][1] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g + 4);
+                f[kk][0] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g);
+                f[kk][1] = ld4(src + (int64_t)qrow * st + 16 * kk + 8 * g + 4);
             }
-            amax = absmax8_finite(amax, raw[kk][0], raw[kk][1]);
         }
-        const int k = scale_class(max_xor32(amax));
-#pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) f[kk] = split2(raw[kk][0], raw[kk][1], class_scale(k));
-        return k;
     };
-    qinv = class_inv(load_row(Q, p.sq.t, qf));
-    {
-        const int k = load_row(dO, p.sdo.t, df);
-        doscale = class_scale(k);
-        doinv = class_inv(k);
-    }
-    const float Lq = qrow < p.Tq ? fmaf(p.lse[(int64_t)bh * p.Tq + qrow], kLog2e, -kBwdPBits) : 0.f;
-    const float Dq = qrow < p.Tq ? p.delta[(int64_t)bh * p.Tq + qrow] * doscale : 0.f;
-    const float Dqlo = bwd_short_row(p, qrow) ? p.delta_lo[(int64_t)bh * p.Tq + qrow] * doscale : 0.f;
+    load_row(Q, p.sq.t, qr);
+    load_row(dO, p.sdo.t, dr);
+    const float Lq = qrow < p.Tq ? p.lse[(int64_t)bh * p.Tq + qrow] * kLog2e : 0.f;
+    const float Dq = qrow < p.Tq ? p.delta[(int64_t)bh * p.Tq + qrow] : 0.f;
+    const float Dqlo = bwd_short_row(p, qrow) ? p.delta_lo[(int64_t)bh * p.Tq + qrow] : 0.f;
     const bool one_key = qrow < p.Tq && bwd_one_key_row(p, qrow);
     const bool one_key_wave = p.causal ? (-p.off >= q0w && -p.off < q0w + 32) : p.Tk == 1;  // wave-uniform
 
@@ -854,47 +813,14 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
             r.v[i][1] = buffer_ld4(rv, v_voff + 16, vo);
         }
     };
-    int kcls = 2, vcls = 2;  // classes of the tile in LDS (as in the forward)
-    auto need_classes = [&](const Raw& r, int par) {
-        float mk = 0.f, mv = 0.f;
+    auto sstore = [&](const Raw& r, int buf) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
-            mk = absmax8(mk, r.k[i][0], r.k[i][1]);
-            mv = absmax8(mv, r.v[i][0], r.v[i][1]);
-        }
-        int nk = 0, nv = 0;
-        if (__any(mk >= class_limit(kcls) || mv >= class_limit(vcls))) {
-            mk = mv = 0.f;
-#pragma unroll
-            for (int i = 0; i < CPT; ++i) {
-                mk = absmax8_finite(mk, r.k[i][0], r.k[i][1]);
-                mv = absmax8_finite(mv, r.v[i][0], r.v[i][1]);
-            }
-            nk = scale_class(wave_max(mk));
-            nv = scale_class(wave_max(mv));
-        }
-        if (lane == 0) {
-            cls_s[0][par][wave] = nk;
-            cls_s[1][par][wave] = nv;
-        }
-    };
-    auto class_of = [&](int which, int par, int cur) {  // after the barrier
-        int m = cur;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m = max(m, cls_s[which][par][i]);
-        return __builtin_amdgcn_readfirstlane(m);
-    };
-    auto sstore = [&](const Raw& r, int buf, int kc, int vc) {
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int f = tid + 256 * i, row = f / C8, col = 8 * (f % C8);
+            const int f = tid + 256 * i;
             if (NCH % 256 == 0 || f < NCH) {
-                const Half2x8 k = split2(r.k[i][0], r.k[i][1], class_scale(kc));
-                const Half2x8 v = split2(r.v[i][0], r.v[i][1], class_scale(vc));
-                *reinterpret_cast<f16x8*>(&Ks[buf][0][row][col]) = k.h;
-                *reinterpret_cast<f16x8*>(&Ks[buf][1][row][col]) = k.l;
-                *reinterpret_cast<f16x8*>(&Vs[buf][0][row][col]) = v.h;
-                *reinterpret_cast<f16x8*>(&Vs[buf][1][row][col]) = v.l;
+                char* at = lds + 3 * buf * PART + T::at(f / C8, f % C8);
+                T::put(at + K_OFF, split3<true>(r.k[i][0], r.k[i][1]), PART);
+                T::put(at + V_OFF, split3(r.v[i][0], r.v[i][1]), PART);
             }
         }
     };
@@ -902,50 +828,41 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
     f32x16 dq[NDB];
 #pragma unroll
     for (int i = 0; i < NDB; ++i) dq[i] = f32x16{};
-    int dscls = 2;  // class of the row's largest |ds| so far, per lane
 
     Raw ra, rb;
     gload(ra, 0);
-    need_classes(ra, 0);
     gload(rb, 1);
-    __syncthreads();
-    kcls = class_of(0, 0, kcls);
-    vcls = class_of(1, 0, vcls);
-    sstore(ra, 0, kcls, vcls);
-    need_classes(rb, 1);
+    sstore(ra, 0);
     __syncthreads();
     auto step = [&](int u, Raw& nxt, Raw& far) {
         const int buf = u & 1;
         const int k0 = u * BN;
         gload(far, u + 2);
-        const int nk = class_of(0, (u + 1) & 1, kcls), nv = class_of(1, (u + 1) & 1, vcls);
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk)  // split again for each tile, not held (as in the main kernel)
+            asm volatile("" : "+v"(qr[kk][0]), "+v"(qr[kk][1]), "+v"(dr[kk][0]), "+v"(dr[kk][1]));
         if (k0 < wave_kend) {
-            f32x16 s, dp;
+            Split3Sum ss, dps;
+            ss.hi = ss.lo = dps.hi = dps.lo = f32x16{};
 #pragma unroll
             for (int kk = 0; kk < NKK; ++kk) {
-                Half2x8 k, v;
-                k.h = *reinterpret_cast<const f16x8*>(&Ks[buf][0][l32][16 * kk + 8 * g]);
-                k.l = *reinterpret_cast<const f16x8*>(&Ks[buf][1][l32][16 * kk + 8 * g]);
-                v.h = *reinterpret_cast<const f16x8*>(&Vs[buf][0][l32][16 * kk + 8 * g]);
-                v.l = *reinterpret_cast<const f16x8*>(&Vs[buf][1][l32][16 * kk + 8 * g]);
-                s = mfma_split(k, qf[kk], kk == 0 ? f32x16{} : s);
-                dp = mfma_split(v, df[kk], kk == 0 ? f32x16{} : dp);
+                mfma_split3(T::row_frag(lds + K_OFF + 3 * buf * PART, T::row_lane(lane), kk, PART), split3(qr[kk][0], qr[kk][1]), ss);
+                mfma_split3(T::row_frag(lds + V_OFF + 3 * buf * PART, T::row_lane(lane), kk, PART), split3(dr[kk][0], dr[kk][1]), dps);
             }
+            f32x16 s = ss.sum(), dp = dps.sum();
             // reg r: key k0 + 8 (r / 4) + 4 g + r % 4 of query qrow
             const bool need_mask = (k0 + BN > p.Tk) || (qtile * BM + BM > p.Tq) || (p.causal && (k0 + BN - 1 > q0w + p.off));
             const int lim = p.causal ? min(p.Tk - 1, qrow + p.off) : p.Tk - 1;
-            const float cs = p.c * qinv * class_inv(kcls), vscale = class_scale(vcls);
             // the visibility test only on tiles that cross the diagonal or the ends
-            float mx = 0.f;
             auto p_ds = [&](auto masked) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    float pr = fast_exp2(fmaf(s[r], cs, -Lq));
+                    float pr = fast_exp2(fmaf(s[r], p.c, -Lq));
                     if constexpr (decltype(masked)::value) {
                         const int key = k0 + 8 * (r >> 2) + 4 * g + (r & 3);
                         pr = (key <= lim && qrow < p.Tq) ? pr : 0.f;
                     }
-                    s[r] = pr * fmaf(-Dqlo, vscale, fmaf(-Dq, vscale, dp[r]));  // dS^T
+                    s[r] = pr * ((dp[r] - Dq) - Dqlo);  // dS^T
                 }
             };
             if (need_mask)
@@ -953,43 +870,17 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
             else
                 p_ds(std::false_type{});
             if (one_key_wave && k0 == 0 && one_key) s = f32x16{};  // one visible key: dS = P (dP - dP) = 0
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fabsf(s[r]));
-            if (__any(mx >= class_limit(dscls))) {  // a row's dQ is kept in units of its ds scale
-                mx = 0.f;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, finite_abs(s[r]));
-                const int nc = max(dscls, min(31, scale_class(max_xor32(mx))));
-                const float f = class_scale(nc) * class_inv(dscls);
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) dq[db] *= f;
-                dscls = nc;
-            }
-            const float sc = class_scale(dscls);
             // dQ^T[d][q] += K^T[d][keys] dS^T[keys][q]: step m takes keys 16 m + 4 g + {0..3} and + 8
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
-                const Half2x8 ds = split2(f32x4{s[8 * m], s[8 * m + 1], s[8 * m + 2], s[8 * m + 3]},
-                                          f32x4{s[8 * m + 4], s[8 * m + 5], s[8 * m + 6], s[8 * m + 7]}, sc);
-                const int r0 = 16 * m + 4 * g + tr_row;
+                const Bf3x8 ds = split3(f32x4{s[8 * m], s[8 * m + 1], s[8 * m + 2], s[8 * m + 3]},
+                                        f32x4{s[8 * m + 4], s[8 * m + 5], s[8 * m + 6], s[8 * m + 7]});
 #pragma unroll
-                for (int db = 0; db < NDB; ++db) {
-                    Half2x8 kt;
-                    kt.h = tr_frag([&](int r) { return &Ks[buf][0][r0 + r][db * 32 + tr_col]; });
-                    kt.l = tr_frag([&](int r) { return &Ks[buf][1][r0 + r][db * 32 + tr_col]; });
-                    dq[db] = mfma_split(kt, ds, dq[db]);
-                }
+                for (int db = 0; db < NDB; ++db)
+                    dq[db] = mfma_split3(T::tr_frag(lds + K_OFF + 3 * buf * PART, T::tr_lane(lane), 16 * m, db, PART), ds, dq[db]);
             }
         }
-        if (nk != kcls || nv != vcls) {  // ... and of K's and V's scales
-            const float f = (class_scale(nk) * class_inv(kcls)) * (class_scale(nv) * class_inv(vcls));
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) dq[db] *= f;
-        }
-        kcls = nk;
-        vcls = nv;
-        sstore(nxt, buf ^ 1, nk, nv);
-        need_classes(far, u & 1);
+        sstore(nxt, buf ^ 1);
         __syncthreads();
     };
     for (int u = 0; u < nt; u += 2) {
@@ -997,14 +888,13 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
         if (u + 1 < nt) step(u + 1, ra, rb);
     }
     if (qrow < p.Tq) {
-        const float unit = class_inv(dscls) * kBwdPInv * class_inv(vcls) * doinv * class_inv(kcls) * p.scale;
         float* dst = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)qrow * p.sdq.t;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 st4(dst + db * 32 + 8 * j + 4 * g,
-                    f32x4{dq[db][4 * j], dq[db][4 * j + 1], dq[db][4 * j + 2], dq[db][4 * j + 3]} * unit);
+                    f32x4{dq[db][4 * j], dq[db][4 * j + 1], dq[db][4 * j + 2], dq[db][4 * j + 3]} * p.scale);
     }
 }
 
@@ -1258,7 +1148,7 @@ static int launch_bwd_t(const BwdParams& p_in, hipStream_t s) {
     const int64_t rows = (int64_t)p.B * p.H * p.Tq;
     const dim3 pre_grid((unsigned)((rows + RPB - 1) / RPB));  // bwd_cvt: 4 elements per thread
     constexpr int PRE_RPB = bwd_pre_rows_per_block<D, E>();
-    const dim3 delta_grid((unsigned)(sizeof(E) == 4 ? (int64_t)p.B * p.H * p.n_amax : (rows + PRE_RPB - 1) / PRE_RPB));
+    const dim3 delta_grid((unsigned)((rows + PRE_RPB - 1) / PRE_RPB));
     if (!p.pre_delta && !p.dq_direct) {
         // zeroing only: a few grid-stride workgroups per CU
         const int64_t n4 = rows * D / 4;

@@ -1,13 +1,14 @@
 // attn_fwd.hip -- fused causal attention forward for gfx950, fp32.
 //
 // One workgroup = 8 waves = 256 query rows of one (b, h); each wave owns 32
-// rows for the whole kernel.  Both products run on the fp16 matrix cores, every
-// operand split into two fp16 parts (common.h), three MFMAs per product step.
+// rows for the whole kernel.  Both products run on the bf16 matrix cores, every
+// operand split into three bf16 parts (common.h), six MFMAs per product step: no
+// scales, so a row depends on what it sees alone, at any magnitude.
 // K and V tiles of BN keys are loaded two tiles ahead into registers, split
 // once for all eight waves into double-buffered LDS, one barrier per tile.  Per
 // wave and tile:
 //
-//   S^T (keys x queries) = K Q^T      v_mfma_f32_32x32x16_f16, A = K from LDS,
+//   S^T (keys x queries) = K Q^T      v_mfma_f32_32x32x16_bf16, A = K from LDS,
 //                                     B = Q^T resident in VGPRs, split
 //   online softmax on S^T             query = lane%32, so the row max needs one
 //                                     xor-32 exchange; the row sum stays
@@ -20,15 +21,15 @@
 // part: a thread loads one column of the 8 keys that an operand takes together,
 // so the transposition costs no store.
 //
-// At D = 128 the kernel keeps the matrix cores 49% busy at a 1.97 GHz shader
-// clock (the rest is softmax and split VALU work, 39% of the issue slots, that
-// overlaps only in part); at D = 64 a workgroup's serial chain of tiles, about
-// 6500 cycles each for 3072 of MFMA, sets causal grids of a round or two.
-// Against the fp32-MFMA kernel it replaced (us): config 2 128.8 -> 58.4, config 4
-// 2281 -> 726, B8 H12 T1024 D32 73 -> 38, B1 H12 T1024 D64 37 -> 26.  With three
-// bf16 parts and six MFMAs instead: 78.6 and 1229.  128-row workgroups of four
-// waves (each tile split twice as often) lost at every D = 128 shape and config
-// 4 (726 -> 988), gaining only on large D = 64 grids (B16 H12 117 -> 110).
+// At D = 128 the kernel keeps the matrix cores 67% busy at a shader clock that the
+// load holds at 1.9 GHz (VALU work, 30% of the issue slots, overlaps in part): 1.65
+// PFLOP of MFMAs in 1.27 ms, the rate of a large library product in bf16.  At D = 64 a
+// workgroup's serial chain of tiles sets causal grids of a round or two (51% busy).
+// Against the fp32 MFMAs (us): config 2 128.8 -> 82.6, config 4 2281 -> 1270.  Two
+// fp16 parts per operand, scaled by the largest value of a tile, and three MFMAs took
+// 58.4 and 726, but a value 2^10 below its tile's largest lost bits, also to a key
+// that the row can't see.  128-row workgroups of four waves split each tile twice as
+// often.
 //
 // Keeping queries on the lane axis in both products is what lets P stay in
 // registers.  The scale is folded into exp2: p = exp2(s*c - m) with
@@ -65,15 +66,11 @@ struct FwdTile {
     static constexpr int NW = 8;  // waves per workgroup, 32 query rows each
     static constexpr int BM = 32 * NW;
     static constexpr int BN = D == 32 ? 128 : D == 64 ? 64 : 32;  // keys per LDS tile: one 8-element unit per thread
-    static constexpr int KS = D + 8;                              // K row stride in LDS (fp16 elements)
+    static constexpr int KS = D + 8;                              // K row stride in LDS (bf16 elements)
 };
 
 // Headroom of the forward's lazy rescaling, in exp2 units: P <= 2^8.
 constexpr float kLazyLog2 = 8.f;
-// P enters its products as 2^kPBits P, at most 2^14: the low part of a
-// probability of 2^-9 or more is then a normal fp16 number, and a smaller one
-// carries an absolute error of 2^-31 of the row's reference.
-constexpr float kPBits = 6.f, kPInv = 1.f / 64.f;
 
 template <int D>
 __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdParams p) {
@@ -88,11 +85,10 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
     constexpr int UPT = BN * C8 / NT;    // 8-element units per thread per tensor per tile
     static_assert(BN * C8 % NT == 0 && NT % D == 0 && NT % C8 == 0, "whole staging passes");
 
-    __shared__ __attribute__((aligned(16))) _Float16 Ks0[2][BN][KS];
-    __shared__ __attribute__((aligned(16))) _Float16 Ks1[2][BN][KS];
-    __shared__ f16x8 Vt0[2][BN / 8][D];
-    __shared__ f16x8 Vt1[2][BN / 8][D];
-    __shared__ __attribute__((aligned(16))) int cls_s[2][2][8];  // scale class that each wave's loads need: [K, V][tile parity]
+    __shared__ __attribute__((aligned(16))) __bf16 Ks0[3][BN][KS];
+    __shared__ __attribute__((aligned(16))) __bf16 Ks1[3][BN][KS];
+    __shared__ bf16x8 Vt0[3][BN / 8][D];
+    __shared__ bf16x8 Vt1[3][BN / 8][D];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -124,26 +120,16 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
     const int q0w = qtile * BM + wave * 32;  // first query row of this wave
     const int qrow = q0w + l32;              // this lane's query row
 
-    // Q^T operand: MFMA step kk takes Q[qrow][16 kk + 8 g .. + 7], scaled by the
-    // row's own class.
-    Half2x8 qf[NKK];
-    float cq;  // scale * log2(e) over the row's scale
-    {
-        f32x4 qa[NKK][2];
-        float amax = 0.f;
+    // Q^T operand: MFMA step kk takes Q[qrow][16 kk + 8 g .. + 7].
+    Bf3x8 qf[NKK];
 #pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) {
-            qa[kk][0] = qa[kk][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (qrow < p.Tq) {
-                qa[kk][0] = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g);
-                qa[kk][1] = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g + 4);
-            }
-            amax = absmax8_finite(amax, qa[kk][0], qa[kk][1]);
+    for (int kk = 0; kk < NKK; ++kk) {
+        f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f}, b2 = a;
+        if (qrow < p.Tq) {
+            a = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g);
+            b2 = ld4(Q + (int64_t)qrow * p.sq.t + 16 * kk + 8 * g + 4);
         }
-        const int k = scale_class(max_xor32(amax));
-        cq = p.c * class_inv(k);
-#pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) qf[kk] = split2(qa[kk][0], qa[kk][1], class_scale(k));
+        qf[kk] = split3(a, b2);
     }
 
     // Keys this workgroup needs, and this wave's visible limit (exclusive).
@@ -182,53 +168,19 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
                                        (uint32_t)((int64_t)((D >= 64 ? r0 : 0) + (e & 3) + 8 * (e >> 2)) * p.sv.t * 4));
         }
     };
-    // K and V tiles are scaled by the class of the largest magnitude so far in
-    // the workgroup's range (kk_cls, kv_cls: the classes of the split tile in
-    // LDS).  A wave whose loads of a tile exceed the classes that it knows says so
-    // in LDS one barrier ahead of the split; ordinary tensors do it once.
-    int kk_cls = 2, kv_cls = 2;
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     auto v4 = [](const float (&v)[8], int j) { return f32x4{v[j], v[j + 1], v[j + 2], v[j + 3]}; };
-    auto need_classes = [&](const Raw& r, int par) {
-        float mk = 0.f, mv = 0.f;
-#pragma unroll
-        for (int i = 0; i < UPT; ++i) {
-            mk = absmax8(mk, r.k[i][0], r.k[i][1]);
-            mv = absmax8(mv, v4(r.v[i], 0), v4(r.v[i], 4));
-        }
-        int nk = 0, nv = 0;
-        if (__any(mk >= class_limit(kk_cls) || mv >= class_limit(kv_cls))) {
-            mk = mv = 0.f;
-#pragma unroll
-            for (int i = 0; i < UPT; ++i) {
-                mk = absmax8_finite(mk, r.k[i][0], r.k[i][1]);
-                mv = absmax8_finite(mv, v4(r.v[i], 0), v4(r.v[i], 4));
-            }
-            nk = scale_class(wave_max(mk));
-            nv = scale_class(wave_max(mv));
-        }
-        if (lane == 0) {
-            cls_s[0][par][wave_u] = nk;
-            cls_s[1][par][wave_u] = nv;
-        }
-    };
-    auto class_of = [&](int which, int par, int cur) {  // after the barrier
-        int m = cur;
-#pragma unroll
-        for (int w = 0; w < FwdTile<D>::NW; ++w) m = max(m, cls_s[which][par][w]);
-        return __builtin_amdgcn_readfirstlane(m);
-    };
-    auto sstore = [&](const Raw& r, _Float16 (&Kd)[2][BN][KS], f16x8 (&Vd)[2][BN / 8][D], int kc, int vc) {
-        const float ks = class_scale(kc), vs = class_scale(vc);
+    auto sstore = [&](const Raw& r, __bf16 (&Kd)[3][BN][KS], bf16x8 (&Vd)[3][BN / 8][D]) {
 #pragma unroll
         for (int i = 0; i < UPT; ++i) {
             const int f = tid + NT * i;
-            const Half2x8 k = split2(r.k[i][0], r.k[i][1], ks);
-            const Half2x8 v = split2(v4(r.v[i], 0), v4(r.v[i], 4), vs);
-            *reinterpret_cast<f16x8*>(&Kd[0][f / C8][8 * (f % C8)]) = k.h;
-            *reinterpret_cast<f16x8*>(&Kd[1][f / C8][8 * (f % C8)]) = k.l;
+            const Bf3x8 k = split3(r.k[i][0], r.k[i][1]);
+            *reinterpret_cast<bf16x8*>(&Kd[0][f / C8][8 * (f % C8)]) = k.h;
+            *reinterpret_cast<bf16x8*>(&Kd[1][f / C8][8 * (f % C8)]) = k.m;
+            *reinterpret_cast<bf16x8*>(&Kd[2][f / C8][8 * (f % C8)]) = k.l;
+            const Bf3x8 v = split3(v4(r.v[i], 0), v4(r.v[i], 4));
             Vd[0][f / D][f % D] = v.h;
-            Vd[1][f / D][f % D] = v.l;
+            Vd[1][f / D][f % D] = v.m;
+            Vd[2][f / D][f % D] = v.l;
         }
     };
 
@@ -236,17 +188,12 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
 #pragma unroll
     for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
     float m_run = -INFINITY;  // reference max of row qrow's scores, in exp2 units
-    float l_run = 0.f;        // this lane's partial sum of 2^kPBits p (its half of the keys)
+    float l_run = 0.f;        // this lane's partial sum of p (its half of the keys)
 
     Raw ra, rb;
     gload(ra, t_begin);
-    need_classes(ra, t_begin & 1);
     gload(rb, t_begin + 1);
-    __syncthreads();
-    kk_cls = class_of(0, t_begin & 1, kk_cls);
-    kv_cls = class_of(1, t_begin & 1, kv_cls);
-    sstore(ra, Ks0, Vt0, kk_cls, kv_cls);
-    need_classes(rb, (t_begin + 1) & 1);
+    sstore(ra, Ks0, Vt0);
     __syncthreads();
 
     // Step t reads tile t from buffer BUF = (t - t_begin) % 2 while tile t + 2
@@ -255,25 +202,29 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
     // previous step's barrier.
     auto step = [&](int t, auto buf_c, Raw& nxt, Raw& far) {
         constexpr int BUF = decltype(buf_c)::value;
-        _Float16(&Kc)[2][BN][KS] = BUF ? Ks1 : Ks0;
-        f16x8(&Vc)[2][BN / 8][D] = BUF ? Vt1 : Vt0;
+        __bf16(&Kc)[3][BN][KS] = BUF ? Ks1 : Ks0;
+        bf16x8(&Vc)[3][BN / 8][D] = BUF ? Vt1 : Vt0;
         const int k0 = t * BN;
         gload(far, t + 2);
-        const int nk = class_of(0, (t + 1) & 1, kk_cls), nv = class_of(1, (t + 1) & 1, kv_cls);
         if (k0 < wave_kend) {
             f32x16 s[NKB];
+            {
+                Split3Sum st[NKB];
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk)
+                for (int kb = 0; kb < NKB; ++kb) st[kb].hi = st[kb].lo = f32x16{};
 #pragma unroll
-                for (int kb = 0; kb < NKB; ++kb) {
-                    Half2x8 a;
-                    a.h = *reinterpret_cast<const f16x8*>(&Kc[0][kb * 32 + l32][16 * kk + 8 * g]);
-                    a.l = *reinterpret_cast<const f16x8*>(&Kc[1][kb * 32 + l32][16 * kk + 8 * g]);
-                    s[kb] = mfma_split(a, qf[kk], kk == 0 ? f32x16{} : s[kb]);
-                }
-            // scores in exp2 units are s * cs (at least the smallest normal
-            // number, so a masked score times it stays -inf)
-            const float cs = fmaxf(cq * class_inv(kk_cls), 1.17549435e-38f);
+                for (int kk = 0; kk < NKK; ++kk)
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb) {
+                        Bf3x8 a;
+                        a.h = *reinterpret_cast<const bf16x8*>(&Kc[0][kb * 32 + l32][16 * kk + 8 * g]);
+                        a.m = *reinterpret_cast<const bf16x8*>(&Kc[1][kb * 32 + l32][16 * kk + 8 * g]);
+                        a.l = *reinterpret_cast<const bf16x8*>(&Kc[2][kb * 32 + l32][16 * kk + 8 * g]);
+                        mfma_split3(a, qf[kk], st[kb]);
+                    }
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) s[kb] = st[kb].sum();
+            }
             // reg 4j+cc of s[kb] holds key kb*32 + 8j + 4g + cc
             const bool need_mask = (k0 + BN > p.Tk) || (p.causal && (k0 + BN - 1 > q0w + p.off));
             if (need_mask) {
@@ -291,7 +242,7 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mp[r & 3] = fmaxf(mp[r & 3], s[kb][r]);
-            const float mloc = max_xor32(fmaxf(fmaxf(mp[0], mp[1]), fmaxf(mp[2], mp[3]))) * cs;
+            const float mloc = max_xor32(fmaxf(fmaxf(mp[0], mp[1]), fmaxf(mp[2], mp[3]))) * p.c;
             // Lazy rescaling: a row's reference max m_run moves only when the row
             // sees a score more than kLazyLog2 above it, so P stays
             // <= 2^kLazyLog2; the O / l rescale and its exp2 run only on tiles where
@@ -309,14 +260,14 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
                 for (int db = 0; db < NDB; ++db) o[db] *= alpha;
                 m_run = grow ? mloc : m_run;
             }
-            const float mc = m_run == -INFINITY ? 0.f : kPBits - m_run;
+            const float mc = m_run == -INFINITY ? 0.f : -m_run;
             // row sum as four independent partial chains
             float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const float e = fast_exp2(fmaf(s[kb][r], cs, mc));
+                    const float e = fast_exp2(fmaf(s[kb][r], p.c, mc));
                     s[kb][r] = e;
                     ls[r & 3] += e;
                 }
@@ -326,30 +277,22 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
 #pragma unroll
                 for (int mm = 0; mm < 2; ++mm) {
                     const f32x16& e = s[kb];
-                    const Half2x8 pb =
-                        split2(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
-                               f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]}, 1.f);
+                    const Bf3x8 pb = split3(f32x4{e[8 * mm], e[8 * mm + 1], e[8 * mm + 2], e[8 * mm + 3]},
+                                            f32x4{e[8 * mm + 4], e[8 * mm + 5], e[8 * mm + 6], e[8 * mm + 7]});
 #pragma unroll
                     for (int db = 0; db < NDB; ++db) {
-                        Half2x8 a;
+                        Bf3x8 a;
                         a.h = Vc[0][4 * kb + 2 * mm + g][db * 32 + l32];
-                        a.l = Vc[1][4 * kb + 2 * mm + g][db * 32 + l32];
-                        o[db] = mfma_split(a, pb, o[db]);
+                        a.m = Vc[1][4 * kb + 2 * mm + g][db * 32 + l32];
+                        a.l = Vc[2][4 * kb + 2 * mm + g][db * 32 + l32];
+                        o[db] = mfma_split3(a, pb, o[db]);
                     }
                 }
         }
-        if (nv != kv_cls) {  // O is kept in units of V's scale
-            const float f = class_scale(nv) * class_inv(kv_cls);
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) o[db] *= f;
-        }
-        kk_cls = nk;
-        kv_cls = nv;
         if constexpr (BUF)
-            sstore(nxt, Ks0, Vt0, nk, nv);
+            sstore(nxt, Ks0, Vt0);
         else
-            sstore(nxt, Ks1, Vt1, nk, nv);
-        need_classes(far, t & 1);
+            sstore(nxt, Ks1, Vt1);
         __syncthreads();
     };
     using B0 = std::integral_constant<int, 0>;
@@ -358,10 +301,9 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
         step(t, B0{}, rb, ra);
         if (t + 1 < n_tiles) step(t + 1, B1{}, ra, rb);
     }
-    float o_unit = class_inv(kv_cls);  // the accumulators' unit over 2^kPBits
 
     // ---- non-finite inputs ------------------------------------------------------
-    // An infinity in q, k or v (or a value past the largest bf16) is NaN in its
+    // An infinity in q, k or v, or a value past the largest bf16, is NaN in its
     // split parts, where the fp32 formula may still be finite or infinite (a
     // score of -inf is a probability of 0).  A wave whose sums are not finite
     // recomputes its rows from memory in plain fp32, one key at a time.
@@ -373,7 +315,6 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
     if (__any(chk != 0.f)) {
         m_run = -INFINITY;
         l_run = 0.f;
-        o_unit = 1.f;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
         const int j_end = qrow < p.Tq ? min(n_tiles * BN, p.causal ? min(p.Tk, qrow + p.off + 1) : p.Tk) : 0;
@@ -388,7 +329,7 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
             const float mn = fmaxf(m_run, s);
             const float mc = mn == -INFINITY ? 0.f : mn;
             const float alpha = m_run == -INFINITY ? 0.f : fast_exp2(m_run - mc);
-            const float e = fast_exp2(s - mc + kPBits);
+            const float e = fast_exp2(s - mc);
             m_run = mn;
             l_run = fmaf(l_run, alpha, g == 0 ? e : 0.f);
             const float* vp = V + (int64_t)j * p.sv.t + 4 * g;
@@ -412,7 +353,7 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     st4(po + db * 32 + 8 * j + 4 * g,
-                        f32x4{o[db][4 * j + 0], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]} * o_unit);
+                        f32x4{o[db][4 * j + 0], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]});
             if (g == 0) {
                 float* pml = p.part + (int64_t)p.n_slots * BH * BM * D + (((int64_t)slot * BH + bh) * BM + r) * 2;
                 pml[0] = m_run;
@@ -421,7 +362,7 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
         }
         return;
     }
-    const float inv = o_unit / l_tot;
+    const float inv = 1.f / l_tot;
     if (qrow < p.Tq) {
         float* dst = O + (int64_t)qrow * p.so.t;
 #pragma unroll
@@ -435,7 +376,7 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
                 val[3] = o[db][4 * j + 3] * inv;
                 st4(dst + db * 32 + 8 * j + 4 * g, val);
             }
-        if (g == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] = fmaf(m_run, kLn2, logf(l_tot * kPInv));
+        if (g == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] = fmaf(m_run, kLn2, logf(l_tot));
     }
 }
 
@@ -481,7 +422,7 @@ __global__ __launch_bounds__(256) void attn_fwd_merge_kernel(FwdParams p) {
     E* dst = (E*)p.o + b * p.so.b + h * p.so.h + (int64_t)qrow * p.so.t + 4 * c4;
     st4(dst, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
     if (c4 == 0 && p.lse) p.lse[(int64_t)bh * p.Tq + qrow] =
-            sizeof(E) == 4 ? fmaf(M, kLn2, logf(L * kPInv)) : M * p.scale + logf(L);
+            sizeof(E) == 4 ? fmaf(M, kLn2, logf(L)) : M * p.scale + logf(L);
 }
 
 template <int D, typename E>

@@ -133,16 +133,11 @@ int inf_get_deterministic(void) { return g_deterministic.load(); }
 namespace {
 
 // INF_OK, or INF_ERR_HIP when an earlier call left a HIP error pending.
-size_t amax_bytes(size_t bh, int Tq, int D) {  // the heads' maxima (fp32)
-    return round_up(bh * inf::bwd_amax_blocks(Tq, D) * 2 * sizeof(float));
-}
-
 int bwd_workspace_bytes(int det, int B, int H, int Tq, int Tk, int D, inf_dtype dt, size_t* out) {
     const size_t bh = (size_t)B * H;
     size_t n = 2 * round_up(bh * Tq * sizeof(float));  // delta and its low part (short rows)
     if (dt == INF_BF16 && !dq_from_pass(det, B, H, Tq, Tk, D, dt))
         n += round_up(bh * Tq * (size_t)D * sizeof(float));  // dQ accumulator
-    if (dt == INF_F32) n += amax_bytes(bh, Tq, D);
     inf::BwdPlan plan;                                        // causal split plan
     if (inf::bwd_plan(B, H, Tq, Tk, D, 1, dt == INF_BF16, &plan)) return INF_ERR_HIP;
     *out = n + round_up(inf::bwd_split_workspace_bytes(plan, B, H, D));
@@ -252,8 +247,6 @@ int inf_attn_bwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     } else {
         p.dq_acc = static_cast<float*>(dq);
         p.sacc = view(sdq);
-        p.amax = reinterpret_cast<float*>(ws + 2 * round_up(bh * Tq * sizeof(float)));
-        p.n_amax = inf::bwd_amax_blocks(Tq, D);
     }
     p.B = B; p.H = H; p.Tq = Tq; p.Tk = Tk; p.D = D;
     p.causal = causal ? 1 : 0;
@@ -272,7 +265,6 @@ int inf_attn_bwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     if (plan.n_groups) {
         size_t offset = 2 * round_up(bh * Tq * sizeof(float));
         if (dt == INF_BF16 && !p.dq_direct) offset += round_up(bh * Tq * (size_t)D * sizeof(float));
-        if (dt == INF_F32) offset += amax_bytes(bh, Tq, D);
         const size_t part_bytes = (size_t)plan.n_slots * bh * 2 * (size_t)D * plan.bk * sizeof(float);
         p.part = reinterpret_cast<float*>(ws + offset);
         p.counters = reinterpret_cast<unsigned*>(ws + offset + part_bytes);

@@ -19,6 +19,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -120,6 +121,84 @@ struct BF16 {
 
 // Load 4 consecutive elements as fp32 (16-byte load for fp32, 8-byte for bf16).
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+// ---- fp32 products on the bf16 matrix cores -----------------------------------
+// An fp32 value as the sum of three bf16 ones, h = bf16(x), m = bf16(x - h), l =
+// x - h - m.  Rounding to nearest leaves 16 and then 8 bits, so h + m + l is x
+// exactly, for every |x| from 2^-109 to the largest bf16 (2^-134 off at most below
+// that; bf16 has fp32's exponents and its MFMAs keep subnormals).  So there is no
+// scale to agree on and a value's neighbours don't matter.  A product of two such
+// values is the six part products l h, h l, m m, m h, h m and h h, each exact in
+// fp32; the ones left out are below 2^-25 of it.  bf16 MFMAs run 16 times as fast
+// as fp32 ones, so a product takes 6/16 of the fp32 matrix time, and an MFMA rounds
+// once per 16 terms where the fp32 instruction rounds every one or two.  (Sums of
+// low-precision parts as in Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", 2019.)
+// The remainders come from v_dot2c_f32_bf16 on the packed pair, h * -1 + 0 * h' + x
+// (exact): 3.5 instructions per value, 5.5 if the pair is unpacked first.
+// An infinity or NaN, or a value past the largest bf16, makes its m and l parts NaN
+// and so every product of it; by the term 0 * h' also those of the value beside it,
+// unless the pair is unpacked (APART: where that value belongs to other results).
+struct Bf3x8 {
+    bf16x8 h, m, l;
+};
+__device__ __forceinline__ bf16x2 split_pick(bool high) {  // {0, -1} or {-1, 0}
+    // (in a register: an inline constant -1.0 would select the other half)
+    uint32_t c = high ? 0xBF800000u : 0x0000BF80u;
+    asm("" : "+s"(c));
+    return __builtin_bit_cast(bf16x2, c);
+}
+template <bool APART = false>
+__device__ __forceinline__ Bf3x8 split3(f32x4 a, f32x4 b) {
+    const bf16x2 lo = split_pick(false), hi = split_pick(true);
+    Bf3x8 r;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        float x0 = i < 4 ? a[i & 3] : b[i & 3], x1 = i < 4 ? a[(i + 1) & 3] : b[(i + 1) & 3];
+        auto part = [&](bf16x8& dst) {
+            const bf16x2 h = {(__bf16)x0, (__bf16)x1};
+            dst[i] = h[0];
+            dst[i + 1] = h[1];
+            if constexpr (APART) {
+                x0 -= (float)h[0];
+                x1 -= (float)h[1];
+            } else {
+                x0 = __builtin_amdgcn_fdot2_f32_bf16(h, lo, x0, false);
+                x1 = __builtin_amdgcn_fdot2_f32_bf16(h, hi, x1, false);
+            }
+        };
+        part(r.h);
+        part(r.m);
+        r.l[i] = (__bf16)x0;
+        r.l[i + 1] = (__bf16)x1;
+    }
+    return r;
+}
+// c += a b of two split operands, the small part products first.
+__device__ __forceinline__ f32x16 mfma_split3(const Bf3x8& a, const Bf3x8& b, f32x16 c) {
+    c = mfma32x32x16bf16(a.l, b.h, c);
+    c = mfma32x32x16bf16(a.h, b.l, c);
+    c = mfma32x32x16bf16(a.m, b.m, c);
+    c = mfma32x32x16bf16(a.m, b.h, c);
+    c = mfma32x32x16bf16(a.h, b.m, c);
+    return mfma32x32x16bf16(a.h, b.h, c);
+}
+// The same with the small part products in a sum of their own, which takes their
+// roundings away from the result's last bits.  SWAP exchanges the operands' roles in
+// the order, so that a product with swapped operands is formed to the same bits.
+struct Split3Sum {
+    f32x16 hi, lo;
+    __device__ __forceinline__ f32x16 sum() const { return hi + lo; }
+};
+template <bool SWAP = false>
+__device__ __forceinline__ void mfma_split3(const Bf3x8& a, const Bf3x8& b, Split3Sum& c) {
+    c.lo = SWAP ? mfma32x32x16bf16(a.h, b.l, c.lo) : mfma32x32x16bf16(a.l, b.h, c.lo);
+    c.hi = mfma32x32x16bf16(a.h, b.h, c.hi);
+    c.lo = SWAP ? mfma32x32x16bf16(a.l, b.h, c.lo) : mfma32x32x16bf16(a.h, b.l, c.lo);
+    c.lo = mfma32x32x16bf16(a.m, b.m, c.lo);
+    c.lo = SWAP ? mfma32x32x16bf16(a.h, b.m, c.lo) : mfma32x32x16bf16(a.m, b.h, c.lo);
+    c.lo = SWAP ? mfma32x32x16bf16(a.m, b.h, c.lo) : mfma32x32x16bf16(a.h, b.m, c.lo);
+}
 
 // ---- fp32 products on the fp16 matrix cores -----------------------------------
 // An fp32 value times a power of two as the sum of two fp16 ones, h = fp16(x),

@@ -100,8 +100,6 @@ struct BwdParams {
     int B, H, Tq, Tk, D;
     int causal, off;
     float scale, c;
-    float* amax;          // fp32: workspace, [B*H, n_amax, 2] largest |q| and |dO| of bwd_pre's workgroups
-    int n_amax;
     int n_kblocks;
     int keys_per_wg;
     int dq_direct;          // bf16: dQ from the query-major pass (no accumulator, no atomics)
@@ -351,8 +349,6 @@ inline int bwd_keys_per_wg(int bf16, int D, int64_t BH, int Tq, int Tk) {
     const int64_t wgs = BH * ((Tk + 127) / 128);
     return Tk <= 128 || (wgs <= 256 && wgs * ((Tq + 31) / 32) < 4096) ? 128 : 256;
 }
-// bwd_pre's workgroups per head, fp32 (256 threads, 4 elements each).
-inline int bwd_amax_blocks(int Tq, int D) { return (Tq + 1024 / D - 1) / (1024 / D); }
 constexpr int kBwdBQ = 32;       // query rows per backward inner step
 // Leading query rows whose visible keys all lie in key block 0 (keys_per_wg
 // keys): their softmax-backward row dot is formed inside the block-0

@@ -1,12 +1,13 @@
-"""The fp32 attention kernels' products on two fp16 parts per operand: magnitudes far from 1 and
-far apart, non-finite inputs, and the sizes where a tile, a key block or the choice between the
-wide and the narrow backward ends, against 64-bit torch.
+"""The fp32 attention kernels' products on three bf16 parts per operand: magnitudes far from 1 and
+far apart, within a tile, a row or a column, blocks of zeros, non-finite inputs, and the sizes where
+a tile, a key block or the choice between the wide and the narrow backward ends, against 64-bit torch.
 
-Bar: a split operand is within 2^-22.7 of its value, so a score is within about D 2^-21.7 max|q k|
-in the worst case and sqrt(D) times that for terms of either sign, below 3e-6 of the largest score
-(at most ~8 here, so a probability is within ~3e-6 absolutely); sums over keys and queries add
-rounding of either sign.  1e-5 of a tensor's norm is several times what such errors add up to
-(measured: 2e-7 to 7e-7), and a part dropped or a scale missed shows at 1e-4 or more."""
+Bar: operands are held exactly and a product of them is within 2^-25, so a score carries the fp32
+rounding of its sum, below 2^-22 of the largest score's terms (at most ~8 here, so a probability is
+within ~2e-6 absolutely); sums over keys and queries add rounding of either sign.  1e-5 of a tensor's
+norm is several times what such errors add up to (measured: 2e-7 to 7e-7), and a part dropped shows
+at 1e-4 or more.
+"""
 import math
 
 import pytest
@@ -152,3 +153,121 @@ def test_nonfinite_gradient_stays_local(ia):
     keep = [i for i in range(300) if i != 100]
     assert rel(dq[:, :, keep], ref[0][:, :, keep].double()) <= BAR
     assert not torch.isfinite(dq[:, :, 100]).all() and not torch.isfinite(dv[:, :, :101, 5]).any()
+
+
+def row_err(x, r, skip=None):
+    """The largest relative error of a row (2-norms over the last dim; rows of zeros must be zeros)."""
+    d, n = (x.double() - r).norm(dim=-1), r.norm(dim=-1)
+    e = torch.where(n > 0, d / n.clamp(min=1e-300), d)
+    if skip is not None:
+        e = e[..., skip:]
+    return e.max().item() if e.isfinite().all() else math.inf
+
+
+def both_modes(ia, q, k, v, do, scale, causal=True):
+    for det in (False, True):
+        ia.set_deterministic(det)
+        try:
+            yield det, run(ia, q, k, v, do, scale, causal)
+        finally:
+            ia.set_deterministic(False)
+
+
+# Blocks of zero keys (padding) where a wave's, a pair's or a tile's keys are: an all-zero operand beside
+# ordinary ones.  (8, 16): the wide key blocks; D = 64 and 32 have 64 keys to a pair there, else 32.
+@pytest.mark.parametrize("B,H", [(1, 3), (8, 16)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("what", ["k", "v", "kv"])
+def test_zero_key_blocks(ia, B, H, D, causal, what):
+    c = 1 / math.sqrt(D)
+    for a, n in ((0, 64), (64, 64), (32, 32), (96, 32), (128, 128), (192, 108)):
+        print(f"[case] zero {what} keys {a}..{a + n - 1} B{B} H{H} D{D} causal={causal}", flush=True)
+        q, k, v, do = make(B, H, 300, 300, D, seed=5)
+        for t, name in ((k, "k"), (v, "v")):
+            if name in what:
+                t[:, :, a:a + n] = 0
+        want = exact(q, k, v, do, c, causal)
+        for det, got in both_modes(ia, q, k, v, do, c, causal):
+            for n_, x, r in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+                assert torch.isfinite(x).all() and rel(x, r) <= BAR, (n_, det)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_probabilities_that_underflow(ia, D):
+    """Scores hundreds apart: whole blocks of keys have probabilities of 0 or next to it for every query.
+    A score of 300 is rounded by up to 2^-16, which moves its probability by as much: 1e-4."""
+    q, k, v, do = make(1, 3, 300, 300, D, seed=6, qs=8.0, ks=8.0)
+    c = 1 / math.sqrt(D)
+    q[..., 0] = q[..., 0].abs() + 8
+    k[:, :, 64:128, 0] -= 300 * math.sqrt(D) / 8
+    want = exact(q, k, v, do, c)
+    for det, got in both_modes(ia, q, k, v, do, c):
+        for n_, x, r in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+            assert torch.isfinite(x).all() and rel(x, r) <= 1e-4, (n_, det)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("factor", [2.0**20, 1e30])
+def test_a_key_that_is_hidden(ia, D, factor):
+    """A key 2^20 or 1e30 times as large as the others, in k, in v and in both, changes nothing for the
+    rows that the mask keeps from it: every row by itself, forward and backward."""
+    T, j = 500, 300
+    c = 1 / math.sqrt(D)
+    q, k, v, do = make(1, 2, T, T, D, seed=7)
+    do[:, :, j:] = 0  # the rows that see the key send no gradient back
+    want = exact(q, k, v, do, c)
+    for kf, vf in ((factor, 1.0), (1.0, factor), (factor, factor)):
+        k2, v2 = k.clone(), v.clone()
+        k2[:, :, j] *= kf
+        v2[:, :, j] *= vf
+        o, lse = ia.attn_fwd(q, k2, v2, scale=c)
+        assert row_err(o[:, :, :j], want[0][:, :, :j]) <= BAR, (kf, vf)
+        assert rel(lse[:, :, :j], want[1][:, :, :j]) <= BAR
+        if factor > 1e9:
+            continue  # past the largest float in the rows that see the key
+        for det, got in both_modes(ia, q, k2, v2, do, c):
+            assert row_err(got[2][:, :, 1:j], want[2][:, :, 1:j]) <= 3 * BAR, (kf, vf, det)
+            for x, r in zip(got[3:], want[3:]):
+                assert row_err(x[:, :, :j], r[:, :, :j]) <= 3 * BAR, (kf, vf, det)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_rows_and_columns_of_unlike_size(ia, D):
+    """Rows and columns far below the largest of their tensor keep their own precision: the first value
+    rows, single columns of v and dO, single rows of q, dO rows that alone see the last keys, q and k
+    scaled against each other by column.  Bar: fp32 rounding of scores of about 10 to 30 and of the
+    differences that make up a row of dS: 3e-5 of a row."""
+    T, c, bar = 400, 1 / math.sqrt(D), 3e-5
+    print(f"[case] unlike rows and columns D{D}", flush=True)
+    q, k, v, do = make(1, 2, T, T, D, seed=8)
+    small = v.clone()
+    small[:, :, :3] *= 1e-9
+    o, _ = ia.attn_fwd(q, k, small, scale=c)
+    assert row_err(o[:, :, :3], exact(q, k, small, do, c)[0][:, :, :3]) <= 2e-6
+    # a large column of v: the others, each by itself
+    wide = v.clone()
+    wide[..., 5] *= 2.0**24
+    o, _ = ia.attn_fwd(q, k, wide, scale=c)
+    e = exact(q, k, wide, do, c)[0]
+    assert row_err(o.transpose(2, 3), e.transpose(2, 3)) <= 2e-6
+    # columns of q against those of k (the scores stay)
+    s = torch.exp2(torch.linspace(-15, 15, D, device="cuda"))[torch.randperm(D, generator=torch.Generator().manual_seed(9)).cuda()]
+    cases = {"columns": (q * s, k / s, v, do)}
+    # one row of q 1e6 times the others, where it sees its own key only at the end of a long row
+    ql = q.clone()
+    ql[:, :, 37] *= 1e6
+    cases["q row"] = (ql, k, v, do)
+    # the last rows' gradients 1e9 times smaller: the last keys are seen by them alone
+    dl = do.clone()
+    dl[:, :, 200:] *= 1e-9
+    cases["dO rows"] = (q, k, v, dl)
+    for name, args in cases.items():
+        want = exact(*args, c)
+        for det, got in both_modes(ia, *args, c):
+            keep = [i for i in range(1, T) if not (name == "q row" and i == 37)]
+            assert row_err(got[2][:, :, keep], want[2][:, :, keep]) <= bar, (name, det)
+            lo = 38 if name == "q row" else 0
+            # (the last key is seen by the last row alone: its dK row is one cancelling difference)
+            assert row_err(got[3][:, :, lo:T - 8], want[3][:, :, lo:T - 8]) <= bar, (name, det)
+            assert row_err(got[4][:, :, lo:], want[4][:, :, lo:]) <= bar, (name, det)
