@@ -276,9 +276,10 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     //     reads dQ; xr[..][0] is the l part in S's layout and xr[..][1], in entry
     //     step, the one in dQ's.
     f32x4 xr[NKB][NKK][2];
+    bool k_past = false;
+    const float* X = role ? (const float*)p.v + b * p.sv.b + h * p.sv.h : (const float*)p.k + b * p.sk.b + h * p.sk.h;
+    const int64_t xt = role ? p.sv.t : p.sk.t;
     {
-        const float* X = role ? (const float*)p.v + b * p.sv.b + h * p.sv.h : (const float*)p.k + b * p.sk.b + h * p.sk.h;
-        const int64_t xt = role ? p.sv.t : p.sk.t;
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) {
             const int key = k0p + kb * 32 + l32;
@@ -293,6 +294,8 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
         }
         gload(q_begin, p.Tq);
         if (role == 0) {
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) k_past |= any_past_bf16(xr[kb]);
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
@@ -339,8 +342,10 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
     };
     // The S (role 0) or dP (role 1) chains of the staged tile and the pair's keys;
     // SWAP: queries as the MFMA's rows (the main loop), else keys (the short rows),
-    // in the same order, to the same bits.
-    auto scores = [&](f32x16 (&s)[NKB], auto swap_c) {
+    // in the same order, to the same bits.  Scores of keys with an infinity are formed
+    // from memory in plain fp32: a key that scores -inf has probability 0, and
+    // dK and dV of 0.  (Infinities in q, v and dO leave nothing finite that they meet.)
+    auto scores = [&](f32x16 (&s)[NKB], int q0, auto swap_c) {
         constexpr bool SWAP = decltype(swap_c)::value;
         fresh_xr();
         fresh_off();
@@ -353,7 +358,15 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
         };
         // a step's LDS operands are read while the step before runs
         constexpr int N = NKB * NKK;
-        if (role == 0) {
+        if (k_past) {  // (role 0)
+            const float* yp = q0 + l32 < p.Tq ? Q + (int64_t)(q0 + l32) * p.sq.t : nullptr;
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) {
+                const int key = k0p + 32 * kb + l32;
+                const float* xp = key < p.Tk ? X + (int64_t)key * xt : nullptr;
+                s[kb] = SWAP ? dot_rows_f32<D>(yp, xp, g) : dot_rows_f32<D>(xp, yp, g);
+            }
+        } else if (role == 0) {
             Bf3x8 y[2];
             y[0] = T::row_frag(lds, row_off, 0, PART);
             bf16x8 k[2][2];
@@ -429,7 +442,7 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
             f32x16 st[NKB];
             f32x4* X = reinterpret_cast<f32x4*>(lds + X_OFF + pr * XPAIR);
             if (active) {
-                scores(st, std::false_type{});
+                scores(st, q0, std::false_type{});
                 if (role == 0) {
                     const int qi = q0 + l32;
                     const float L = lse_s[l32];
@@ -496,7 +509,7 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
         f32x4* X = reinterpret_cast<f32x4*>(lds + X_OFF + pr * XPAIR);
         f32x16 s[NKB];
         if (active) {
-            scores(s, std::true_type{});
+            scores(s, q0, std::true_type{});
             // reg 4j + cc of s[kb]: query row 8 j + 4 g + cc of the tile, key 32 kb + l32 of the pair
             if (role == 0) {
                 // Only tiles that cross the causal diagonal or the end of the
@@ -850,6 +863,9 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
                 mfma_split3(T::row_frag(lds + V_OFF + 3 * buf * PART, T::row_lane(lane), kk, PART), split3(dr[kk][0], dr[kk][1]), dps);
             }
             f32x16 s = ss.sum(), dp = dps.sum();
+            if (any_nonfinite(s))  // (as in the main kernel)
+                s = dot_rows_f32<D>(k0 + l32 < p.Tk ? K + (int64_t)(k0 + l32) * p.sk.t : nullptr,
+                                    qrow < p.Tq ? Q + (int64_t)qrow * p.sq.t : nullptr, g);
             // reg r: key k0 + 8 (r / 4) + 4 g + r % 4 of query qrow
             const bool need_mask = (k0 + BN > p.Tk) || (qtile * BM + BM > p.Tq) || (p.causal && (k0 + BN - 1 > q0w + p.off));
             const int lim = p.causal ? min(p.Tk - 1, qrow + p.off) : p.Tk - 1;

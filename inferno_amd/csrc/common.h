@@ -3,6 +3,8 @@
 // Wave64 throughout.  MFMA operand/result layouts used by every kernel here
 // (lane l = 0..63, l32 = l % 32, g = l / 32; checked on the GPU by
 // tests/test_gpu_parity.py through the attention results themselves):
+//   v_mfma_f32_32x32x2_f32          A: lane gives A[l32][g]   B: lane gives B[g][l32]
+//                                   D: as below
 //   v_mfma_f32_32x32x16_{bf16,f16}  A: lane gives A[l32][8*g .. 8*g+7]  B: B[8*g .. 8*g+7][l32]
 //                                   D: reg r holds D[8*(r/4) + 4*g + r%4][l32]
 // The reduction index of an MFMA may be permuted freely as long as A and B
@@ -31,6 +33,9 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
+__device__ __forceinline__ f32x16 mfma32x32x2(float a, float b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
 __device__ __forceinline__ f32x16 mfma32x32x16bf16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -198,6 +203,46 @@ __device__ __forceinline__ void mfma_split3(const Bf3x8& a, const Bf3x8& b, Spli
     c.lo = mfma32x32x16bf16(a.m, b.m, c.lo);
     c.lo = SWAP ? mfma32x32x16bf16(a.h, b.m, c.lo) : mfma32x32x16bf16(a.m, b.h, c.lo);
     c.lo = SWAP ? mfma32x32x16bf16(a.m, b.h, c.lo) : mfma32x32x16bf16(a.h, b.m, c.lo);
+}
+
+// Whether one of the wave's values is an infinity or past the largest bf16.  (A NaN
+// needs no care: its products are NaN either way.)
+template <int N>
+__device__ __forceinline__ bool any_past_bf16(const f32x4 (&v)[N][2]) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(fmaxf(m, fabsf(v[i][0][e])), fabsf(v[i][1][e]));
+    return __any(m > 3.3895313892515355e38f);  // (2 - 2^-7) 2^127
+}
+// The fp32 formula itself, for operands that the parts can't hold: the products of 32 rows with 32 rows of D floats on
+// the fp32 matrix cores, straight from memory.  a, b: this lane's rows (l32), or null
+// for zeros; result reg r: row 8 (r / 4) + 4 g + r % 4 of A's, column l32 of B's.
+// U: 8-column steps whose loads are in flight together (8 registers each).
+template <int D, int U = 1>
+__device__ __forceinline__ f32x16 dot_rows_f32(const float* a, const float* b, int g) {
+    f32x16 c = {};
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int d = 0; d < D; d += 8 * U) {
+        f32x4 x[U], y[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) x[i] = a ? *reinterpret_cast<const f32x4*>(a + d + 8 * i + 4 * g) : zero;
+#pragma unroll
+        for (int i = 0; i < U; ++i) y[i] = b ? *reinterpret_cast<const f32x4*>(b + d + 8 * i + 4 * g) : zero;
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c = mfma32x32x2(x[i][e], y[i][e], c);
+    }
+    return c;
+}
+__device__ __forceinline__ bool any_nonfinite(const f32x16& v) {  // in the wave
+    float chk = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) chk = fmaf(v[r], 0.f, chk);
+    return __any(chk != 0.f);
 }
 
 // ---- fp32 products on the fp16 matrix cores -----------------------------------

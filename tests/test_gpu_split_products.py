@@ -271,3 +271,55 @@ def test_rows_and_columns_of_unlike_size(ia, D):
             # (the last key is seen by the last row alone: its dK row is one cancelling difference)
             assert row_err(got[3][:, :, lo:T - 8], want[3][:, :, lo:T - 8]) <= bar, (name, det)
             assert row_err(got[4][:, :, lo:], want[4][:, :, lo:]) <= bar, (name, det)
+
+
+@pytest.mark.parametrize("B,H", [(1, 3), (8, 16)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_a_key_that_scores_minus_infinity_backward(ia, B, H, D):
+    """Its probability is 0, so its dK and dV are 0 and nothing else changes: only the column of dQ
+    that multiplies the infinity is 0 * inf.  Among the first keys (whose rows have their own row
+    dots) and far from them; every query sees it or not."""
+    c = 1 / math.sqrt(D)
+    for causal in (True, False):
+        for j in (5, 40, 250):
+            print(f"[case] -inf key {j} B{B} H{H} D{D} causal={causal}", flush=True)
+            q, k, v, do = make(B, H, 300, 300, D, seed=10)
+            q[..., 0] = q[..., 0].abs() + 0.1
+            k2 = k.clone()
+            k2[:, :, j, 0] = -math.inf
+            keep = [i for i in range(300) if i != j]
+            # without the key: causal rows before it see the same keys, rows behind it one less
+            mask = torch.ones(300, 300, dtype=torch.bool, device="cuda").triu(1) if causal else torch.zeros(
+                300, 300, dtype=torch.bool, device="cuda")
+            mask[:, j] = True
+            qd, kd, vd = (x.double().requires_grad_() for x in (q, k, v))
+            s = torch.matmul(qd, kd.transpose(2, 3).contiguous()) * c
+            s = s.masked_fill(mask, -math.inf)
+            o = torch.matmul(torch.softmax(s, -1), vd)
+            o.backward(do.double())
+            for det, got in both_modes(ia, q, k2, v, do, c, causal):
+                assert rel(got[0], o.detach()) <= BAR, det
+                assert (got[3][:, :, j] == 0).all() and (got[4][:, :, j] == 0).all(), det
+                assert rel(got[3][:, :, keep], kd.grad[:, :, keep]) <= BAR, det
+                assert rel(got[4][:, :, keep], vd.grad[:, :, keep]) <= BAR, det
+                assert rel(got[2][..., 1:], qd.grad[..., 1:]) <= BAR, det
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,Tq,Tk,causal", [(1, 2, 1100, 1100, True), (2, 3, 130, 700, False), (1, 2, 100, 1030, True)])
+def test_rows_beside_nonfinite_keys(ia, B, H, Tq, Tk, causal, D):
+    """Rows that are formed again in plain fp32 (a key at -inf that all of them see, before many others):
+    whole blocks of visible keys, the diagonal's, the ragged end, chunks of a split key range."""
+    c = 1 / math.sqrt(D)
+    q, k, v, _ = make(B, H, Tq, Tk, D, seed=11)
+    q[..., 0] = q[..., 0].abs() + 0.1
+    k2 = k.clone()
+    k2[:, :, 17, 0] = -math.inf
+    mask = torch.ones(Tq, Tk, dtype=torch.bool, device="cuda").triu(1 + Tk - Tq) if causal else torch.zeros(
+        Tq, Tk, dtype=torch.bool, device="cuda")
+    mask[:, 17] = True
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * c
+    s = s.masked_fill(mask, -math.inf)
+    o, lse = ia.attn_fwd(q, k2, v, causal=causal, scale=c)
+    assert row_err(o, torch.matmul(torch.softmax(s, -1), v.double())) <= BAR
+    assert rel(lse, torch.logsumexp(s, -1)) <= BAR
