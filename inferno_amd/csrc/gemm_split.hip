@@ -40,13 +40,14 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_split_rule.h"
 #include "kernels.h"
 
 namespace inf {
 
 namespace {
 
-constexpr int kBM = 256, kBN = 128, kBK = 32, kNT = 512;
+constexpr int kBM = kSplitBM, kBN = kSplitBN, kBK = kSplitBK, kNT = 512;
 constexpr int kKG = kBK / 8;  // 8-k units per row and step
 
 struct GemmSplitParams {
@@ -363,11 +364,10 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmSplitParams 
     }
 }
 
-// Whether the kernel takes the problem: fp32; a K-contiguous operand is read 8
-// elements at a time in halves (K % 4, 16-byte rows); 32-bit offsets inside a tile's panel;
-// alpha = 0 must not read operands that may hold infinities.
-static bool split_takes(const GemmArgs& g) {
-    if (g.bf16 || g.alpha == 0.f || (g.K % 4 != 0 && !(g.ta && !g.tb)) || g.lda > (1 << 20) || g.ldb > (1 << 20)) return false;
+// Whether the kernel can read the operands: a K-contiguous one 8 elements at a time in
+// halves (16-byte rows).  (alpha = 0 must not read operands that may hold infinities.)
+static bool split_reads(const GemmArgs& g) {
+    if (g.bf16 || g.alpha == 0.f) return false;
     auto rows16 = [](const void* p, int64_t ld, int64_t stride) {
         return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && stride % 4 == 0;
     };
@@ -378,7 +378,10 @@ static bool split_takes(const GemmArgs& g) {
 
 int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
     *taken = false;
-    if (!split_takes(g)) return 0;
+    if (!split_reads(g)) return 0;
+    const bool ws_ok = reinterpret_cast<uintptr_t>(g.ws) % 16 == 0;
+    const int ks = gemm_split_ranges(g.ta, g.tb, g.M, g.N, g.K, g.batch, g.lda, g.ldb, ws_ok ? g.ws_bytes : 0);
+    if (!ks) return 0;
     GemmSplitParams p{};
     p.A = (const float*)g.A;
     p.B = (const float*)g.B;
@@ -397,33 +400,8 @@ int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken) {
     p.beta = g.beta;
     p.tiles_m = (int)((g.M + kBM - 1) / kBM);
     p.tiles_n = (int)((g.N + kBN - 1) / kBN);
-    // The number of K ranges: the cheapest under a model (microseconds) fitted to
-    // measured shapes: the longest chain of K steps on a CU (1.65 a step, 8 steps
-    // for a workgroup's start and end) or, where the device is full and its clock
-    // falls with the load, the steps over the rate that large products reach;
-    // partials pass through memory once more.
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * g.batch;
     const int nk = (p.K + kBK - 1) / kBK;
-    if (tiles > (1 << 24)) return 0;  // 32-bit work counts
-    double best = 1e30;
-    int ks = 1;
-    for (int c = 1; c <= 8; ++c) {
-        if (c > 1 && (g.batch > 1 || nk / c < 8 || (size_t)c * g.M * g.N * sizeof(float) > g.ws_bytes ||
-                      reinterpret_cast<uintptr_t>(g.ws) % 16))
-            break;
-        const double wgs = (double)(tiles * c), steps = (nk + c - 1) / c + 8;
-        double cost = std::max(steps * 1.65 * std::ceil(wgs / 256), wgs * steps / 146.0);
-        if (c > 1) cost += 4.0 + (double)(c + 1) * g.M * g.N * 4 / 4e6;
-        if (cost < best) {
-            best = cost;
-            ks = c;
-        }
-    }
-    // The vendor library's fp32 kernels (about 142 TFLOP/s, 118 at ragged sizes, and
-    // better split for small problems) where the model says that they are no
-    // slower: 1024^3 19 us there and 35 here, 1536^3 62 and 47, M = 32 9-18 and 25.
-    const bool whole = g.M % 128 == 0 && g.N % 128 == 0 && g.K % 32 == 0;
-    if (best > 2.0 * g.M * g.N * g.K * g.batch / (whole ? 142e6 : 118e6) + 8.0) return 0;
     p.kchunk = (nk + ks - 1) / ks * kBK;
     p.ksplit = (p.K + p.kchunk - 1) / p.kchunk;
     p.part = (float*)g.ws;
