@@ -275,17 +275,18 @@ int inf_copy_strided(const void* src, const int64_t* src_strides, void* dst,
 
 enum { INF_OP_GEMM = 3, INF_OP_LAYERNORM_BWD = 4, INF_OP_COL_SUM = 5, INF_OP_CROSS_ENTROPY = 6 };
 
-/* Workspace bytes for a model op: INF_OP_GEMM (any shape), INF_OP_LAYERNORM_BWD (rows, cols = dim), INF_OP_COL_SUM (rows,
- * cols), INF_OP_CROSS_ENTROPY (rows, cols = vocab). */
+/* Workspace bytes for a model op: INF_OP_GEMM (any shape), INF_OP_LAYERNORM_BWD
+ * (rows, cols = dim), INF_OP_COL_SUM (rows, cols), INF_OP_CROSS_ENTROPY (rows,
+ * cols = vocab). */
 int inf_nn_workspace_bytes(int op, int64_t rows, int64_t cols, size_t* out_bytes);
 
 /* C[b] = alpha * op(A[b]) op(B[b]) + beta * C[b] (+ bias[n] added to every row)
  * for b < batch, row-major: op(A) is M x K (A stored M x K, or K x M when
  * trans_a), op(B) is K x N (B stored K x N, or N x K when trans_b); batch
- * strides in elements.  Large fp32 products run on the fp16 matrix cores, every
- * operand split into two fp16 parts (the accuracy of fp32 sums; a workspace too
- * small for partial sums costs speed only); the others run on hipBLASLt (fp32
- * matrix cores for fp32).
+ * strides in elements.  Large fp32 products run on the bf16 matrix cores, every
+ * operand split into three bf16 parts, which hold it exactly (the accuracy of fp32
+ * sums, for operands of any magnitude; a workspace too small for partial sums costs
+ * speed only); the others run on hipBLASLt (fp32 matrix cores for fp32).
  * Replaces cublas_mm_strided_batched_row_major and cuda_matmul
  * (src/inferno/cuda/cudamatmul.cu:120-216, 1114-1179) behind matmul
  * (src/inferno/core/ops.cpp:437-735) and Linear::forward (linear.cpp:49-54). */

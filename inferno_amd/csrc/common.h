@@ -5,7 +5,7 @@
 // tests/test_gpu_parity.py through the attention results themselves):
 //   v_mfma_f32_32x32x2_f32          A: lane gives A[l32][g]   B: lane gives B[g][l32]
 //                                   D: as below
-//   v_mfma_f32_32x32x16_{bf16,f16}  A: lane gives A[l32][8*g .. 8*g+7]  B: B[8*g .. 8*g+7][l32]
+//   v_mfma_f32_32x32x16_bf16        A: lane gives A[l32][8*g .. 8*g+7]  B: B[8*g .. 8*g+7][l32]
 //                                   D: reg r holds D[8*(r/4) + 4*g + r%4][l32]
 // The reduction index of an MFMA may be permuted freely as long as A and B
 // agree, which is how the kernels feed a result tile straight back in as the
@@ -22,9 +22,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
@@ -77,16 +74,6 @@ __device__ __forceinline__ float group_sum(float v) {
     if constexpr (W >= 8) v += dpp_mov<0x141>(v);  // row_half_mirror
     if constexpr (W >= 16) v += dpp_mov<0x140>(v); // row_mirror
     if constexpr (W >= 32) v += shfl_xor(v, 16);
-    return v;
-}
-
-template <int W>
-__device__ __forceinline__ float group_max(float v) {
-    static_assert(W == 4 || W == 8 || W == 16, "group width");
-    v = fmaxf(v, dpp_mov<0xB1>(v));
-    v = fmaxf(v, dpp_mov<0x4E>(v));
-    if constexpr (W >= 8) v = fmaxf(v, dpp_mov<0x141>(v));
-    if constexpr (W >= 16) v = fmaxf(v, dpp_mov<0x140>(v));
     return v;
 }
 
@@ -245,82 +232,6 @@ __device__ __forceinline__ bool any_nonfinite(const f32x16& v) {  // in the wave
     return __any(chk != 0.f);
 }
 
-// ---- fp32 products on the fp16 matrix cores -----------------------------------
-// An fp32 value times a power of two as the sum of two fp16 ones, h = fp16(x),
-// l = fp16(x - h): 11 + 11 significant bits and a sign, within 2^-23 |x| (2^-24.4
-// rms) of x while |x| stays between 2^-3 and 2^15, and within 2^-25 absolutely
-// below that.  A product of two such values is the three part products l h, h l
-// and h h (l l is below 2^-22 and half the time of either sign: 2^-25 rms).  fp16
-// MFMAs run 16 times as fast as fp32 ones, so a product takes 3/16 of the fp32
-// matrix time; the part products are exact in fp32 and an MFMA rounds once per 16
-// of them, where the fp32 instruction rounds every one or two, so a dot product
-// comes out closer to its 64-bit value, not further.
-// The remainder comes from v_fma_mix_f32, which reads one half of the packed
-// pair (x - h as h * -1 + x, exact): 2 instructions per value, 3 with the
-// scale.  (The compiler unpacks the pair first; x has passed at least the
-// conversion to h, so the asm never reads a result still in flight.)
-// An infinity or NaN makes a part NaN, and so every product of it.
-struct Half2x8 {
-    f16x8 h, l;
-};
-__device__ __forceinline__ Half2x8 split2(f32x4 a, f32x4 b, float scale) {
-    Half2x8 r;
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-        const float x0 = (i < 4 ? a[i & 3] : b[i & 3]) * scale, x1 = (i < 4 ? a[(i + 1) & 3] : b[(i + 1) & 3]) * scale;
-        const f16x2 h = {(_Float16)x0, (_Float16)x1};
-        r.h[i] = h[0];
-        r.h[i + 1] = h[1];
-        float d0, d1;
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(d0) : "v"(h), "v"(x0));
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d1) : "v"(h), "v"(x1));
-        r.l[i] = (_Float16)d0;
-        r.l[i + 1] = (_Float16)d1;
-    }
-    return r;
-}
-__device__ __forceinline__ f32x16 mfma32x32x16f16(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-// c += a b of two split operands, the small part products first; a's low part
-// before b's (ALO) or after, so that a product with swapped operands can be
-// formed in the same order, to the same bits.
-template <bool ALO = true>
-__device__ __forceinline__ f32x16 mfma_split(const Half2x8& a, const Half2x8& b, f32x16 c) {
-    c = ALO ? mfma32x32x16f16(a.l, b.h, c) : mfma32x32x16f16(a.h, b.l, c);
-    c = ALO ? mfma32x32x16f16(a.h, b.l, c) : mfma32x32x16f16(a.l, b.h, c);
-    return mfma32x32x16f16(a.h, b.h, c);
-}
-// Scale classes.  A block of values is scaled by a power of two that puts its
-// largest magnitude between 2^7 and 2^15: class k covers magnitudes
-// [2^(8k - 131), 2^(8k - 123)) (k = 16: 1/8 to 32), so what lies far below the
-// largest keeps an absolute error of 2^-32 of it or less.  Scaling by powers of
-// two changes no bit of a result except through that floor; classes 8 binades
-// wide keep the scale the same for all blocks of ordinary tensors.
-__device__ __forceinline__ int scale_class(float amax) {
-    return max(2, (int)(((__float_as_uint(amax) >> 23) & 0xff) + 4) >> 3);
-}
-__device__ __forceinline__ float class_limit(int k) { return __uint_as_float((uint32_t)(8 * k + 4) << 23); }  // upper end
-__device__ __forceinline__ float class_scale(int k) { return __uint_as_float((uint32_t)(265 - 8 * k) << 23); }
-__device__ __forceinline__ float class_inv(int k) { return __uint_as_float((uint32_t)(8 * k - 11) << 23); }
-// |x|, or 0 for an infinity or NaN: one such value in a block must not set the
-// block's scale (it spoils only its own products).
-__device__ __forceinline__ float finite_abs(float x) {
-    const float a = fabsf(x);
-    return a < INFINITY ? a : 0.f;
-}
-__device__ __forceinline__ float absmax8_finite(float m, f32x4 a, f32x4 b) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m = fmaxf(fmaxf(m, finite_abs(a[i])), finite_abs(b[i]));
-    return m;
-}
-__device__ __forceinline__ float absmax8(float m, f32x4 a, f32x4 b) {
-    m = fmaxf(fmaxf(m, fabsf(a[0])), fabsf(a[1]));
-    m = fmaxf(fmaxf(m, fabsf(a[2])), fabsf(a[3]));
-    m = fmaxf(fmaxf(m, fabsf(b[0])), fabsf(b[1]));
-    return fmaxf(fmaxf(m, fabsf(b[2])), fabsf(b[3]));
-}
-
 // Raw buffer resource over `bytes` bytes from `base` (gfx9 dword 3: raw
 // addressing, no swizzle).  A load whose offset falls at or past `bytes`
 // returns zeros without a memory access.  Callers pass wave-uniform values;
@@ -372,10 +283,6 @@ __device__ __forceinline__ void buffer_ld16_lds(__amdgpu_buffer_rsrc_t r, void* 
 __device__ __forceinline__ bf16x4 ds_read_tr16(const __bf16* p) {
     return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                                           (__attribute__((address_space(3))) s16x4*)(p)));
-}
-__device__ __forceinline__ f16x4 ds_read_tr16_f16(const _Float16* p) {
-    return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                         (__attribute__((address_space(3))) s16x4*)(p)));
 }
 // Resource over rows [row0, row0 + rows) of a row-major fp32 matrix with
 // row stride `st` elements and `cols` used columns (rows <= 0: empty).

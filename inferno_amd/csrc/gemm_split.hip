@@ -1,5 +1,5 @@
-// gemm_split.hip -- fp32 GEMM on the fp16 matrix cores: every operand split into
-// two fp16 parts (common.h), three MFMAs per product step, fp32 accumulators.
+// gemm_split.hip -- fp32 GEMM on the bf16 matrix cores: every operand split into
+// three bf16 parts (common.h), six MFMAs per product step, fp32 accumulators.
 //
 // Row-major C = alpha * op(A) op(B) + beta * C (+ bias per row).  One workgroup
 // = 8 waves = a 256 x 128 tile of C, each wave 64 x 64 of it (2 x 2 MFMA blocks: a
@@ -12,29 +12,29 @@
 //   K-strided operand (A transposed, or B): a thread loads 8 k of one column
 //     (eight 4-byte loads, each a run over the lanes), so the transposition costs
 //     no store.
-// Every row of A and column of B is scaled by the class of its largest magnitude
-// so far, which the threads that stage it agree on without LDS (neighbouring
-// lanes).  When a row's class grows (as a rule in the first step only), the
-// accumulators, kept in units of row times column scale, move with it.
-// The matrix cores' fp16 sums round a little towards -infinity (2e-8 of a result's
-// rms on average, which a sum over thousands of rows of C would show): half of the
-// rows and columns, by the parity of their index's bits, are negated with their
-// scale, so that half of the results are formed as their negatives and what is left
-// cancels in sums over rows or columns of C (8192 rows summed: 1.8e-6 off without,
-// 5e-7 with the vendor library's fp32 kernel, 3e-7 here).
+// The operands are taken times 2^24 and the results times 2^-48, which moves the
+// range that three bf16 parts hold exactly to all of fp32's small numbers; a sum that
+// this takes past the largest float is formed again in plain fp32 (below).
+// The matrix cores' sums round a little towards -infinity (2e-8 of a result's rms
+// on average, which a sum over thousands of rows of C would show): half of the rows
+// and columns, by the parity of their index's bits, are negated, so that half of
+// the results are formed as their negatives and what is left cancels in sums over
+// rows or columns of C.  The small part products have accumulators of their own.
 // A non-finite element makes its row's or column's results NaN; the epilogue
 // forms those again one by one in plain fp32, so infinities come out as before.
 //
 // Few tiles and a long K: the K range is split over workgroups, their partial
 // tiles go to the workspace and a second kernel sums them in order.
 //
-// Bound by the splitting VALU work and the MFMAs, which overlap only in part
-// (4096^3: matrix cores busy 42% of the cycles, VALU 44%), at a shader clock that
-// falls to 1.7-2.0 GHz with the load.  Against the vendor library's fp32 kernels
-// (us): 8192 x 3072 x 768 280 -> 174, 8192 x 768 x 3072 266 -> 152, 768 x 3072 x 8192
-// (A transposed) 291 -> 160, 4096^3 915 -> 460, 3309 x 664 x 2656 110 -> 62.  Tiles of 128 x 128 in four-wave
-// workgroups, two per CU, split a third more and took 5-8% longer except at
-// 8192 x 2304 x 768 (159 against 169).
+// Bound by the MFMAs and the splitting VALU work beside them, at a shader clock that
+// falls with the load: 4096^3 at 1.18 PFLOP/s of MFMAs, where a large library product
+// in bf16 reaches 1.25.  Against the vendor library's fp32 kernels (us): 8192 x 3072 x
+// 768 342 -> 253, 8192 x 768 x 3072 308 -> 249, 768 x 3072 x 8192 300 -> 220, 4096^3
+// 917 -> 701, 2905 x 2240 x 560 115 -> 55, 3309 x 664 x 2656 114 -> 85; the distance of
+// the MLP's outputs to 64 bits 1.7e-6 -> 4e-7.  Two fp16 parts with a scale per row
+// and column and three MFMAs took 185, 177, 159, 466, 52 and 73, but lost the bits
+// of what lies far below its row's largest (2e-3 of the result where features and
+// their weights are scaled against each other by 2^13).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -49,6 +49,12 @@ namespace {
 
 constexpr int kBM = kSplitBM, kBN = kSplitBN, kBK = kSplitBK, kNT = 512;
 constexpr int kKG = kBK / 8;  // 8-k units per row and step
+constexpr float kUp = 0x1p24f, kDown = 0x1p-48f;  // the operands' factor, and what takes it from a result
+
+// v, negated where i has an odd number of bits
+__device__ __forceinline__ float with_parity(float v, uint32_t i) {
+    return __uint_as_float(__float_as_uint(v) ^ (uint32_t)__popc(i) << 31);
+}
 
 struct GemmSplitParams {
     const float* A;
@@ -69,11 +75,9 @@ struct GemmSplitParams {
 template <bool KC, int ROWS, int U>
 struct Stage {
     static constexpr int US = ROWS + 4;  // units per 8-k group in LDS (64 bytes of padding)
-    static constexpr bool ONE_ROW = !KC && U == 2;  // a thread's units belong to one row
     using Raw = f32x4[U][2];
     Raw raw[2];          // two steps' loads
-    int cls[U];          // scale class of the unit's row
-    uint32_t neg[U];     // sign bit of the row's scale
+    float sgn[U];        // 2^kUp or -2^kUp, the unit's row's factor
     const float* base;   // KC: row row0, k 0; else: k 0, column row0
     int64_t ld;
     int rows, row_a;     // rows of the operand in this tile; this thread's first row
@@ -96,13 +100,7 @@ struct Stage {
             voff = (uint32_t)(((int64_t)(8 * kg) * ld + row_a) * 4);
         }
 #pragma unroll
-        for (int i = 0; i < U; ++i) {
-            cls[i] = 2;
-            neg[i] = (uint32_t)__popc(KC ? row_a + ROWS / 2 * i : row_a) << 31;
-        }
-    }
-    __device__ __forceinline__ float with_sign(float v, int i) const {
-        return __uint_as_float(__float_as_uint(v) ^ neg[i]);
+        for (int i = 0; i < U; ++i) sgn[i] = with_parity(kUp, KC ? row_a + ROWS / 2 * i : row_a);
     }
     // k0 .. k0 + 31 below kend; elements outside read as zeros.
     __device__ __forceinline__ void load(Raw& r, int k0, int kend) const {
@@ -128,65 +126,16 @@ struct Stage {
                     r[i][e >> 2][e & 3] = buffer_ld1(rs, voff, (uint32_t)((int64_t)(16 * i + e) * ld * 4));
         }
     }
-    // The rows' classes for the loaded step; chg[row] = what the row's accumulators
-    // are to be multiplied by.  Returns whether some row's class changed.
-    __device__ __forceinline__ bool classes(const Raw& r, float (&chg)[ROWS]) {
-        float mx[U], f[U];
-        bool over = false;
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            mx[i] = absmax8(0.f, r[i][0], r[i][1]);
-            over |= mx[i] >= class_limit(cls[i]);
-            f[i] = 1.f;
-        }
-        const bool grow = __any(over);
-        if (grow) {
-#pragma unroll
-            for (int i = 0; i < U; ++i) mx[i] = absmax8_finite(0.f, r[i][0], r[i][1]);
-            agree(mx);
-#pragma unroll
-            for (int i = 0; i < U; ++i) {
-                const int nc = max(cls[i], scale_class(mx[i]));
-                f[i] = class_scale(nc) * class_inv(cls[i]);
-                cls[i] = nc;
-            }
-        }
-        put_rows(chg, f);
-        return grow;
-    }
     // Split the loaded step into LDS (no branch, so that it can be scheduled between
     // the MFMAs of the step before: 3-5% of the time).
-    __device__ __forceinline__ void store(const Raw& r, f16x8 (&L)[2][kKG][US]) const {
+    __device__ __forceinline__ void store(const Raw& r, bf16x8 (&L)[3][kKG][US]) const {
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-            const Half2x8 h = split2(r[i][0], r[i][1], with_sign(class_scale(cls[i]), i));
+            const Bf3x8 h = split3(r[i][0] * sgn[i], r[i][1] * sgn[i]);
             const int g = KC ? kg : kg + 2 * i, row = KC ? row_a + ROWS / 2 * i : row_a;
             L[0][g][row] = h.h;
-            L[1][g][row] = h.l;
-        }
-    }
-    __device__ __forceinline__ void put_units(float (&dst)[ROWS]) const {
-        float u[U];
-#pragma unroll
-        for (int i = 0; i < U; ++i) u[i] = with_sign(class_inv(cls[i]), i);
-        put_rows(dst, u);
-    }
-
-private:
-    // the largest over the lanes that hold parts of a row's step
-    static __device__ __forceinline__ void agree(float (&mx)[U]) {
-        if constexpr (ONE_ROW) mx[0] = mx[U - 1] = fmaxf(mx[0], mx[U - 1]);
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            if constexpr (KC) mx[i] = group_max<4>(mx[i]);
-            if constexpr (!KC && U == 1) mx[i] = fmaxf(mx[i], shfl_xor(mx[i], 16));
-            if constexpr (!KC) mx[i] = max_xor32(mx[i]);
-        }
-    }
-    __device__ __forceinline__ void put_rows(float (&dst)[ROWS], const float (&v)[U]) const {
-        if (kg == 0) {
-            dst[row_a] = v[0];
-            if constexpr (KC && U == 2) dst[row_a + ROWS / 2] = v[1];
+            L[1][g][row] = h.m;
+            L[2][g][row] = h.l;
         }
     }
 };
@@ -197,11 +146,8 @@ template <bool AKC, bool BKC>
 __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
     using StageA = Stage<AKC, kBM, 2>;
     using StageB = Stage<BKC, kBN, 1>;
-    __shared__ f16x8 Ua[2][2][kKG][StageA::US];  // [buffer][part][8-k group][row]
-    __shared__ f16x8 Ub[2][2][kKG][StageB::US];
-    __shared__ __attribute__((aligned(16))) float chg_a[2][kBM];
-    __shared__ __attribute__((aligned(16))) float chg_b[2][kBN];
-    __shared__ int tag_s[2];  // the last step whose staging changed a class, per buffer
+    __shared__ bf16x8 Ua[2][3][kKG][StageA::US];  // [buffer][part][8-k group][row]
+    __shared__ bf16x8 Ub[2][3][kKG][StageB::US];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -229,24 +175,18 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
     sa.init(A, p.lda, m0, p.M, tid);
     sb.init(B, p.ldb, n0, p.N, tid);
 
-    f32x16 acc[2][2];
+    f32x16 acc[2][2], lo[2][2];  // the main part products, and the small ones apart: their roundings stay off the result's last bits
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+        for (int j = 0; j < 2; ++j) acc[i][j] = lo[i][j] = f32x16{};
 
-    if (tid < 2) tag_s[tid] = -1;
     sa.load(sa.raw[0], kb, ke);
     sb.load(sb.raw[0], kb, ke);
     sa.load(sa.raw[1], kb + kBK, ke);
     sb.load(sb.raw[1], kb + kBK, ke);
-    __syncthreads();
-    {
-        const bool ga = sa.classes(sa.raw[0], chg_a[0]), gb = sb.classes(sb.raw[0], chg_b[0]);
-        sa.store(sa.raw[0], Ua[0]);
-        sb.store(sb.raw[0], Ub[0]);
-        if ((ga || gb) && lane == 0) tag_s[0] = 0;
-    }
+    sa.store(sa.raw[0], Ua[0]);
+    sb.store(sb.raw[0], Ub[0]);
     __syncthreads();
 
     // Step t computes on buffer BUF = t % 2; step t + 1, loaded in the previous
@@ -255,40 +195,28 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
         constexpr int BUF = decltype(buf_c)::value;
         sa.load(sa.raw[BUF], kb + (t + 2) * kBK, ke);
         sb.load(sb.raw[BUF], kb + (t + 2) * kBK, ke);
-        if (__builtin_amdgcn_readfirstlane(tag_s[BUF]) == t) {
-            float fb[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) fb[j] = chg_b[BUF][64 * wn + 32 * j + l32];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float fa = chg_a[BUF][64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3)];
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) acc[i][j][r] *= fa * fb[j];
-                }
-        }
-        const bool ga = sa.classes(sa.raw[BUF ^ 1], chg_a[BUF ^ 1]);
-        const bool gb = sb.classes(sb.raw[BUF ^ 1], chg_b[BUF ^ 1]);
-        if ((ga || gb) && lane == 0) tag_s[BUF ^ 1] = t + 1;
 #pragma unroll
         for (int kk = 0; kk < kBK / 16; ++kk) {
-            Half2x8 a[2], b[2];
+            Bf3x8 a[2], b[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                a[i].h = Ua[BUF][0][2 * kk + g][64 * wm + 32 * i + l32];
-                a[i].l = Ua[BUF][1][2 * kk + g][64 * wm + 32 * i + l32];
-                b[i].h = Ub[BUF][0][2 * kk + g][64 * wn + 32 * i + l32];
-                b[i].l = Ub[BUF][1][2 * kk + g][64 * wn + 32 * i + l32];
+                const int ra = 64 * wm + 32 * i + l32, rb = 64 * wn + 32 * i + l32;
+                a[i] = Bf3x8{Ua[BUF][0][2 * kk + g][ra], Ua[BUF][1][2 * kk + g][ra], Ua[BUF][2][2 * kk + g][ra]};
+                b[i] = Bf3x8{Ub[BUF][0][2 * kk + g][rb], Ub[BUF][1][2 * kk + g][rb], Ub[BUF][2][2 * kk + g][rb]};
             }
-            // the small part products first, four independent accumulators in turn
-#pragma unroll
-            for (int q = 0; q < 3; ++q)
+            // four independent accumulators in turn
+            auto product = [&](f32x16 (&c)[2][2], auto pa, auto pb) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = mfma32x32x16f16(q == 0 ? a[i].l : a[i].h, q == 1 ? b[j].l : b[j].h, acc[i][j]);
+                    for (int j = 0; j < 2; ++j) c[i][j] = mfma32x32x16bf16(a[i].*pa, b[j].*pb, c[i][j]);
+            };
+            product(lo, &Bf3x8::l, &Bf3x8::h);
+            product(lo, &Bf3x8::h, &Bf3x8::l);
+            product(lo, &Bf3x8::m, &Bf3x8::m);
+            product(lo, &Bf3x8::m, &Bf3x8::h);
+            product(lo, &Bf3x8::h, &Bf3x8::m);
+            product(acc, &Bf3x8::h, &Bf3x8::h);
         }
         sa.store(sa.raw[BUF ^ 1], Ua[BUF ^ 1]);
         sb.store(sb.raw[BUF ^ 1], Ub[BUF ^ 1]);
@@ -302,33 +230,28 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
     }
 
     // ---- epilogue ------------------------------------------------------------------
-    sa.put_units(chg_a[0]);
-    sb.put_units(chg_b[0]);
-    __syncthreads();
     float chk = 0.f;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+            acc[i][j] += lo[i][j];
 #pragma unroll
             for (int r = 0; r < 16; ++r) chk = fmaf(acc[i][j][r], 0.f, chk);
+        }
+    // A result that is not finite (an infinity or NaN in its operands, or a sum that only
+    // their factors took past the largest float) is formed again in plain fp32.
     const bool bad = __any(chk != 0.f);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int n = n0 + 64 * wn + 32 * j + l32;
-        const float ub = chg_b[0][64 * wn + 32 * j + l32];
+        const int nl = 64 * wn + 32 * j + l32, n = n0 + nl;
         const float bias = p.bias && n < p.N && p.ksplit == 1 ? p.bias[n] : 0.f;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int ml = 64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-                const int m = m0 + ml;
-                // the smaller scale first: a row near the largest floats times a column
-                // of tiny ones must not pass through an infinity
-                const float ua = chg_a[0][ml];
-                const bool a_first = fabsf(ua) < fabsf(ub);
-                float v = acc[i][j][r] * (a_first ? ua : ub) * (a_first ? ub : ua);
+                const int ml = 64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), m = m0 + ml;
+                float v = acc[i][j][r] * with_parity(kDown, ml ^ nl);
                 if (bad && __any(!(fabsf(v) < INFINITY))) {
                     if (!(fabsf(v) < INFINITY) && m < p.M && n < p.N) {
                         v = 0.f;

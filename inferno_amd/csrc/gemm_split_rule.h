@@ -23,16 +23,17 @@ inline int gemm_split_ranges(int ta, int tb, int64_t M, int64_t N, int64_t K, in
     const int64_t tm = (M + kSplitBM - 1) / kSplitBM, tn = (N + kSplitBN - 1) / kSplitBN;
     if (tm * tn > (1 << 24) || tm * tn * batch > (1 << 24)) return 0;
     const int64_t tiles = tm * tn * batch, nk = (K + kSplitBK - 1) / kSplitBK;
-    // The cheapest under a model (microseconds) fitted to measured shapes: the longest
-    // chain of K steps on a CU (1.65 a step, 8 steps for a workgroup's start and end)
-    // or, where the device is full and its clock falls with the load, the steps over
-    // the rate that large products reach; partials pass through memory once more.
+    // The cheapest under a model (microseconds, within 8% rms of 31 measured shapes): the
+    // longest chain of K steps on a CU (2.2 a step, 5 steps for a workgroup's start
+    // and end) or, where the device is full and its clock falls with the load, the
+    // steps over the rate that large products reach; partials pass through memory
+    // once more.
     double best = 1e30;
     int ks = 1;
     for (int c = 1; c <= 8; ++c) {
         if (c > 1 && (batch > 1 || nk / c < 8 || (double)c * M * N * sizeof(float) > (double)ws_bytes)) break;
-        const double wgs = (double)(tiles * c), steps = (double)((nk + c - 1) / c + 8);
-        double cost = std::max(steps * 1.65 * std::ceil(wgs / 256), wgs * steps / 146.0);
+        const double wgs = (double)(tiles * c), steps = (double)((nk + c - 1) / c + 5);
+        double cost = std::max(steps * 2.2 * std::ceil(wgs / 256), wgs * steps / 100.0);
         if (c > 1) cost += 4.0 + (double)(c + 1) * M * N * 4 / 4e6;
         if (cost < best) {
             best = cost;
@@ -41,7 +42,9 @@ inline int gemm_split_ranges(int ta, int tb, int64_t M, int64_t N, int64_t K, in
     }
     // The vendor library's fp32 kernels (about 142 TFLOP/s, 118 at ragged sizes, and
     // better split for small problems) where the model says that they are no
-    // slower: 1024^3 19 us there and 35 here, 1536^3 62 and 47, M = 32 9-18 and 25.
+    // slower, us there and here: 1024^3 20 and 37, 1200 x 512 x 2048 28 and 39, 1024 x 768
+    // x 3072 40 and 48, 8192 x 256 x 1024 38 and 41; but 8192 x 1024 x 256 40 and 34,
+    // 2048^3 122 and 102.
     const bool whole = M % 128 == 0 && N % 128 == 0 && K % 32 == 0;
     return best > 2.0 * M * N * K * batch / (whole ? 142e6 : 118e6) + 8.0 ? 0 : ks;
 }

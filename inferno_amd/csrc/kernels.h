@@ -235,7 +235,7 @@ struct GemmArgs {         // row-major C = alpha * op(A) op(B) + beta * C (+ bia
 };
 // 0 = ok, 1 = library error, 2 = no algorithm for the problem
 int launch_gemm(const GemmArgs& g, hipStream_t s);
-// fp32 on the fp16 matrix cores (gemm_split.hip); *taken: whether the problem is one of its
+// fp32 on the bf16 matrix cores (gemm_split.hip); *taken: whether the problem is one of its
 // own (else nothing was launched).  Returns a hipError_t value.
 int launch_gemm_split(const GemmArgs& g, hipStream_t s, bool* taken);
 

@@ -1,8 +1,8 @@
-"""The fp32 GEMM on two fp16 parts per operand (gemm_split.hip), at the sizes where a tile, a K step,
-a K range or the route to the vendor library ends, against 64-bit torch.
+"""The fp32 GEMM on three bf16 parts per operand (gemm_split.hip), at the sizes where a tile, a K step,
+a K range or the route to the vendor library ends, and at magnitudes far apart, against 64-bit torch.
 
-Bar: a product of split operands is within 2^-21.5 of itself (2^-23.8 rms) and an MFMA rounds 16 of
-them at once, so a result lies within a few 1e-7 of the norm of its terms; with terms of either sign
+Bar: operands are held exactly, a product of them is within 2^-25 and an MFMA rounds 16 of them at
+once, so a result lies within a few 1e-7 of the norm of its terms; with terms of either sign
 that norm is the result's own on average: 2e-6 (measured 1e-7 to 7e-7, what fp32 sums give too)."""
 import math
 
@@ -139,3 +139,56 @@ def test_batched(ia):
     assert st == 0
     for i in range(B):
         assert rel(c[i], ref(a[i], b[i], 0, 0)) <= BAR
+
+
+@pytest.mark.parametrize("e", [10, 13, 15, 30])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_columns_of_a_against_rows_of_b(ia, ta, tb, e):
+    """Columns of A and rows of B scaled against each other by up to 2^e either way, in any order
+    (features in unlike units with weights learnt for them): the terms are of one size again, so
+    every row and column of C is as exact as without the scales."""
+    M, N, K = 2048, 1600, 1024
+    a, b = make(M, N, K, ta, tb, seed=6)
+    s = torch.exp2(torch.linspace(-e, e, K).round()[torch.randperm(K, generator=torch.Generator().manual_seed(e))]).cuda()
+    a = a * (s[:, None] if ta else s)
+    b = b / (s if tb else s[:, None])
+    got, r = ia.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb)), ref(a, b, ta, tb)
+    d = got.double() - r
+    assert (d.norm(dim=1) / r.norm(dim=1)).max() <= BAR and (d.norm(dim=0) / r.norm(dim=0)).max() <= BAR
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_products_with_a_permutation_are_exact(ia, ta, tb):
+    """A times a permutation matrix is A's columns in that order, bit for bit, whatever stands beside an
+    element in its row: an outlier of 2^40, zeros, subnormal numbers; and a permutation times B."""
+    M, N, K = 2048, 1536, 1536
+    a, b = make(M, N, K, ta, tb, seed=7)
+    a = a.contiguous()
+    rows = a if not ta else a.t()
+    rows[:, 0] = 2.0**40
+    rows[5] *= 1e-38
+    rows[7] = torch.tensor([2.0**-149, -3 * 2.0**-140, 0.0, 1.0]).cuda().repeat(K // 4)
+    rows[9] *= 1e25
+    perm = torch.randperm(K, generator=torch.Generator().manual_seed(8)).cuda()
+    eye = torch.zeros(K, K, device="cuda")
+    eye[perm, torch.arange(K, device="cuda")] = 1.0  # column j picks element perm[j]
+    got = ia.gemm(a, eye.t().contiguous() if tb else eye, trans_a=bool(ta), trans_b=bool(tb))
+    assert torch.equal(got, rows[:, perm])
+    pick = torch.zeros(M, K, device="cuda")
+    src = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(9)).cuda()
+    pick[torch.arange(M, device="cuda"), src] = 1.0
+    b = b.contiguous()
+    cols = b if not tb else b.t()
+    cols[0] = -(2.0**40)
+    got = ia.gemm(pick.t().contiguous() if ta else pick, b, trans_a=bool(ta), trans_b=bool(tb))
+    assert torch.equal(got, cols[src])
+
+
+def test_results_past_the_operands_factors(ia):
+    """Results and operands whose size times the kernel's factors is past the largest float."""
+    M, N, K = 2048, 1600, 1024
+    for ea, eb in ((110, 10), (60, 40), (10, 110), (126, -126)):
+        a, b = make(M, N, K, 0, 0, seed=10)
+        a, b = a.clamp(-1.9, 1.9) * 2.0**ea, b.clamp(-1.9, 1.9) * 2.0**eb
+        got = ia.gemm(a, b)
+        assert got.isfinite().all() and rel(got, ref(a, b, 0, 0)) <= BAR, (ea, eb)
