@@ -20,8 +20,8 @@
 // and columns, by the parity of their index's bits, are negated, so that half of
 // the results are formed as their negatives and what is left cancels in sums over
 // rows or columns of C.  The small part products have accumulators of their own.
-// A non-finite element makes its row's or column's results NaN; the epilogue
-// forms those again one by one in plain fp32, so infinities come out as before.
+// A non-finite element makes its row's or column's results NaN; the wave that has one
+// forms its 64 x 64 again on the fp32 matrix cores, so infinities come out as before.
 //
 // Few tiles and a long K: the K range is split over workgroups, their partial
 // tiles go to the workspace and a second kernel sums them in order.
@@ -239,9 +239,49 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) chk = fmaf(acc[i][j][r], 0.f, chk);
         }
-    // A result that is not finite (an infinity or NaN in its operands, or a sum that only
-    // their factors took past the largest float) is formed again in plain fp32.
-    const bool bad = __any(chk != 0.f);
+    // A result that is not finite: an infinity or NaN in its operands, or a sum that only
+    // their factors took past the largest float.  The wave's 64 x 64 results are formed
+    // again in plain fp32, straight from memory.
+    const bool plain = __any(chk != 0.f);
+    if (plain) {
+        const float* ap[2];
+        const float* bp[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {  // null: zeros
+            const int m = m0 + 64 * wm + 32 * i + l32, n = n0 + 64 * wn + 32 * i + l32;
+            ap[i] = m < p.M ? A + (AKC ? (int64_t)m * p.lda : m) : nullptr;
+            bp[i] = n < p.N ? B + (BKC ? (int64_t)n * p.ldb : n) : nullptr;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+        }
+        auto load4 = [&](const float* q, int64_t ld, bool kc, int k) {  // k .. k + 3 below ke
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            if (q && k < ke) {
+                if (kc) {  // (ke is a multiple of 4 then)
+                    v = *reinterpret_cast<const f32x4*>(q + k);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = k + e < ke ? q[(int64_t)(k + e) * ld] : 0.f;
+                }
+            }
+            return v;
+        };
+#pragma unroll 1
+        for (int k = kb + 4 * g; k - 4 * g < ke; k += 8) {
+            f32x4 a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = load4(ap[i], p.lda, AKC, k);
+                b[i] = load4(bp[i], p.ldb, BKC, k);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x2(a[i][e], b[j][e], acc[i][j]);
+        }
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int nl = 64 * wn + 32 * j + l32, n = n0 + nl;
@@ -251,16 +291,7 @@ __global__ __launch_bounds__(kNT, 2) void gemm_split_kernel(GemmSplitParams p) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int ml = 64 * wm + 32 * i + 8 * (r >> 2) + 4 * g + (r & 3), m = m0 + ml;
-                float v = acc[i][j][r] * with_parity(kDown, ml ^ nl);
-                if (bad && __any(!(fabsf(v) < INFINITY))) {
-                    if (!(fabsf(v) < INFINITY) && m < p.M && n < p.N) {
-                        v = 0.f;
-#pragma unroll 1
-                        for (int k = kb; k < ke && v == v; ++k)  // a NaN stays one
-                            v = fmaf(AKC ? A[(int64_t)m * p.lda + k] : A[(int64_t)k * p.lda + m],
-                                     BKC ? B[(int64_t)n * p.ldb + k] : B[(int64_t)k * p.ldb + n], v);
-                    }
-                }
+                float v = acc[i][j][r] * (plain ? 1.f : with_parity(kDown, ml ^ nl));
                 if (m < p.M && n < p.N) {
                     if (p.ksplit > 1) {
                         p.part[((int64_t)split * p.M + m) * p.N + n] = v;

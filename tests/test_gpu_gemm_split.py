@@ -192,3 +192,22 @@ def test_results_past_the_operands_factors(ia):
         a, b = a.clamp(-1.9, 1.9) * 2.0**ea, b.clamp(-1.9, 1.9) * 2.0**eb
         got = ia.gemm(a, b)
         assert got.isfinite().all() and rel(got, ref(a, b, 0, 0)) <= BAR, (ea, eb)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(2048, 1600, 1024), (2049, 1537, 776), (770, 3070, 8192)])
+def test_results_beside_nonfinite_ones(ia, ta, tb, M, N, K):
+    """Infinities of one sign in a row and NaN in a column, in the middle and at the ragged ends (the last
+    row, column and k): what they don't reach, in the same tile and K range, is an ordinary result."""
+    a, b = make(M, N, K, ta, tb, seed=11)
+    rows, cols = (a.t() if ta else a), (b.t() if tb else b)
+    rows[100, K - 1] = math.inf
+    rows[M - 1, 3] = -math.inf
+    cols[K - 1, N - 1] = math.nan
+    got = ia.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb))
+    km = [i for i in range(M) if i not in (100, M - 1)]
+    want = ref(a, b, ta, tb)
+    assert rel(got[km, :N - 1], want[km, :N - 1]) <= BAR
+    assert torch.isnan(got[:, N - 1]).all()
+    assert torch.equal(got[100, :N - 1], torch.sign(cols[K - 1, :N - 1]) * math.inf)
+    assert torch.equal(got[M - 1, :N - 1], torch.sign(cols[3, :N - 1]) * -math.inf)
