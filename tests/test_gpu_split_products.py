@@ -174,8 +174,9 @@ def both_modes(ia, q, k, v, do, scale, causal=True):
 
 
 # Blocks of zero keys (padding) where a wave's, a pair's or a tile's keys are: an all-zero operand beside
-# ordinary ones.  (8, 16): the wide key blocks; D = 64 and 32 have 64 keys to a pair there, else 32.
-@pytest.mark.parametrize("B,H", [(1, 3), (8, 16)])
+# ordinary ones.  Wide key blocks (64 keys to a pair of waves, else 32): D = 32 with (8, 16), D = 64 with
+# (24, 12), both without a mask with (8, 16).
+@pytest.mark.parametrize("B,H", [(1, 3), (8, 16), (24, 12)])
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("what", ["k", "v", "kv"])
@@ -323,3 +324,23 @@ def test_rows_beside_nonfinite_keys(ia, B, H, Tq, Tk, causal, D):
     o, lse = ia.attn_fwd(q, k2, v, causal=causal, scale=c)
     assert row_err(o, torch.matmul(torch.softmax(s, -1), v.double())) <= BAR
     assert rel(lse, torch.logsumexp(s, -1)) <= BAR
+
+
+@pytest.mark.parametrize("B,H", [(1, 3), (1, 288)])
+@pytest.mark.parametrize("which", ["q", "k", "v", "do"])
+def test_largest_row_stride(ia, B, H, which):
+    """Rows 2^22 elements apart, the largest stride that is taken: a tile of rows spans just less than 2^31
+    bytes (narrow key blocks, and wide ones with 288 heads).  The same results as from dense rows: the
+    same bits, but for the order in which dQ's atomics arrive."""
+    D, T, c = 64, 300, 0.125
+    print(f"[case] row stride 2^22 of {which} H{H}", flush=True)
+    q, k, v, do = make(B, H, T, T, D, seed=12)
+    want = run(ia, q, k, v, do, c)
+    buf = torch.empty(((T - 1) << 22) + H * D, device="cuda")
+    t = {"q": q, "k": k, "v": v, "do": do}
+    far = buf.as_strided((B, H, T, D), (0, D, 1 << 22, 1))
+    far.copy_(t[which])
+    t[which] = far
+    got = run(ia, t["q"], t["k"], t["v"], t["do"], c)
+    for n, x, r in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+        assert (rel(x, r.double()) <= 1e-6) if n == "dq" else torch.equal(x, r), n
