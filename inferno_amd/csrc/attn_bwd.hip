@@ -916,18 +916,20 @@ __global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void bwd_dq_kernel(BwdParams
 
 // ---- split plan (host) ------------------------------------------------------------
 //
-// Under a causal mask key block j has ~(Tq - 128 j) / 32 query tiles, so at
-// config-2 sizes the first key blocks carry up to 8x the work of the last.
-// Measured on MI355X: a workgroup alone on a CU runs ~1.85x faster than each
-// of two sharing it (two resident workgroups give ~8% more throughput than
-// one), so the heaviest workgroups, which always share their CU with lighter
-// ones, set the kernel's length.  bwd_plan simulates the dispatch (workgroup w
-// to XCD w % 8, each XCD's workgroups placed in order on its least-loaded CU
-// with a free slot) for splits of the heaviest key blocks' tile ranges into
-// chunks, and keeps the best if it beats the unsplit order by 3%.
+// Under a causal mask key block j has ~(Tq - bk j) / 32 query tiles, so the first key
+// blocks carry many times the work of the last, and the heaviest workgroups set the
+// kernel's length.  bwd_plan simulates the dispatch (workgroup w to XCD w % 8, each
+// XCD's workgroups placed in order on its least-loaded CU with a free slot) for
+// splits of the heaviest key blocks' tile ranges into chunks, and keeps the best if it
+// beats the unsplit order by 3%.
+//
+// fp32 (one workgroup per CU): against splits forced into halves to eighths, at 77
+// shapes of 1 to 192 heads, T 100 to 8192, D 32 to 128, the plan's choice is within 5%
+// of the fastest but for B H 4, T 512, D 128 (48 and 45 us); without a split 2 to 5
+// times as slow at few heads (1 x 1024 x 64 136 us, split 41).
 
-static constexpr double kBwdPairGain = 0.08;  // throughput gained per extra resident workgroup
-// Per-workgroup fixed cost (K/V loads, K^T staging) and the partial store /
+static constexpr double kBwdPairGain = 0.08;  // throughput gained per extra resident workgroup (bf16 at D = 32: two per CU)
+// Per-workgroup fixed cost (K/V loads, K staging) and the partial store /
 // reduction of a split chunk, in query tiles of that dtype's kernel.  A bf16
 // tile costs a fraction of an fp32 one while the fixed costs take about the
 // same time; the bf16 figures are set from measurement (splits lost 5-8% at
@@ -1019,7 +1021,7 @@ static int bwd_slots(int D, int bf16, int* per_cu, int* cus_per_xcd) {
 static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int per_cu, int cus_per_xcd,
                              BwdPlan* out) {
     const int BH = B * H;
-    const int bk = bwd_keys_per_wg(bf16, D, BH, Tq, Tk);
+    const int bk = bwd_keys_per_wg(bf16, D, BH, Tq, Tk, 1);
     const int nkb = (Tk + bk - 1) / bk;
     const int off = Tk - Tq;
     if ((int64_t)nkb * BH > 8LL * 8 * cus_per_xcd * per_cu) return;  // the tail is a small share
@@ -1035,10 +1037,8 @@ static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int 
     struct G { double cost; int kb, a, b, chunk, n; };
     // A key block of more than ch tiles is split into ceil(n / ch) chunks of
     // near-equal cost, block 0's short tiles counted with the prologue's share
-    // pro.  The chunk size is chosen with pro = 0: counting the prologue there
-    // moved the choice to plans measured slower (config 2 fp32: ch 27-31, which
-    // leave key block 1 whole, +6-10%), while cutting block 0 at the weighted
-    // midpoint recovered half of the prologue's cost at the chosen size.
+    // pro.  The chunk size is chosen with pro = 0 (block 0's short tiles alone must
+    // not move it); the cuts of block 0 are then made with the prologue's share.
     auto build = [&](int ch, double pro, std::vector<G>& g) {
         g.clear();
         for (int j = 0; j < nkb; ++j) {
@@ -1114,7 +1114,7 @@ static void bwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, int 
 
 int bwd_plan(int B, int H, int Tq, int Tk, int D, int causal, int bf16, BwdPlan* out) {
     *out = BwdPlan{};
-    out->bk = bwd_keys_per_wg(bf16, D, (int64_t)B * H, Tq, Tk);
+    out->bk = bwd_keys_per_wg(bf16, D, (int64_t)B * H, Tq, Tk, 1);
     if (!causal) return 0;
     int per_cu = 0, cus_per_xcd = 0;
     if (const int e = bwd_slots(D, bf16, &per_cu, &cus_per_xcd)) return e;

@@ -423,9 +423,10 @@ __global__ __launch_bounds__(64 * FwdTile<D>::NW, 2) void attn_fwd_kernel(FwdPar
     }
 }
 
-// Combines the partial slots of each split query tile: per row
-// M = max_s m_s, w_s = exp2((m_s - M) c), O = sum_s w_s O_s / sum_s w_s l_s,
-// LSE = M * scale + ln(sum_s w_s l_s).  One thread per (row, 4 columns).
+// Combines the partial slots of each split query tile: per row M = max_s m_s,
+// w_s = 2^(m_s - M), O = sum_s w_s O_s / sum_s w_s l_s, LSE = M ln 2 + ln(sum_s w_s l_s),
+// where m is in exp2 units (fp32; bf16: in units of the scores, so times c, and
+// the scale).  One thread per (row, 4 columns).
 template <int D, typename E>
 __global__ __launch_bounds__(256) void attn_fwd_merge_kernel(FwdParams p) {
     constexpr int BM = fwd_bm(sizeof(E) == 2);
@@ -552,25 +553,32 @@ static int fwd_slots(int D, int bf16, FwdSlots* out) {
 
 // Causal forward split plan.  Without a split the query tiles run heaviest
 // first, one workgroup per (tile, head).  When the whole grid fits in the
-// resident slots at once, the heaviest tile alone sets the kernel time (1.9x
-// to 3.2x measured at B1 H2 T8192 D128 and B1 H4 T2048 D128), so its key range
-// is cut.  With more workgroups than slots the tail balances itself (a
-// workgroup left alone on a CU runs faster), and at B8 H12 T1024 D64 a split
-// made the forward 4% slower, merge pass included: such grids never split.
-// Each candidate chunk length CH cuts every tile with more than CH key tiles
-// into ceil(n / CH) near-equal chunks; the candidate with the smallest
-// simulated makespan (plus the merge pass) wins if it beats the unsplit order
-// by more than 2%.
+// resident slots at once, the heaviest tile alone sets the kernel time (fp32, us,
+// unsplit and split: B H 1, T 8192, D 64 490 and 126; 4, 2048, 128 240 and 58), so its
+// key range is cut.  With more workgroups than slots the tail balances itself: such
+// grids never split (96 x 1024 x 64 93 us, cut 90 to 128; 192 x 512 x 64 61 and 79 to 98;
+// 96 x 1024 x 128 152 and 160 to 217).  Each candidate chunk length CH cuts every tile
+// with more than CH key tiles into ceil(n / CH) near-equal chunks; the candidate with
+// the smallest simulated makespan (plus the merge pass) wins if it beats the unsplit
+// order by more than 2%.
+//
+// fp32: a key tile (128, 64, 32 keys at D = 32, 64, 128) takes about 4 us; the merge costs
+// two of them and the time that the partials take to memory and back (4 TB/s).  Over
+// 77 shapes the plan's time is 1.4% above the fastest of six forced splits (3.4% with
+// half a tile and nothing for the partials: 96 x 333 x 64 split 40 us, unsplit 30; one
+// workgroup of 200 rows 24 and 20).
 //
 // bf16 (constants fitted to measurements at T = 1024..8192, D = 32..128): a
-// bf16 key tile costs about a fifth of an fp32 one, so the workgroup's fixed
+// bf16 key tile costs about a fifth of an fp32-MFMA one, so the workgroup's fixed
 // cost and the merge weigh more in its units; up to four workgroups share a CU,
 // whose resident workgroups together run about 1.1 tiles in the time one runs
 // alone, so the makespan is also bounded below by the total work over the
 // CUs; and tiles under 32 key tiles (2048 keys) never split (B1 H12 T1024 D64
 // measured 19.9 us unsplit, 24.1 us split).
 static constexpr double kFwdOverhead[2] = {0.35, 2.0};   // per-workgroup fixed cost, in key tiles (fp32, bf16)
-static constexpr double kFwdMergeCost[2] = {0.5, 12.0};  // merge kernel, in key tiles
+static constexpr double kFwdMergeCost[2] = {2.0, 12.0};  // merge kernel, in key tiles
+// ... and per float of the partials (written and read: 8 bytes at 4 TB/s over 4 us)
+static constexpr double kFwdMergeFloat[2] = {8.0 / 16e6, 0.0};
 static constexpr double kFwdCuRate[2] = {0.0, 1.1};      // tiles per CU per tile time (0: no bound)
 static constexpr int kFwdMinSplitTiles[2] = {0, 32};
 
@@ -633,7 +641,9 @@ static void fwd_plan_compute(int B, int H, int Tq, int Tk, int D, int bf16, FwdS
         if ((int)g.size() > kMaxFwdGroups || n_split > kMaxFwdGroups / 2) continue;
         cost.resize(g.size());
         for (size_t i = 0; i < g.size(); ++i) cost[i] = g[i].n;
-        const double ms = span(cost) + merge_cost;
+        int64_t parts = 0;
+        for (const G& x : g) parts += x.t1 - x.t0 < nt[(size_t)x.qt];
+        const double ms = span(cost) + merge_cost + kFwdMergeFloat[ix] * (double)(parts * BH * BM * (D + 2));
         if (ms < best) {
             best = ms;
             best_ch = ch;

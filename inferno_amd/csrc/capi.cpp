@@ -28,7 +28,7 @@ std::atomic<int> g_deterministic{0};
 // in the deterministic mode, else bf16 shapes where the atomics bound the
 // fused kernel (bwd_dq_direct).
 bool dq_from_pass(int det, int B, int H, int Tq, int Tk, int D, inf_dtype dt) {
-    return det || (dt == INF_BF16 && inf::bwd_dq_direct(B * H, Tq, Tk, D, inf::bwd_keys_per_wg(1, D, (int64_t)B * H, Tq, Tk)));
+    return det || (dt == INF_BF16 && inf::bwd_dq_direct(B * H, Tq, Tk, D, inf::bwd_keys_per_wg(1, D, (int64_t)B * H, Tq, Tk, 1)));
 }
 
 size_t round_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
@@ -253,7 +253,7 @@ int inf_attn_bwd(const void* q, inf_strides sq, const void* k, inf_strides sk, c
     p.off = Tk - Tq;
     p.scale = scale;
     p.c = scale * 1.4426950408889634f;
-    const int bk = inf::bwd_keys_per_wg(dt == INF_BF16, D, (int64_t)B * H, Tq, Tk);
+    const int bk = inf::bwd_keys_per_wg(dt == INF_BF16, D, (int64_t)B * H, Tq, Tk, causal ? 1 : 0);
     p.keys_per_wg = bk;
     p.n_kblocks = (Tk + bk - 1) / bk;
     p.n_short = inf::bwd_short_rows(B, H, Tq, Tk, p.causal, inf::bwd_short_keys(dt == INF_BF16, bk));

@@ -337,17 +337,23 @@ constexpr int kFwdBf16BN = 64;   // keys per K/V tile of the bf16 forward (every
 // three 4-wave workgroups per CU.  D = 128 runs its own kernel, 8 waves x 16
 // keys: 128 keys per workgroup, as with 4 x 32.
 constexpr int bwd_bf16_waves(int D) { return D == 64 ? 8 : 4; }
-// BH = B * H.  fp32 at D <= 64 takes 256 keys (64 per pair of waves: fewer dQ
-// atomics, each staged query tile serves twice the keys), or 128 where a
-// workgroup's serial walk over few query tiles is what counts: with one key
-// block, or a grid that leaves CUs idle and short walks (B1 H12 T333 D64 backward
-// 40.6 -> 26.0 us, B8 H12 T256 44 -> 37; but B2 H12 T1024 64 -> 78, B8 H12 T1024
-// 159 -> 207).
-inline int bwd_keys_per_wg(int bf16, int D, int64_t BH, int Tq, int Tk) {
+// BH = B * H.  fp32 at D <= 64 takes 256 keys (64 per pair of waves) or 128: a query
+// tile takes 1.65 times as long with twice the keys (1.5 at D = 32), so 256 where the
+// grid is many rounds of the 256 CUs, and 128 where that leaves CUs idle or the longest
+// workgroup's walk sets the time.  Backward us, 128 and 256 keys, D = 64 (BH x T):
+//   causal: 1 x 333 28 and 44, 1 x 1536 68 and 75, 12 x 1024 67 and 68, 96 x 512 89 and 107,
+//   64 x 1024 167 and 173; but 12 x 1536 117 and 111, 96 x 1024 250 and 239, 64 x 2048
+//   624 and 562, 1 x 2048 106 and 97.  (D = 32: 4 x 1024 34 and 40, 16 x 1024 55 and 48.)
+//   no mask: 64 x 512 (one round of 128) 87 and 123, 64 x 777 (two, and one) 226 and 186,
+//   96 x 777 (three, and two) 326 and 351, D = 32 253 and 228.
+inline int bwd_keys_per_wg(int bf16, int D, int64_t BH, int Tq, int Tk, int causal) {
     if (D == 128) return 128;
     if (bf16) return 32 * bwd_bf16_waves(D);
-    const int64_t wgs = BH * ((Tk + 127) / 128);
-    return Tk <= 128 || (wgs <= 256 && wgs * ((Tq + 31) / 32) < 4096) ? 128 : 256;
+    const int64_t w128 = BH * ((Tk + 127) / 128), w256 = BH * ((Tk + 255) / 256);
+    if (!causal) return (w128 + 255) / 256 * 100 < (w256 + 255) / 256 * (D == 64 ? 158 : 145) ? 128 : 256;
+    if (Tk <= 128 || Tk > 1536) return Tk <= 128 ? 128 : 256;
+    if (w128 <= 256 && w128 * ((Tq + 31) / 32) < 4096) return 128;
+    return D == 64 && Tk <= 1024 && BH * Tk <= 80000 ? 128 : 256;
 }
 constexpr int kBwdBQ = 32;       // query rows per backward inner step
 // Leading query rows whose visible keys all lie in key block 0 (keys_per_wg
