@@ -181,6 +181,21 @@ def test_cross_entropy_row_splits(ia, rows, vocab, hide):
     assert (g.double() - gw).abs().max() <= 1e-5 * max(gw.abs().max().item(), 0.5 / rows)
 
 
+@pytest.mark.parametrize("rows,vocab", [(5000, 64), (3000, 9001)])
+def test_cross_entropy_mean_rounds_once(ia, rows, vocab):
+    """The mean over thousands of rows is within its own rounding (2^-24 at most) and what the first sums
+    leave (a few 2^-26 rms): 1e-7.  A sum that goes on in 32 bits to the end is 1.4e-7 off at times."""
+    gen = torch.Generator(device="cuda")
+    for s in range(8):
+        gen.manual_seed(s * 31 + 7)
+        x = torch.randn(rows, vocab, device="cuda", generator=gen) * 2
+        t = torch.randint(0, vocab, (rows,), device="cuda", generator=gen, dtype=torch.int32)
+        loss, _ = ia.cross_entropy_fwd(x, t)
+        xd = x.double()
+        want = (torch.logsumexp(xd, 1) - xd.gather(1, t.long()[:, None])[:, 0]).mean().item()
+        assert abs(loss.double().item() / want - 1) <= 1e-7, s
+
+
 def test_cross_entropy_bad_target_is_nan(ia):
     x = rnd(17, (2, 8))
     loss, _ = ia.cross_entropy_fwd(dev(x), dev(np.array([1, 8], np.int32)))
