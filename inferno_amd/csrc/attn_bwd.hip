@@ -573,8 +573,10 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
             }
             // dV^T += dO^T P or dK^T += Q^T dS, rows read transposed; step mm takes
             // queries 16 mm + 4 g + {0..3} and + 8
+            // (a step's rows are read while the step before runs where their registers fit)
+            constexpr bool AHEAD = NKB == 1;
             Bf3x8 pb[NKB], a[2];
-            a[0] = T::tr_frag(lds, tr_off, 0, 0, PART);
+            if constexpr (AHEAD) a[0] = T::tr_frag(lds, tr_off, 0, 0, PART);
 #pragma unroll
             for (int st = 0; st < 2 * NDB; ++st) {
                 const int mm = st / NDB, db = st % NDB;
@@ -596,11 +598,14 @@ __global__ __launch_bounds__(512, 2) void bwd_main_kernel(BwdParams p) {
                         }
                     }
                 }
-                if (st + 1 < 2 * NDB) a[(st + 1) & 1] = T::tr_frag(lds, tr_off, 16 * ((st + 1) / NDB), (st + 1) % NDB, PART);
+                const int rd = AHEAD ? st + 1 : st;
+                if (rd < 2 * NDB) a[rd & 1] = T::tr_frag(lds, tr_off, 16 * (rd / NDB), rd % NDB, PART);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int kb = 0; kb < NKB; ++kb) acc[db][kb] = mfma_split3(a[st & 1], pb[kb], acc[db][kb]);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int kb = 0; kb < NKB; ++kb) {
+                    acc[db][kb] = mfma_split3_once(a[st & 1], pb[kb], acc[db][kb]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         __syncthreads();

@@ -175,6 +175,16 @@ __device__ __forceinline__ f32x16 mfma_split3(const Bf3x8& a, const Bf3x8& b, f3
     c = mfma32x32x16bf16(a.h, b.m, c);
     return mfma32x32x16bf16(a.h, b.h, c);
 }
+// The same where c is the sum of many steps: the step's small part products meet it
+// in one addition, two roundings a step instead of six.
+__device__ __forceinline__ f32x16 mfma_split3_once(const Bf3x8& a, const Bf3x8& b, f32x16 c) {
+    f32x16 t = mfma32x32x16bf16(a.l, b.h, f32x16{});
+    t = mfma32x32x16bf16(a.h, b.l, t);
+    t = mfma32x32x16bf16(a.m, b.m, t);
+    t = mfma32x32x16bf16(a.m, b.h, t);
+    t = mfma32x32x16bf16(a.h, b.m, t);
+    return mfma32x32x16bf16(a.h, b.h, c + t);
+}
 // The same with the small part products in a sum of their own, which takes their
 // roundings away from the result's last bits.  SWAP exchanges the operands' roles in
 // the order, so that a product with swapped operands is formed to the same bits.
