@@ -26,11 +26,11 @@
 // The K rows' h and m parts lie in LDS, their l parts in registers, V in registers
 // as fp32 (its parts don't fit; split again for each tile).  S is formed in the
 // forward's order, to the same bits, so P is consistent with the LSE.
-// Bound by the MFMAs: 55% busy at D = 128 (7680 of 14000 cycles per tile and SIMD) at a
-// clock that the load holds at 1.9 GHz, which is 1.1 PFLOP/s of them where a large
-// library product reaches 1.25; at D = 64 (42% busy) also by the phases' latency.
-// Against the fp32 MFMAs, the backward call (us): config 2 308 -> 238, config 4 5980 ->
-// 3700.  Two scaled fp16 parts and three MFMAs took 163 and 2170, but blocks shared
+// Bound by the MFMAs: 51% busy at D = 128 (7680 of 15000 cycles per tile and SIMD) at a
+// clock that the load holds at 2.0 GHz, which is 1.07 PFLOP/s of them where a large
+// library product reaches 1.25; at D = 64 (39% busy) also by the phases' latency.
+// Against the fp32 MFMAs, the backward call (us): config 2 308 -> 248, config 4 5980 ->
+// 3870.  Two scaled fp16 parts and three MFMAs took 163 and 2170, but blocks shared
 // a scale: a block of zero keys gave infinities, small rows lost bits.
 //
 // bf16 inputs use the bf16-MFMA main kernel (attn_bwd_bf16.hip) between the
